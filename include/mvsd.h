@@ -338,6 +338,33 @@ int mvsd_spec_logprobs(int32_t* ids, float* lps, int32_t* ranks, const float* ta
                        int64_t width, int64_t k, int logits_mode, mvsd_stream_t stream);
 
 /* ------------------------------------------------------------------------------------ */
+/* spec_logprobs_split / topk_scores_split — mvsd_spec_logprobs and mvsd_topk_scores with   */
+/* each row split over workgroups, for k <= 128.  The same results (the sum of exponentials */
+/* in another order) from a workspace of mvsd_logprobs_workspace_bytes(positions, V, k)     */
+/* bytes, 16-byte aligned, caller-owned, no initial contents needed; positions = batch_size */
+/* * width, or num_rows.  That function returns 0 where this path does not apply; the calls */
+/* then return MVSD_E_RANGE.  Rows are MVSD_F32 / MVSD_BF16 / MVSD_F16 (dtype, common to     */
+/* target and bonus), upcast exactly, at any element alignment; bonus_rows [batch_size]     */
+/* selects request q's bonus row (NULL: row q).  topk_scores_split reads int64 tokens and   */
+/* writes int64 ids and ranks.                                                              */
+/* ------------------------------------------------------------------------------------ */
+int64_t mvsd_logprobs_workspace_bytes(int64_t positions, int64_t vocab_size, int64_t k);
+
+int mvsd_spec_logprobs_split(int32_t* ids, float* lps, int32_t* ranks, const void* target,
+                             int dtype, int64_t target_stride, const int32_t* target_rows,
+                             const void* bonus, int64_t bonus_stride, const int32_t* bonus_rows,
+                             const int32_t* cu_num_sampled_tokens,
+                             const int32_t* sampled_token_ids, int64_t sampled_stride,
+                             int64_t batch_size, int64_t num_tokens, int64_t vocab_size,
+                             int64_t width, int64_t k, int logits_mode, void* workspace,
+                             int64_t workspace_bytes, mvsd_stream_t stream);
+
+int mvsd_topk_scores_split(int64_t* ids, float* scores, int64_t* ranks, const void* logits,
+                           int dtype, int64_t logits_stride, const int64_t* token_ids,
+                           int64_t num_rows, int64_t vocab_size, int64_t k, int logits_mode,
+                           void* workspace, int64_t workspace_bytes, mvsd_stream_t stream);
+
+/* ------------------------------------------------------------------------------------ */
 /* sampler_rows — row operations of the regular sampler on fp32 rows x + r * stride.       */
 /* Replaces, in minivllm/sample/sampler.py: greedy_sample (:295-298, op 0: ids[r] = argmax */
 /* of row r, NaN first, lowest index on ties), apply_min_p (:280-293, op 1: with p the      */

@@ -448,7 +448,7 @@ int mvsd_spec_logprobs(int32_t* ids, float* lps, int32_t* ranks, const float* ta
     return MVSD_E_INVALID;
   if (num_tokens > 0 && (!target || target_stride < vocab_size)) return MVSD_E_INVALID;
   if (bonus_stride < vocab_size || sampled_stride < width) return MVSD_E_INVALID;
-  mvsd::LogprobParams p;
+  mvsd::LogprobParams p{};
   p.target = target;
   p.tstride = target_stride;
   p.target_rows = target_rows;
@@ -495,6 +495,91 @@ int mvsd_topk_scores(int32_t* ids, float* scores, int32_t* ranks, const float* l
   p.lps = scores;
   p.ranks = ranks;
   return hip_status(mvsd::launch_spec_logprobs(p, (hipStream_t)stream));
+}
+
+int64_t mvsd_logprobs_workspace_bytes(int64_t positions, int64_t vocab_size, int64_t k) {
+  if (positions < 0 || vocab_size <= 0 || vocab_size > 0x7fffffff || k < 0) return 0;
+  return mvsd::split_logprobs_workspace_bytes(positions, vocab_size, k);
+}
+
+int mvsd_spec_logprobs_split(int32_t* ids, float* lps, int32_t* ranks, const void* target,
+                             int dtype, int64_t target_stride, const int32_t* target_rows,
+                             const void* bonus, int64_t bonus_stride, const int32_t* bonus_rows,
+                             const int32_t* cu_num_sampled_tokens,
+                             const int32_t* sampled_token_ids, int64_t sampled_stride,
+                             int64_t batch_size, int64_t num_tokens, int64_t vocab_size,
+                             int64_t width, int64_t k, int logits_mode, void* workspace,
+                             int64_t workspace_bytes, mvsd_stream_t stream) {
+  if (batch_size < 0 || num_tokens < 0 || vocab_size <= 0 || width < 0 || k < 0)
+    return MVSD_E_INVALID;
+  if (batch_size == 0 || width == 0) return MVSD_OK;
+  if (k > vocab_size) return MVSD_E_RANGE;
+  if (batch_size * width > 0x7fffffff || num_tokens > 0x7fffffff || vocab_size > 0x7fffffff)
+    return MVSD_E_RANGE;
+  if (dtype != MVSD_F32 && dtype != MVSD_BF16 && dtype != MVSD_F16) return MVSD_E_INVALID;
+  if (!ids || !lps || !ranks || !bonus || !cu_num_sampled_tokens || !sampled_token_ids)
+    return MVSD_E_INVALID;
+  if (num_tokens > 0 && (!target || target_stride < vocab_size)) return MVSD_E_INVALID;
+  if (bonus_stride < vocab_size || sampled_stride < width) return MVSD_E_INVALID;
+  const int64_t need =
+      mvsd::split_logprobs_workspace_bytes(batch_size * width, vocab_size, k);
+  if (need == 0) return MVSD_E_RANGE;
+  if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15) != 0)
+    return MVSD_E_WORKSPACE;
+  mvsd::LogprobParams p{};
+  p.target = target;
+  p.tstride = target_stride;
+  p.target_rows = target_rows;
+  p.bonus = bonus;
+  p.bstride = bonus_stride;
+  p.bonus_rows = bonus_rows;
+  p.cu_sampled = cu_num_sampled_tokens;
+  p.tokens = sampled_token_ids;
+  p.tok_stride = sampled_stride;
+  p.B = (int)batch_size;
+  p.P = (int)num_tokens;
+  p.V = (int)vocab_size;
+  p.W = (int)width;
+  p.k = (int)k;
+  p.logits_mode = logits_mode ? 1 : 0;
+  p.ids = ids;
+  p.lps = lps;
+  p.ranks = ranks;
+  return hip_status(mvsd::launch_split_logprobs(p, dtype, workspace, (hipStream_t)stream));
+}
+
+int mvsd_topk_scores_split(int64_t* ids, float* scores, int64_t* ranks, const void* logits,
+                           int dtype, int64_t logits_stride, const int64_t* token_ids,
+                           int64_t num_rows, int64_t vocab_size, int64_t k, int logits_mode,
+                           void* workspace, int64_t workspace_bytes, mvsd_stream_t stream) {
+  if (num_rows < 0 || vocab_size <= 0 || k < 0) return MVSD_E_INVALID;
+  if (num_rows == 0) return MVSD_OK;
+  if (k > vocab_size) return MVSD_E_RANGE;
+  if (num_rows > 0x7fffffff || vocab_size > 0x7fffffff) return MVSD_E_RANGE;
+  if (dtype != MVSD_F32 && dtype != MVSD_BF16 && dtype != MVSD_F16) return MVSD_E_INVALID;
+  if (!ids || !scores || !ranks || !logits || !token_ids || logits_stride < vocab_size)
+    return MVSD_E_INVALID;
+  const int64_t need = mvsd::split_logprobs_workspace_bytes(num_rows, vocab_size, k);
+  if (need == 0) return MVSD_E_RANGE;
+  if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15) != 0)
+    return MVSD_E_WORKSPACE;
+  mvsd::LogprobParams p{};
+  p.bonus = logits;
+  p.bstride = logits_stride;
+  p.tokens = token_ids;
+  p.tokens64 = 1;
+  p.ids64 = 1;
+  p.B = (int)num_rows;
+  p.W = 1;
+  p.V = (int)vocab_size;
+  p.k = (int)k;
+  p.logits_mode = logits_mode ? 1 : 0;
+  p.flat = 1;
+  p.rank_raw = 1;
+  p.ids = ids;
+  p.lps = scores;
+  p.ranks = ranks;
+  return hip_status(mvsd::launch_split_logprobs(p, dtype, workspace, (hipStream_t)stream));
 }
 
 int mvsd_sampler_rows(int op, int32_t* ids, float* out, int64_t out_stride, float* x,

@@ -67,28 +67,6 @@ struct ConstraintSmem {
   int count;
 };
 
-// Inverse of ordered_bits (the shared zero key gives +0; unused keys map monotonically).
-__device__ inline float key_float(uint32_t key) {
-  return __uint_as_float((key & 0x80000000u) ? (key & 0x7fffffffu) : ~key);
-}
-
-template <int DT>
-__device__ inline float vec_elem(const u32x4& r, int j);
-template <>
-__device__ inline float vec_elem<MVSD_F32>(const u32x4& r, int j) {
-  return __uint_as_float(r[j]);
-}
-template <>
-__device__ inline float vec_elem<MVSD_BF16>(const u32x4& r, int j) {
-  const uint32_t w = r[j / 2];
-  return __uint_as_float((j & 1) ? (w & 0xffff0000u) : (w << 16));
-}
-template <>
-__device__ inline float vec_elem<MVSD_F16>(const u32x4& r, int j) {
-  const uint32_t w = r[j / 2];
-  return static_cast<float>(__builtin_bit_cast(_Float16, (uint16_t)((j & 1) ? (w >> 16) : w)));
-}
-
 // Calls g(vector index, 16-byte vector) for every vector of a row of nvec vectors: full
 // batches of U vectors per thread, two batches in flight (each iteration issues one buffer's
 // next loads before consuming the other, and the loads of a full batch are unconditional, the

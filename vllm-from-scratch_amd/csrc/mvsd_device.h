@@ -71,6 +71,38 @@ __device__ inline void load_vec(const typename Elem<DT>::storage* __restrict__ p
   }
 }
 
+// The 16-byte vector holding elements p[0 .. kVec) at any element alignment.  The type tells
+// the compiler that only element alignment holds; gfx950's global loads take any alignment, so
+// it emits one global_load_dwordx4 for rows of odd length too.  p[0 .. kVec) must be in bounds.
+typedef u32x4 u32x4_align4 __attribute__((aligned(4)));
+typedef u32x4 u32x4_align2 __attribute__((aligned(2)));
+
+template <int DT>
+__device__ inline u32x4 load_vec_any(const typename Elem<DT>::storage* p) {
+  if constexpr (sizeof(typename Elem<DT>::storage) == 4)
+    return *reinterpret_cast<const u32x4_align4*>(p);
+  else
+    return *reinterpret_cast<const u32x4_align2*>(p);
+}
+
+// Element j of a 16-byte vector, as fp32.
+template <int DT>
+__device__ inline float vec_elem(const u32x4& r, int j);
+template <>
+__device__ inline float vec_elem<MVSD_F32>(const u32x4& r, int j) {
+  return __uint_as_float(r[j]);
+}
+template <>
+__device__ inline float vec_elem<MVSD_BF16>(const u32x4& r, int j) {
+  const uint32_t w = r[j / 2];
+  return __uint_as_float((j & 1) ? (w & 0xffff0000u) : (w << 16));
+}
+template <>
+__device__ inline float vec_elem<MVSD_F16>(const u32x4& r, int j) {
+  const uint32_t w = r[j / 2];
+  return static_cast<float>(__builtin_bit_cast(_Float16, (uint16_t)((j & 1) ? (w >> 16) : w)));
+}
+
 // ------------------------------------------------------------------ comparisons ------
 
 // True when (a, ia) ranks above (b, ib): NaN above numbers, larger value, then lower index.
@@ -281,6 +313,11 @@ __device__ inline uint32_t ordered_bits(float x) {
   const uint32_t b = __float_as_uint(x);
   const uint32_t o = (b & 0x80000000u) ? ~b : (b | 0x80000000u);
   return (x != x) ? 0xffffffffu : (x == 0.f ? 0x80000000u : o);
+}
+
+// Inverse of ordered_bits (the shared zero key gives +0; unused keys map monotonically).
+__device__ inline float key_float(uint32_t key) {
+  return __uint_as_float((key & 0x80000000u) ? (key & 0x7fffffffu) : ~key);
 }
 
 __device__ inline uint64_t argmax_key(float v, int idx) {

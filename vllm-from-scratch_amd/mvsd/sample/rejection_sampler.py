@@ -93,6 +93,7 @@ class RejectionSampler:
                 logits: torch.Tensor, sampling_metadata: SamplingMetadata):
         """``logits`` is the compact ``[P + B, V]`` tensor in metadata row order (:153-225)."""
         from ..outputs import SamplerOutput
+        from .sampler import Sampler as DeviceSampler
 
         assert metadata.max_spec_len <= MAX_SPEC_LEN
         if len(sampling_metadata.prompt_token_ids) != len(metadata.num_draft_tokens):
@@ -115,9 +116,14 @@ class RejectionSampler:
         # full-row logits are asked for only when logprobs are (the sampled tokens do not
         # depend on it, and the copy is a [B, V] write)
         bonus_logits = logits[metadata.bonus_logits_indices]
+        # the raw modes report the bonus rows as they arrive, which mvsd.sample.Sampler would
+        # only hand back as an fp32 copy
+        bonus_rows_in_place = (max_num_logprobs is not None
+                               and not self.is_processed_logprobs_mode
+                               and type(self.sampler) is DeviceSampler)
         bonus_out = self.sampler.forward(
             bonus_logits, replace(sampling_metadata, max_num_logprobs=(
-                -1 if max_num_logprobs is not None else None)),
+                -1 if max_num_logprobs is not None and not bonus_rows_in_place else None)),
             predict_bonus_token=True,
             logprobs_mode_override=("processed_logits" if self.is_processed_logprobs_mode
                                     else "raw_logits"))
@@ -160,7 +166,8 @@ class RejectionSampler:
         # 4) logprobs of every output position (:212-223); raw modes read the raw verify rows
         logprobs_tensors = None
         if max_num_logprobs is not None:
-            bonus_rows = bonus_out.logprobs_tensors.logprobs
+            bonus_rows = (None if bonus_rows_in_place
+                          else bonus_out.logprobs_tensors.logprobs)
             if self.is_processed_logprobs_mode:
                 logprobs_tensors = self._get_logprobs_tensors(
                     max_num_logprobs, metadata, logits, target_logits, bonus_rows,
@@ -227,7 +234,7 @@ class RejectionSampler:
 
     def _get_logprobs_tensors(self, max_num_logprobs: int, metadata: "SpecDecodeMetadata",
                               logits: torch.Tensor, target_logits: torch.Tensor | None,
-                              bonus_logits: torch.Tensor,
+                              bonus_logits: torch.Tensor | None,
                               sampled_token_ids: torch.Tensor):
         """Logprobs of every output position ``[B * (max_spec_len + 1)]`` (:229-300).
 
@@ -236,9 +243,11 @@ class RejectionSampler:
         read their own row and padding positions read rows that parse_output drops with the
         same valid mask.  Verify rows come from ``target_logits`` ([P, V], the processed rows
         in the processed modes) or, when it is None, from ``logits`` at
-        ``metadata.target_logits_indices``; the bonus rows from ``bonus_logits`` [B, V].  The
-        values are the log-softmax of each row, or the rows themselves in the ``*_logits``
-        modes.  One ``mvsd_spec_logprobs`` launch.
+        ``metadata.target_logits_indices``; the bonus rows from ``bonus_logits`` [B, V] or, when
+        it is None, from ``logits`` at ``metadata.bonus_logits_indices``.  The values are the
+        log-softmax of each row, or the rows themselves in the ``*_logits`` modes.  One
+        ``mvsd_spec_logprobs_split`` call (``mvsd_spec_logprobs`` above 128 logprobs); when both
+        kinds of rows come from ``logits`` the former reads them in place in their own dtype.
         """
         from ..outputs import LogprobsTensors
 
@@ -248,21 +257,32 @@ class RejectionSampler:
         device = sampled_token_ids.device
         nat.require_device_tensor(sampled_token_ids, "sampled_token_ids")
         B, W = sampled_token_ids.shape
-        V = int(bonus_logits.shape[-1])
+        V = int(logits.shape[-1] if bonus_logits is None else bonus_logits.shape[-1])
         num_tokens = int(metadata.draft_token_ids.shape[0])
         if not 0 <= max_num_logprobs <= V:
             raise ValueError(f"logprobs={max_num_logprobs} outside [0, {V}]")
         keep = []
-        rows = None
+        handle = nat.lib()
+        ws_bytes = handle.mvsd_logprobs_workspace_bytes(B * W, V, max_num_logprobs)
+        rows = bonus_rows = None
         if target_logits is None:
             target_logits, rows = logits, _as(metadata.target_logits_indices, torch.int32, device)
-        if target_logits.dtype != torch.float32 or target_logits.stride(-1) != 1:
-            target_logits = (target_logits if rows is None else target_logits[rows.long()]).float()
-            target_logits = target_logits.contiguous()
-            rows = None
-        bonus = bonus_logits.to(torch.float32)
-        if bonus.stride(-1) != 1:
-            bonus = bonus.contiguous()
+        if bonus_logits is None:
+            bonus, bonus_rows = logits, _as(metadata.bonus_logits_indices, torch.int32, device)
+        else:
+            bonus = bonus_logits.to(torch.float32)
+        in_place = (ws_bytes > 0 and target_logits is bonus
+                    and bonus.dtype in (torch.float32, torch.bfloat16, torch.float16)
+                    and bonus.stride(-1) == 1)
+        if not in_place:
+            if target_logits.dtype != torch.float32 or target_logits.stride(-1) != 1:
+                target_logits = (target_logits if rows is None
+                                 else target_logits[rows.long()]).float().contiguous()
+                rows = None
+            if bonus_rows is not None:
+                bonus, bonus_rows = bonus[bonus_rows.long()].float(), None
+            if bonus.stride(-1) != 1:
+                bonus = bonus.contiguous()
         tokens = _as(sampled_token_ids, torch.int32, device)
         cu = _as(metadata.cu_num_sampled_tokens, torch.int32, device)
         keep += [target_logits, bonus, tokens, cu]
@@ -270,7 +290,18 @@ class RejectionSampler:
         ids = torch.empty((B * W, n_out), dtype=torch.int32, device=device)
         lps = torch.empty((B * W, n_out), dtype=torch.float32, device=device)
         ranks = torch.empty((B * W,), dtype=torch.int32, device=device)
-        nat.check(nat.lib().mvsd_spec_logprobs(
+        if ws_bytes > 0:
+            workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
+            nat.check(handle.mvsd_spec_logprobs_split(
+                ids.data_ptr(), lps.data_ptr(), ranks.data_ptr(),
+                target_logits.data_ptr() if num_tokens else None, nat.dtype_code(bonus.dtype),
+                target_logits.stride(0), nat.ptr(rows), bonus.data_ptr(), bonus.stride(0),
+                nat.ptr(bonus_rows), cu.data_ptr(), tokens.data_ptr(), tokens.stride(0), B,
+                num_tokens, V, W, max_num_logprobs, 1 if self.is_logits_logprobs_mode else 0,
+                workspace.data_ptr(), ws_bytes, nat.stream_of(device)),
+                "mvsd_spec_logprobs_split")
+            return LogprobsTensors(ids, lps, ranks)
+        nat.check(handle.mvsd_spec_logprobs(
             ids.data_ptr(), lps.data_ptr(), ranks.data_ptr(),
             target_logits.data_ptr() if num_tokens else None, target_logits.stride(0),
             None if rows is None else rows.data_ptr(), bonus.data_ptr(), bonus.stride(0),
