@@ -241,6 +241,28 @@ int mvsd_apply_top_k_top_p(float* logits, int64_t logits_stride, const int64_t* 
                            mvsd_stream_t stream);
 
 /* ------------------------------------------------------------------------------------ */
+/* mvsd_rejection_sample, mvsd_sampling_masks and mvsd_apply_top_k_top_p with the sampling  */
+/* constraints' rows split over workgroups: the same results, from scratch of               */
+/* mvsd_constraints_scratch_bytes(rows, V) bytes (rows = num_tokens or num_rows), 256-byte  */
+/* aligned, caller-owned, no initial contents needed.  That function returns 0 where the    */
+/* split path does not apply (above 128 rows): rejection_sample_split and                   */
+/* sampling_masks_split then (and with scratch or top_p NULL) take the other path,          */
+/* apply_top_k_top_p_split returns MVSD_E_RANGE.                                            */
+/* ------------------------------------------------------------------------------------ */
+int64_t mvsd_constraints_scratch_bytes(int64_t num_rows, int64_t vocab_size);
+
+int mvsd_rejection_sample_split(const mvsd_rejection_args* args, void* scratch,
+                                int64_t scratch_bytes, mvsd_stream_t stream);
+
+int mvsd_sampling_masks_split(const mvsd_rejection_args* args, float* masks, void* scratch,
+                              int64_t scratch_bytes, mvsd_stream_t stream);
+
+int mvsd_apply_top_k_top_p_split(float* logits, int64_t logits_stride, const int64_t* top_k,
+                                 const float* top_p, int64_t num_rows, int64_t vocab_size,
+                                 void* scratch, int64_t scratch_bytes, mvsd_stream_t stream);
+
+
+/* ------------------------------------------------------------------------------------ */
 /* ngram_valid_sampled — the valid sampled tokens of one step, per request.               */
 /* Replaces: NgramProposerGPU.update_token_ids_ngram                                     */
 /*           (minivllm/spec_decode/ngram_proposer_gpu.py:247-290).                        */

@@ -1,0 +1,100 @@
+"""Sampling constraints with rows split over workgroups (mvsd_sampling_masks_split,
+mvsd_apply_top_k_top_p_split) against the one-workgroup-per-row path (mvsd_sampling_masks,
+mvsd_apply_top_k_top_p): both find the same first kept entry with the same exact integer sums, so
+the masks are equal bit for bit."""
+
+import math
+
+import pytest
+import torch
+
+from mvsd import _native as nat
+from mvsd.sample.metadata import SamplingMetadata
+from mvsd.sample.ops.topk_topp_sampler import apply_top_k_top_p
+from mvsd.sample.rejection_sampler import sampling_masks
+
+pytestmark = pytest.mark.gpu
+
+
+def general_masks(x, cu, rows, sm):
+    masks = torch.full((rows.shape[0], 4), 7.0, device=x.device)
+    args = nat.RejectionArgs(
+        target_logits=x.data_ptr(), target_dtype=nat.dtype_code(x.dtype),
+        target_stride=x.stride(0), target_rows=rows.data_ptr(), target_num_rows=x.shape[0],
+        cu_num_draft_tokens=cu.data_ptr(), temperature=nat.ptr(sm.temperature), all_greedy=0,
+        apply_temperature=1, batch_size=cu.shape[0], num_tokens=rows.shape[0],
+        vocab_size=x.shape[1], top_k=nat.ptr(sm.top_k), top_p=nat.ptr(sm.top_p))
+    nat.check(nat.lib().mvsd_sampling_masks(args, masks.data_ptr(), nat.stream_of(x.device)),
+              "mvsd_sampling_masks")
+    return masks
+
+
+def make_rows(V, dtype, device, g):
+    """One row of each kind a pass can go wrong on."""
+    n = torch.randn(8, V, device=device, generator=g)
+    rows = [n[0] * 2, n[1] * 6, n[2] * 0.05, torch.zeros(V, device=device),
+            (n[3] * 3).round(), -n[4].abs() * 100, n[5] * 2 + 80]
+    inf = n[6].clone()
+    inf[V // 2] = math.inf
+    nan = n[7].clone()
+    nan[V - 1] = math.nan
+    some = torch.full((V,), -math.inf, device=device)
+    some[::max(1, V // 7)] = n[0][::max(1, V // 7)]
+    peak = n[1] - 30
+    peak[V // 3] = 20.0
+    return torch.stack([*rows, inf, nan, some, torch.full((V,), -math.inf, device=device),
+                        peak]).to(dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("V", [65536, 65537, 73727, 151936, 524288])
+def test_masks_equal_general_path(device, dtype, V):
+    g = torch.Generator(device=device).manual_seed(V)
+    x = make_rows(V, dtype, device, g)
+    kinds = [(0, 0.9, 0.8), (0, 0.3, 1.5), (0, 0.999, 1.0), (0, 1e-6, 0.7), (0, 0.0, 1.0),
+             (1, 1.0, 0.8), (20, 1.0, 1.3), (50, 0.9, 0.8), (300, 0.5, 1.0), (600, 0.9, 1.0),
+             (V - 1, 0.8, 0.9), (0, 0.9, 0.0), (0, 0.2, 0.0), (5, 0.5, 0.0), (5, 1.0, 0.0),
+             (0, 1.0, 0.9), (0, 0.9, 1e-30), (3, 0.9, 1e25)]
+    n = x.shape[0]
+    # every kind on every row, the rows in another order for each request
+    for part in (kinds[:9], kinds[9:]):  # at most 128 rows a call
+        _compare(x, part, g)
+
+
+def _compare(x, kinds, g):
+    device, n, V = x.device, x.shape[0], x.shape[1]
+    rows = torch.cat([torch.randperm(n, device=device, generator=g) for _ in kinds]).to(torch.int32)
+    assert rows.shape[0] <= 128
+    cu = torch.arange(n, n * len(kinds) + 1, n, dtype=torch.int32, device=device)
+    sm = SamplingMetadata(
+        temperature=torch.tensor([t for _, _, t in kinds], device=device), all_greedy=False,
+        all_random=False,
+        top_k=torch.tensor([k or V for k, _, _ in kinds], dtype=torch.int64, device=device),
+        top_p=torch.tensor([p for _, p, _ in kinds], device=device))
+    for top_k, top_p in ((True, True), (False, True)):
+        part = SamplingMetadata(temperature=sm.temperature, all_greedy=False, all_random=False,
+                                top_k=sm.top_k if top_k else None,
+                                top_p=sm.top_p if top_p else None)
+        got = sampling_masks(x, cu, part, target_rows=rows)
+        want = general_masks(x, cu, rows, part)
+        same = (got.view(torch.int32) == want.view(torch.int32)).all(dim=1)
+        bad = [(kinds[j // n], int(rows[j]), got[j].tolist(), want[j].tolist())
+               for j in (~same).nonzero().view(-1).tolist()]
+        assert not bad, bad[:5]
+
+
+@pytest.mark.parametrize("n,V", [(3, 65536), (5, 65539), (100, 151936)])
+def test_apply_in_place_equals_general_path(device, n, V):
+    """Rows of a wider tensor (an odd stride), in place; the long chunks from 16 rows on."""
+    g = torch.Generator(device=device).manual_seed(n)
+    wide = torch.randn(n, V + 3, device=device, generator=g) * 2.5
+    k = torch.randint(1, 200, (n,), device=device, generator=g)
+    k[::3] = V
+    p = torch.rand(n, device=device, generator=g)
+    p[::4] = 1.0
+    want = wide.clone()
+    nat.check(nat.lib().mvsd_apply_top_k_top_p(
+        want[:, 1:V + 1].data_ptr(), want.stride(0), k.data_ptr(), p.data_ptr(), n, V,
+        nat.stream_of(device)), "mvsd_apply_top_k_top_p")
+    apply_top_k_top_p(wide[:, 1:V + 1], k, p)
+    assert torch.equal(wide, want)

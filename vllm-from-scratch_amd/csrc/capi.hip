@@ -191,9 +191,10 @@ int mvsd_rejection_workspace_init(void* workspace, int64_t workspace_bytes, mvsd
 namespace {
 
 // mvsd_rejection_sample with the workspace `ws` of `ws_bytes` bytes (the args' workspace fields
-// are not read).
+// are not read); with scratch, the sampling constraints' rows are split over workgroups.
 int rejection_sample_impl(const mvsd_rejection_args* a, void* ws_ptr, int64_t ws_bytes,
-                          mvsd_stream_t stream) {
+                          mvsd_stream_t stream, void* scratch = nullptr,
+                          int64_t scratch_bytes = 0) {
   if (!a) return MVSD_E_INVALID;
   const int64_t B = a->batch_size, P = a->num_tokens, V = a->vocab_size;
   if (B < 0 || P < 0 || V <= 0 || a->max_spec_len < 0) return MVSD_E_INVALID;
@@ -286,7 +287,12 @@ int rejection_sample_impl(const mvsd_rejection_args* a, void* ws_ptr, int64_t ws
   // The row masks of the whole batch, then one verify launch per kMaxLaunchRequests requests
   // (their tables live in LDS); the launches share the workspace, which each leaves zeroed.
   if (masked) {
-    err = mvsd::launch_constraints(p, a->target_dtype, (hipStream_t)stream);
+    const int64_t need = scratch && p.top_p ? mvsd::split_constraints_bytes(P, V) : 0;
+    if (need > 0 && (scratch_bytes < need || ((uintptr_t)scratch & 255) != 0))
+      return MVSD_E_WORKSPACE;
+    err = need > 0 ? mvsd::launch_split_constraints(p, a->target_dtype, 0.f, false, false, scratch,
+                                                    (hipStream_t)stream)
+                   : mvsd::launch_constraints(p, a->target_dtype, (hipStream_t)stream);
     if (err != hipSuccess) return hip_status(err);
   }
   const int groups_per_req = (int)((a->max_spec_len + size_plan.g - 1) / size_plan.g);
@@ -334,6 +340,47 @@ int rejection_sample_impl(const mvsd_rejection_args* a, void* ws_ptr, int64_t ws
   return MVSD_OK;
 }
 
+// mvsd_sampling_masks; with scratch, the rows are split over workgroups.
+int sampling_masks_impl(const mvsd_rejection_args* a, float* masks, void* scratch,
+                        int64_t scratch_bytes, mvsd_stream_t stream) {
+  if (!a || !masks) return MVSD_E_INVALID;
+  const int64_t B = a->batch_size, P = a->num_tokens, V = a->vocab_size;
+  if (B < 0 || P < 0 || V <= 0) return MVSD_E_INVALID;
+  if (B > 0x7fffffff || P > 0x7fffffff || V > 0x7fffffff) return MVSD_E_RANGE;
+  if (P == 0) return MVSD_OK;
+  if (!a->target_logits || !a->cu_num_draft_tokens) return MVSD_E_INVALID;
+  if (a->target_dtype != MVSD_F32 && a->target_dtype != MVSD_BF16 && a->target_dtype != MVSD_F16)
+    return MVSD_E_INVALID;
+  if (!a->all_greedy && !a->temperature) return MVSD_E_INVALID;
+  if (a->target_stride < V) return MVSD_E_INVALID;
+  if (a->target_rows && a->target_num_rows < 1) return MVSD_E_INVALID;
+  if ((uintptr_t)masks % 16 != 0) return MVSD_E_ALIGN;
+  mvsd::VerifyParams p;
+  memset(&p, 0, sizeof(p));
+  p.target = a->target_logits;
+  p.target_stride = a->target_stride;
+  p.target_rows = a->target_rows;
+  p.target_num_rows = a->target_num_rows;
+  p.cu = a->cu_num_draft_tokens;
+  p.temperature = a->temperature;
+  p.target_dtype = a->target_dtype;
+  p.all_greedy = a->all_greedy ? 1 : 0;
+  p.apply_temperature = a->apply_temperature ? 1 : 0;
+  p.B = (int)B;
+  p.P = (int)P;
+  p.V = (int)V;
+  p.top_k = a->top_k;
+  p.top_p = a->top_p;
+  p.masks = reinterpret_cast<float4*>(masks);
+  const int64_t need = scratch && p.top_p ? mvsd::split_constraints_bytes(P, V) : 0;
+  if (need > 0) {
+    if (scratch_bytes < need || ((uintptr_t)scratch & 255) != 0) return MVSD_E_WORKSPACE;
+    return hip_status(mvsd::launch_split_constraints(p, a->target_dtype, 0.f, false, false,
+                                                     scratch, (hipStream_t)stream));
+  }
+  return hip_status(mvsd::launch_constraints(p, a->target_dtype, (hipStream_t)stream));
+}
+
 // Static scratch of mvsd_rejection_sample_static: one per device that the library runs on, held
 // until the process ends.  Host code never uses the array's name as an address: the device
 // address comes from hipGetSymbolAddress, once per device, with that device current.
@@ -378,6 +425,17 @@ extern "C" {
 int mvsd_rejection_sample(const mvsd_rejection_args* a, mvsd_stream_t stream) {
   if (!a) return MVSD_E_INVALID;
   return rejection_sample_impl(a, a->workspace, a->workspace_bytes, stream);
+}
+
+int64_t mvsd_constraints_scratch_bytes(int64_t num_rows, int64_t vocab_size) {
+  if (num_rows < 0 || num_rows > 0x7fffffff || vocab_size <= 0 || vocab_size > 0x7fffffff) return 0;
+  return mvsd::split_constraints_bytes(num_rows, vocab_size);
+}
+
+int mvsd_rejection_sample_split(const mvsd_rejection_args* a, void* scratch, int64_t scratch_bytes,
+                                mvsd_stream_t stream) {
+  if (!a) return MVSD_E_INVALID;
+  return rejection_sample_impl(a, a->workspace, a->workspace_bytes, stream, scratch, scratch_bytes);
 }
 
 int64_t mvsd_rejection_static_scratch_bytes(void) { return kStaticScratchBytes; }
@@ -654,36 +712,37 @@ int mvsd_selftest(int test, uint64_t* failures, mvsd_stream_t stream) {
 }
 
 int mvsd_sampling_masks(const mvsd_rejection_args* a, float* masks, mvsd_stream_t stream) {
-  if (!a || !masks) return MVSD_E_INVALID;
-  const int64_t B = a->batch_size, P = a->num_tokens, V = a->vocab_size;
-  if (B < 0 || P < 0 || V <= 0) return MVSD_E_INVALID;
-  if (B > 0x7fffffff || P > 0x7fffffff || V > 0x7fffffff) return MVSD_E_RANGE;
-  if (P == 0) return MVSD_OK;
-  if (!a->target_logits || !a->cu_num_draft_tokens) return MVSD_E_INVALID;
-  if (a->target_dtype != MVSD_F32 && a->target_dtype != MVSD_BF16 && a->target_dtype != MVSD_F16)
-    return MVSD_E_INVALID;
-  if (!a->all_greedy && !a->temperature) return MVSD_E_INVALID;
-  if (a->target_stride < V) return MVSD_E_INVALID;
-  if (a->target_rows && a->target_num_rows < 1) return MVSD_E_INVALID;
-  if ((uintptr_t)masks % 16 != 0) return MVSD_E_ALIGN;
+  return sampling_masks_impl(a, masks, nullptr, 0, stream);
+}
+
+int mvsd_sampling_masks_split(const mvsd_rejection_args* a, float* masks, void* scratch,
+                              int64_t scratch_bytes, mvsd_stream_t stream) {
+  return sampling_masks_impl(a, masks, scratch, scratch_bytes, stream);
+}
+
+int mvsd_apply_top_k_top_p_split(float* logits, int64_t logits_stride, const int64_t* top_k,
+                                 const float* top_p, int64_t num_rows, int64_t vocab_size,
+                                 void* scratch, int64_t scratch_bytes, mvsd_stream_t stream) {
+  if (num_rows < 0 || vocab_size <= 0) return MVSD_E_INVALID;
+  if (num_rows == 0 || (!top_k && !top_p)) return MVSD_OK;
+  if (!logits || logits_stride < vocab_size) return MVSD_E_INVALID;
+  if (vocab_size > 0x7fffffff || num_rows > 0x7fffffff) return MVSD_E_RANGE;
+  const int64_t need = mvsd::split_constraints_bytes(num_rows, vocab_size);
+  if (need == 0) return MVSD_E_RANGE;
+  if (!scratch || scratch_bytes < need || ((uintptr_t)scratch & 255) != 0) return MVSD_E_WORKSPACE;
   mvsd::VerifyParams p;
   memset(&p, 0, sizeof(p));
-  p.target = a->target_logits;
-  p.target_stride = a->target_stride;
-  p.target_rows = a->target_rows;
-  p.target_num_rows = a->target_num_rows;
-  p.cu = a->cu_num_draft_tokens;
-  p.temperature = a->temperature;
-  p.target_dtype = a->target_dtype;
-  p.all_greedy = a->all_greedy ? 1 : 0;
-  p.apply_temperature = a->apply_temperature ? 1 : 0;
-  p.B = (int)B;
-  p.P = (int)P;
-  p.V = (int)V;
-  p.top_k = a->top_k;
-  p.top_p = a->top_p;
-  p.masks = reinterpret_cast<float4*>(masks);
-  return hip_status(mvsd::launch_constraints(p, a->target_dtype, (hipStream_t)stream));
+  p.target = logits;
+  p.target_stride = logits_stride;
+  p.target_num_rows = num_rows;
+  p.target_dtype = MVSD_F32;
+  p.B = (int)num_rows;
+  p.P = (int)num_rows;
+  p.V = (int)vocab_size;
+  p.top_k = top_k;
+  p.top_p = top_p;
+  return hip_status(mvsd::launch_split_constraints(p, MVSD_F32, 0.f, false, true, scratch,
+                                                   (hipStream_t)stream));
 }
 
 int mvsd_apply_top_k_top_p(float* logits, int64_t logits_stride, const int64_t* top_k,

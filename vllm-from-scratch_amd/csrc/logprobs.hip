@@ -300,32 +300,6 @@ static int split_chunk(int64_t positions, int64_t V) {
   return wgs < 1024 && groups_short <= kMaxGroups ? kChunkShort : kChunkLong;
 }
 
-// Row maximum over each 16 lanes, in every lane.
-__device__ inline float max16(float v) {
-  v = fmaxf(v, dpp_f32<kDppXor1>(v));
-  v = fmaxf(v, dpp_f32<kDppXor2>(v));
-  v = fmaxf(v, dpp_f32<kDppHalfMirror>(v));
-  return fmaxf(v, dpp_f32<kDppMirror>(v));
-}
-
-// The vector at column col of a row of V columns, moved back where it would pass the row's end
-// (rows shorter than a vector: element by element), so that every lane issues the same load.
-// Element e is then column inside_col(col, e, V), or none of the vector's columns if that is -1.
-template <int DT>
-__device__ inline u32x4 load_vec_inside(const typename Elem<DT>::storage* row, int col, int V) {
-  constexpr int VEC = Elem<DT>::kVec;
-  if (V >= VEC) return load_vec_any<DT>(row + min(col, V - VEC));
-  typename Elem<DT>::storage e[VEC];
-#pragma unroll
-  for (int j = 0; j < VEC; ++j) e[j] = row[min(j, V - 1)];
-  return *reinterpret_cast<const u32x4_align2*>(e);
-}
-template <int DT>
-__device__ inline int inside_col(int col, int e, int V) {
-  const int i = min(col, max(V - Elem<DT>::kVec, 0)) + e;
-  return i >= col && i < V ? i : -1;
-}
-
 template <int DT, int NV>
 __global__ __launch_bounds__(kThreads) void lp_scan_kernel(LogprobParams p) {
   using S = typename Elem<DT>::storage;

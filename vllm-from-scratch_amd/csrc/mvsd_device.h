@@ -103,6 +103,24 @@ __device__ inline float vec_elem<MVSD_F16>(const u32x4& r, int j) {
   return static_cast<float>(__builtin_bit_cast(_Float16, (uint16_t)((j & 1) ? (w >> 16) : w)));
 }
 
+// The vector at column col of a row of V columns, moved back where it would pass the row's end
+// (rows shorter than a vector: element by element), so that every lane issues the same load.
+// Element e is then column inside_col(col, e, V), or none of the vector's columns if that is -1.
+template <int DT>
+__device__ inline u32x4 load_vec_inside(const typename Elem<DT>::storage* row, int col, int V) {
+  constexpr int VEC = Elem<DT>::kVec;
+  if (V >= VEC) return load_vec_any<DT>(row + min(col, V - VEC));
+  typename Elem<DT>::storage e[VEC];
+#pragma unroll
+  for (int j = 0; j < VEC; ++j) e[j] = row[min(j, V - 1)];
+  return *reinterpret_cast<const u32x4_align2*>(e);
+}
+template <int DT>
+__device__ inline int inside_col(int col, int e, int V) {
+  const int i = min(col, max(V - Elem<DT>::kVec, 0)) + e;
+  return i >= col && i < V ? i : -1;
+}
+
 // ------------------------------------------------------------------ comparisons ------
 
 // True when (a, ia) ranks above (b, ib): NaN above numbers, larger value, then lower index.
@@ -202,6 +220,14 @@ __device__ inline float wave_max(float v) {
   v = fmaxf(v, dpp_f32<kDppMirror>(v));
   return fmaxf(fmaxf(readlane_f32(v, 0), readlane_f32(v, 16)),
                fmaxf(readlane_f32(v, 32), readlane_f32(v, 48)));
+}
+
+// The maximum of each 16 lanes, in every one of them.
+__device__ inline float max16(float v) {
+  v = fmaxf(v, dpp_f32<kDppXor1>(v));
+  v = fmaxf(v, dpp_f32<kDppXor2>(v));
+  v = fmaxf(v, dpp_f32<kDppHalfMirror>(v));
+  return fmaxf(v, dpp_f32<kDppMirror>(v));
 }
 
 __device__ inline float wave_sum(float v) {
@@ -348,6 +374,25 @@ __device__ inline uint64_t wave_max_u64(uint64_t k) {
   k = umax64(k, dpp_u64<kDppMirror>(k));
   return umax64(umax64(readlane_u64(k, 0), readlane_u64(k, 16)),
                 umax64(readlane_u64(k, 32), readlane_u64(k, 48)));
+}
+
+__device__ inline uint32_t wave_max_u32(uint32_t v) {
+  v = max(v, (uint32_t)dpp_i32<kDppXor1>((int)v));
+  v = max(v, (uint32_t)dpp_i32<kDppXor2>((int)v));
+  v = max(v, (uint32_t)dpp_i32<kDppHalfMirror>((int)v));
+  v = max(v, (uint32_t)dpp_i32<kDppMirror>((int)v));
+  return max(max((uint32_t)__builtin_amdgcn_readlane((int)v, 0),
+                 (uint32_t)__builtin_amdgcn_readlane((int)v, 16)),
+             max((uint32_t)__builtin_amdgcn_readlane((int)v, 32),
+                 (uint32_t)__builtin_amdgcn_readlane((int)v, 48)));
+}
+
+__device__ inline uint64_t wave_sum_u64(uint64_t v) {
+  v += dpp_u64<kDppXor1>(v);
+  v += dpp_u64<kDppXor2>(v);
+  v += dpp_u64<kDppHalfMirror>(v);
+  v += dpp_u64<kDppMirror>(v);
+  return (readlane_u64(v, 0) + readlane_u64(v, 16)) + (readlane_u64(v, 32) + readlane_u64(v, 48));
 }
 
 // Per-row maximum of N keys over a block of NW wavefronts; only thread g (< N) receives row

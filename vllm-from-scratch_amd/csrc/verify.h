@@ -135,6 +135,15 @@ hipError_t launch_verify(const VerifyParams& params, int target_dtype, int grid,
 // With params.order set, a plan kernel first writes the masks of the rows that need no work
 // and lists the others heaviest first (random top-p, random top-k, greedy top-p).
 hipError_t launch_constraints(const VerifyParams& params, int target_dtype, hipStream_t stream);
+// The same masks (params.masks, or scratch of its own when that is null) with each row split over
+// workgroups.  The scratch holds split_constraints_bytes(rows, V) bytes, 256-byte aligned; 0 where
+// the split path does not apply (above 128 rows).  Without top-p, launch_constraints is as fast.  params.cu null: one row per request; params.temperature null:
+// no divide, no greedy row.  Rows whose temperature is 0 or below greedy_eps are greedy;
+// skip_greedy leaves them unmasked.  apply: masked entries of the (fp32) rows become -inf.
+int64_t split_constraints_bytes(int64_t rows, int64_t V);
+hipError_t launch_split_constraints(const VerifyParams& params, int target_dtype, float greedy_eps,
+                                    bool skip_greedy, bool apply, void* scratch,
+                                    hipStream_t stream);
 // Top-k / top-p masking in place on fp32 rows logits + r * stride, r < num_rows (one request
 // per row, no temperature): masked entries become -inf.  top_k [num_rows] int64 or null;
 // top_p [num_rows] fp32 or null.

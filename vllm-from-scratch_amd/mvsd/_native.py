@@ -129,6 +129,13 @@ SIGNATURES = {
                                                  c_void_p]),
     "mvsd_topk_scores": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p,
                                  c_int64, c_int64, c_int64, c_int, c_void_p]),
+    "mvsd_constraints_scratch_bytes": (c_int64, [c_int64, c_int64]),
+    "mvsd_rejection_sample_split": (c_int, [ctypes.POINTER(RejectionArgs), c_void_p, c_int64,
+                                            c_void_p]),
+    "mvsd_sampling_masks_split": (c_int, [ctypes.POINTER(RejectionArgs), c_void_p, c_void_p,
+                                          c_int64, c_void_p]),
+    "mvsd_apply_top_k_top_p_split": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64,
+                                             c_int64, c_void_p, c_int64, c_void_p]),
     "mvsd_logprobs_workspace_bytes": (c_int64, [c_int64, c_int64, c_int64]),
     "mvsd_spec_logprobs_split": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int64,
                                          c_void_p, c_void_p, c_int64, c_void_p, c_void_p,

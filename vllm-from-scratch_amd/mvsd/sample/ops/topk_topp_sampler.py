@@ -1,6 +1,7 @@
 """top-k / top-p masking (drop-in for minivllm/sample/ops/topk_topp_sampler.py:48-79).
 
-One HIP workgroup per row (``mvsd_apply_top_k_top_p``): the k-th largest value from the
+Rows split over workgroups (``mvsd_apply_top_k_top_p_split``, up to 128 rows with top-p) or one
+HIP workgroup per row (``mvsd_apply_top_k_top_p``): the k-th largest value from the
 entries at or above the k-th largest per-thread maximum, gathered and sorted in LDS; the
 top-p crossing from a logarithmic mass histogram and the entries of the crossing bin; then one
 masking pass -- no sort of the vocabulary.
@@ -41,8 +42,15 @@ def apply_top_k_top_p(logits: torch.Tensor, k: torch.Tensor | None,
         assert kk.numel() == n
     if pp is not None:
         assert pp.numel() == n
-    nat.check(nat.lib().mvsd_apply_top_k_top_p(
-        logits.data_ptr(), logits.stride(0), None if kk is None else kk.data_ptr(),
-        None if pp is None else pp.data_ptr(), n, V, nat.stream_of(device)),
-        "mvsd_apply_top_k_top_p")
+    handle = nat.lib()
+    size = 0 if pp is None else handle.mvsd_constraints_scratch_bytes(n, V)
+    if size > 0:
+        scratch = torch.empty(size, dtype=torch.uint8, device=device)
+        nat.check(handle.mvsd_apply_top_k_top_p_split(
+            logits.data_ptr(), logits.stride(0), nat.ptr(kk), nat.ptr(pp), n, V,
+            scratch.data_ptr(), size, nat.stream_of(device)), "mvsd_apply_top_k_top_p_split")
+    else:
+        nat.check(handle.mvsd_apply_top_k_top_p(
+            logits.data_ptr(), logits.stride(0), nat.ptr(kk), nat.ptr(pp), n, V,
+            nat.stream_of(device)), "mvsd_apply_top_k_top_p")
     return logits

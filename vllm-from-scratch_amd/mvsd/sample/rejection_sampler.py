@@ -681,8 +681,23 @@ def rejection_sample(
         top_p=nat.ptr(top_p),
         debug_row_stats=nat.ptr(debug_row_stats),
     )
-    nat.check(handle.mvsd_rejection_sample(args, stream), "mvsd_rejection_sample")
+    if top_k is None and top_p is None:
+        nat.check(handle.mvsd_rejection_sample(args, stream), "mvsd_rejection_sample")
+    else:
+        scratch = _constraints_scratch(num_tokens, vocab_size, top_p, device)
+        nat.check(handle.mvsd_rejection_sample_split(
+            args, nat.ptr(scratch), 0 if scratch is None else scratch.numel(), stream),
+            "mvsd_rejection_sample_split")
     return output_token_ids
+
+
+def _constraints_scratch(num_rows: int, vocab_size: int, top_p, device) -> torch.Tensor | None:
+    """Scratch of the sampling constraints' split path for one call; None where one workgroup
+    per row is as fast (no top-p, or more than 128 rows)."""
+    if top_p is None:
+        return None
+    size = nat.lib().mvsd_constraints_scratch_bytes(num_rows, vocab_size)
+    return torch.empty(size, dtype=torch.uint8, device=device) if size > 0 else None
 
 
 def sampling_masks(target_logits: torch.Tensor, cu_num_draft_tokens: torch.Tensor,
@@ -722,8 +737,10 @@ def sampling_masks(target_logits: torch.Tensor, cu_num_draft_tokens: torch.Tenso
         apply_temperature=int(bool(apply_temperature)), batch_size=batch_size,
         num_tokens=num_tokens, vocab_size=target_logits.shape[-1], top_k=nat.ptr(top_k),
         top_p=nat.ptr(top_p))
-    nat.check(nat.lib().mvsd_sampling_masks(args, masks.data_ptr(), nat.stream_of(device)),
-              "mvsd_sampling_masks")
+    scratch = _constraints_scratch(num_tokens, target_logits.shape[-1], top_p, device)
+    nat.check(nat.lib().mvsd_sampling_masks_split(
+        args, masks.data_ptr(), nat.ptr(scratch), 0 if scratch is None else scratch.numel(),
+        nat.stream_of(device)), "mvsd_sampling_masks_split")
     return masks
 
 
