@@ -257,6 +257,20 @@ int mvsd_rejection_sample_split(const mvsd_rejection_args* args, void* scratch,
 int mvsd_sampling_masks_split(const mvsd_rejection_args* args, float* masks, void* scratch,
                               int64_t scratch_bytes, mvsd_stream_t stream);
 
+/* step_masks — sampling_masks_split for a whole step: masks [num_tokens + batch_size, 4],   */
+/* the verify rows' first, then those of each request's bonus row (row bonus_rows[r] of     */
+/* target_logits).  Scratch for num_tokens + batch_size rows; MVSD_E_RANGE where the split   */
+/* path does not apply.  (sampling_masks_split also takes cu_num_draft_tokens NULL, one row  */
+/* per request.)                                                                           */
+int mvsd_step_masks(const mvsd_rejection_args* args, const int32_t* bonus_rows, float* masks,
+                    void* scratch, int64_t scratch_bytes, mvsd_stream_t stream);
+
+/* mvsd_rejection_sample with its verify rows' masks given ([num_tokens, 4], as              */
+/* mvsd_sampling_masks writes them; cleared by the call) in place of computing them; top_k   */
+/* and top_p still say whether constraints apply.                                           */
+int mvsd_rejection_sample_masked(const mvsd_rejection_args* args, float* masks,
+                                 mvsd_stream_t stream);
+
 int mvsd_apply_top_k_top_p_split(float* logits, int64_t logits_stride, const int64_t* top_k,
                                  const float* top_p, int64_t num_rows, int64_t vocab_size,
                                  void* scratch, int64_t scratch_bytes, mvsd_stream_t stream);
@@ -386,6 +400,13 @@ int mvsd_topk_scores_split(int64_t* ids, float* scores, int64_t* ranks, const vo
                            int64_t num_rows, int64_t vocab_size, int64_t k, int logits_mode,
                            void* workspace, int64_t workspace_bytes, mvsd_stream_t stream);
 
+/* spec_logprobs_split of rows that are their own positions: row r with token_ids[r].        */
+int mvsd_row_logprobs_split(int32_t* ids, float* lps, int32_t* ranks, const void* rows, int dtype,
+                            int64_t row_stride, const int32_t* token_ids, int64_t num_rows,
+                            int64_t vocab_size, int64_t k, int logits_mode, void* workspace,
+                            int64_t workspace_bytes, mvsd_stream_t stream);
+
+
 /* ------------------------------------------------------------------------------------ */
 /* sampler_rows — row operations of the regular sampler on fp32 rows x + r * stride.       */
 /* Replaces, in minivllm/sample/sampler.py: greedy_sample (:295-298, op 0: ids[r] = argmax */
@@ -437,6 +458,16 @@ int mvsd_sampler_race_rows(int32_t* ids, const void* x, int x_dtype, int64_t str
                            int64_t noise_stride, const float* temperature, float greedy_eps,
                            int64_t num_rows, int64_t vocab_size, void* workspace,
                            int64_t workspace_bytes, mvsd_stream_t stream);
+
+/* mvsd_sampler_race_rows with row r's entries restricted to those that masks[r] (as         */
+/* mvsd_sampling_masks writes them; NULL: all) keeps, except in rows that take their argmax. */
+int mvsd_sampler_race_rows_masked(int32_t* ids, const void* x, int x_dtype, int64_t stride,
+                                  const int32_t* row_index, int64_t num_x_rows,
+                                  const float* noise, int64_t noise_stride,
+                                  const float* temperature, float greedy_eps, const float* masks,
+                                  int64_t num_rows, int64_t vocab_size, void* workspace,
+                                  int64_t workspace_bytes, mvsd_stream_t stream);
+
 
 /* ------------------------------------------------------------------------------------ */
 /* selftest — on-device check of an arithmetic assumption of the kernels.  No counterpart   */

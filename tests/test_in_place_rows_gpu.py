@@ -1,0 +1,84 @@
+"""The sampler and RejectionSampler.forward on rows read in place (row masks, the masked race, raw
+rows' logprobs) against the general path, which writes the rows' fp32 copy, its quotient by the
+temperature and its masked entries: the same RNG state gives the same tokens, ids and ranks."""
+
+import pytest
+import torch
+
+from mvsd.sample import rejection_sampler as rs
+from mvsd.sample.sampler import Sampler
+from mvsd.testing.spec_metadata import make_metadata, sampling_metadata
+
+pytestmark = pytest.mark.gpu
+
+
+class General(Sampler):
+    """The sampler under another type, which takes the general path."""
+
+
+def params(n, V, limits, greedy, g):
+    temps = [0.0 if i % 4 < greedy else 0.5 + 0.1 * (i % 8) for i in range(n)]
+    top_k = top_p = None
+    if "k" in limits:
+        top_k = [V if i % 3 == 0 else 1 + 17 * i % 200 for i in range(n)]
+        top_k = [min(k, V) for k in top_k]
+    if "p" in limits:
+        top_p = [1.0 if i % 5 == 0 else 0.2 + 0.1 * (i % 8) for i in range(n)]
+    return temps, top_k, top_p
+
+
+def same(a, b, lp_atol):
+    assert torch.equal(a.sampled_token_ids, b.sampled_token_ids)
+    if b.logprobs_tensors is None:
+        assert a.logprobs_tensors is None
+        return
+    ids, lps, ranks = a.logprobs_tensors[:3]
+    want_ids, want_lps, want_ranks = b.logprobs_tensors[:3]
+    assert torch.equal(ids, want_ids) and torch.equal(ranks, want_ranks)
+    assert (lps - want_lps).abs().max() <= lp_atol
+
+
+# logprob values: one fp32 sum in two orders moves the log-sum and then each value (magnitude
+# below 32) by one rounding
+LP_ATOL = 2 * 2.0 ** -20
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("limits", ["", "k", "p", "kp"])
+@pytest.mark.parametrize("n,V,greedy", [(1, 9, 0), (6, 8193, 1), (5, 65537, 2), (129, 1000, 1),
+                                        (4, 2049, 4)])
+def test_sampler(device, dtype, limits, n, V, greedy):
+    g = torch.Generator(device=device).manual_seed(V)
+    logits = (torch.randn(n, V, device=device, generator=g) * 2.5).to(dtype)
+    temps, top_k, top_p = params(n, V, limits, greedy, g)
+    sm = sampling_metadata(temps, [[]] * n, device=device, top_k=top_k, top_p=top_p,
+                           max_num_logprobs=min(5, V))
+    for mode in ("raw_logprobs", "raw_logits"):
+        outs = []
+        for cls in (Sampler, General):
+            torch.manual_seed(7)
+            outs.append(cls(mode).forward(logits.clone(), sm))
+        same(*outs, LP_ATOL)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("limits", ["k", "p", "kp"])
+@pytest.mark.parametrize("V,B", [(4097, 6), (65600, 6), (66001, 40)])
+@pytest.mark.parametrize("greedy", [0, 2])
+def test_forward(device, dtype, limits, V, B, greedy):
+    """40 requests pass the split path's 128 rows; fewer share one call for verify and bonus rows."""
+    g = torch.Generator(device=device).manual_seed(V + B)
+    host = torch.Generator().manual_seed(V)
+    drafts = [torch.randint(0, V, (i % 5,), generator=host).tolist() for i in range(B)]
+    meta = make_metadata(drafts, device=device)
+    P = sum(len(d) for d in drafts)
+    logits = (torch.randn(P + B, V, device=device, generator=g) * 2.5).to(dtype)
+    probs = torch.softmax(torch.randn(P, V, device=device, generator=g) * 2.5, -1)
+    temps, top_k, top_p = params(B, V, limits, greedy, g)
+    sm = sampling_metadata(temps, drafts, device=device, top_k=top_k, top_p=top_p,
+                           max_num_logprobs=3)
+    outs = []
+    for cls in (Sampler, General):
+        torch.manual_seed(11)
+        outs.append(rs.RejectionSampler(cls()).forward(meta, probs, logits.clone(), sm))
+    same(*outs, LP_ATOL)

@@ -191,10 +191,11 @@ int mvsd_rejection_workspace_init(void* workspace, int64_t workspace_bytes, mvsd
 namespace {
 
 // mvsd_rejection_sample with the workspace `ws` of `ws_bytes` bytes (the args' workspace fields
-// are not read); with scratch, the sampling constraints' rows are split over workgroups.
+// are not read); with scratch, the sampling constraints' rows are split over workgroups; with
+// given_masks, the rows' masks are those (cleared as they are used).
 int rejection_sample_impl(const mvsd_rejection_args* a, void* ws_ptr, int64_t ws_bytes,
                           mvsd_stream_t stream, void* scratch = nullptr,
-                          int64_t scratch_bytes = 0) {
+                          int64_t scratch_bytes = 0, float* given_masks = nullptr) {
   if (!a) return MVSD_E_INVALID;
   const int64_t B = a->batch_size, P = a->num_tokens, V = a->vocab_size;
   if (B < 0 || P < 0 || V <= 0 || a->max_spec_len < 0) return MVSD_E_INVALID;
@@ -278,7 +279,8 @@ int rejection_sample_impl(const mvsd_rejection_args* a, void* ws_ptr, int64_t ws
   p.decision = reinterpret_cast<int*>(ws + lay.decision);
   p.top_k = masked ? a->top_k : nullptr;
   p.top_p = masked ? a->top_p : nullptr;
-  p.masks = masked ? reinterpret_cast<float4*>(ws + lay.masks) : nullptr;
+  p.masks = !masked ? nullptr
+                    : reinterpret_cast<float4*>(given_masks ? (char*)given_masks : ws + lay.masks);
   p.order = masked ? reinterpret_cast<int*>(ws + lay.order) : nullptr;
   p.stat_slots = reinterpret_cast<uint64_t*>(ws + lay.stat_slots);
   p.score_slots = reinterpret_cast<uint64_t*>(ws + lay.score_slots);
@@ -286,11 +288,11 @@ int rejection_sample_impl(const mvsd_rejection_args* a, void* ws_ptr, int64_t ws
 
   // The row masks of the whole batch, then one verify launch per kMaxLaunchRequests requests
   // (their tables live in LDS); the launches share the workspace, which each leaves zeroed.
-  if (masked) {
+  if (masked && !given_masks) {
     const int64_t need = scratch && p.top_p ? mvsd::split_constraints_bytes(P, V) : 0;
     if (need > 0 && (scratch_bytes < need || ((uintptr_t)scratch & 255) != 0))
       return MVSD_E_WORKSPACE;
-    err = need > 0 ? mvsd::launch_split_constraints(p, a->target_dtype, 0.f, false, false, scratch,
+    err = need > 0 ? mvsd::launch_split_constraints(p, a->target_dtype, nullptr, false, scratch,
                                                     (hipStream_t)stream)
                    : mvsd::launch_constraints(p, a->target_dtype, (hipStream_t)stream);
     if (err != hipSuccess) return hip_status(err);
@@ -341,19 +343,20 @@ int rejection_sample_impl(const mvsd_rejection_args* a, void* ws_ptr, int64_t ws
 }
 
 // mvsd_sampling_masks; with scratch, the rows are split over workgroups.
-int sampling_masks_impl(const mvsd_rejection_args* a, float* masks, void* scratch,
-                        int64_t scratch_bytes, mvsd_stream_t stream) {
+int sampling_masks_impl(const mvsd_rejection_args* a, const int32_t* bonus_rows, float* masks,
+                        bool need_cu, void* scratch, int64_t scratch_bytes, mvsd_stream_t stream) {
   if (!a || !masks) return MVSD_E_INVALID;
   const int64_t B = a->batch_size, P = a->num_tokens, V = a->vocab_size;
   if (B < 0 || P < 0 || V <= 0) return MVSD_E_INVALID;
   if (B > 0x7fffffff || P > 0x7fffffff || V > 0x7fffffff) return MVSD_E_RANGE;
-  if (P == 0) return MVSD_OK;
-  if (!a->target_logits || !a->cu_num_draft_tokens) return MVSD_E_INVALID;
+  if (P == 0 && !bonus_rows) return MVSD_OK;
+  if (!a->target_logits || (!a->cu_num_draft_tokens && (need_cu || P != B)))
+    return MVSD_E_INVALID;
   if (a->target_dtype != MVSD_F32 && a->target_dtype != MVSD_BF16 && a->target_dtype != MVSD_F16)
     return MVSD_E_INVALID;
   if (!a->all_greedy && !a->temperature) return MVSD_E_INVALID;
   if (a->target_stride < V) return MVSD_E_INVALID;
-  if (a->target_rows && a->target_num_rows < 1) return MVSD_E_INVALID;
+  if ((a->target_rows || bonus_rows) && a->target_num_rows < 1) return MVSD_E_INVALID;
   if ((uintptr_t)masks % 16 != 0) return MVSD_E_ALIGN;
   mvsd::VerifyParams p;
   memset(&p, 0, sizeof(p));
@@ -372,12 +375,14 @@ int sampling_masks_impl(const mvsd_rejection_args* a, float* masks, void* scratc
   p.top_k = a->top_k;
   p.top_p = a->top_p;
   p.masks = reinterpret_cast<float4*>(masks);
-  const int64_t need = scratch && p.top_p ? mvsd::split_constraints_bytes(P, V) : 0;
+  const int64_t need =
+      scratch && p.top_p ? mvsd::split_constraints_bytes(P + (bonus_rows ? B : 0), V) : 0;
   if (need > 0) {
     if (scratch_bytes < need || ((uintptr_t)scratch & 255) != 0) return MVSD_E_WORKSPACE;
-    return hip_status(mvsd::launch_split_constraints(p, a->target_dtype, 0.f, false, false,
+    return hip_status(mvsd::launch_split_constraints(p, a->target_dtype, bonus_rows, false,
                                                      scratch, (hipStream_t)stream));
   }
+  if (bonus_rows) return MVSD_E_RANGE;
   return hip_status(mvsd::launch_constraints(p, a->target_dtype, (hipStream_t)stream));
 }
 
@@ -436,6 +441,14 @@ int mvsd_rejection_sample_split(const mvsd_rejection_args* a, void* scratch, int
                                 mvsd_stream_t stream) {
   if (!a) return MVSD_E_INVALID;
   return rejection_sample_impl(a, a->workspace, a->workspace_bytes, stream, scratch, scratch_bytes);
+}
+
+int mvsd_rejection_sample_masked(const mvsd_rejection_args* a, float* masks,
+                                 mvsd_stream_t stream) {
+  if (!a) return MVSD_E_INVALID;
+  if (a->num_tokens > 0 && !masks) return MVSD_E_INVALID;
+  if ((uintptr_t)masks % 16 != 0) return MVSD_E_ALIGN;
+  return rejection_sample_impl(a, a->workspace, a->workspace_bytes, stream, nullptr, 0, masks);
 }
 
 int64_t mvsd_rejection_static_scratch_bytes(void) { return kStaticScratchBytes; }
@@ -640,6 +653,37 @@ int mvsd_topk_scores_split(int64_t* ids, float* scores, int64_t* ranks, const vo
   return hip_status(mvsd::launch_split_logprobs(p, dtype, workspace, (hipStream_t)stream));
 }
 
+int mvsd_row_logprobs_split(int32_t* ids, float* lps, int32_t* ranks, const void* rows, int dtype,
+                            int64_t row_stride, const int32_t* token_ids, int64_t num_rows,
+                            int64_t vocab_size, int64_t k, int logits_mode, void* workspace,
+                            int64_t workspace_bytes, mvsd_stream_t stream) {
+  if (num_rows < 0 || vocab_size <= 0 || k < 0) return MVSD_E_INVALID;
+  if (num_rows == 0) return MVSD_OK;
+  if (k > vocab_size) return MVSD_E_RANGE;
+  if (num_rows > 0x7fffffff || vocab_size > 0x7fffffff) return MVSD_E_RANGE;
+  if (dtype != MVSD_F32 && dtype != MVSD_BF16 && dtype != MVSD_F16) return MVSD_E_INVALID;
+  if (!ids || !lps || !ranks || !rows || !token_ids || row_stride < vocab_size)
+    return MVSD_E_INVALID;
+  const int64_t need = mvsd::split_logprobs_workspace_bytes(num_rows, vocab_size, k);
+  if (need == 0) return MVSD_E_RANGE;
+  if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15) != 0)
+    return MVSD_E_WORKSPACE;
+  mvsd::LogprobParams p{};
+  p.bonus = rows;
+  p.bstride = row_stride;
+  p.tokens = token_ids;
+  p.B = (int)num_rows;
+  p.W = 1;
+  p.V = (int)vocab_size;
+  p.k = (int)k;
+  p.logits_mode = logits_mode ? 1 : 0;
+  p.flat = 1;
+  p.ids = ids;
+  p.lps = lps;
+  p.ranks = ranks;
+  return hip_status(mvsd::launch_split_logprobs(p, dtype, workspace, (hipStream_t)stream));
+}
+
 int mvsd_sampler_rows(int op, int32_t* ids, float* out, int64_t out_stride, float* x,
                       int64_t stride, const float* aux, int64_t aux_stride, int64_t num_rows,
                       int64_t vocab_size, mvsd_stream_t stream) {
@@ -677,6 +721,16 @@ int mvsd_sampler_race_rows(int32_t* ids, const void* x, int x_dtype, int64_t str
                            int64_t noise_stride, const float* temperature, float greedy_eps,
                            int64_t num_rows, int64_t vocab_size, void* workspace,
                            int64_t workspace_bytes, mvsd_stream_t stream) {
+  return mvsd_sampler_race_rows_masked(ids, x, x_dtype, stride, row_index, num_x_rows, noise,
+                                       noise_stride, temperature, greedy_eps, nullptr, num_rows,
+                                       vocab_size, workspace, workspace_bytes, stream);
+}
+
+int mvsd_sampler_race_rows_masked(int32_t* ids, const void* x, int x_dtype, int64_t stride,
+                                  const int32_t* row_index, int64_t num_x_rows, const float* noise,
+                           int64_t noise_stride, const float* temperature, float greedy_eps, const float* masks,
+                           int64_t num_rows, int64_t vocab_size, void* workspace,
+                           int64_t workspace_bytes, mvsd_stream_t stream) {
   if (num_rows < 0 || vocab_size <= 0) return MVSD_E_INVALID;
   if (num_rows == 0) return MVSD_OK;
   if (x_dtype != MVSD_F32 && x_dtype != MVSD_BF16 && x_dtype != MVSD_F16) return MVSD_E_INVALID;
@@ -687,10 +741,11 @@ int mvsd_sampler_race_rows(int32_t* ids, const void* x, int x_dtype, int64_t str
     return MVSD_E_INVALID;
   if (row_index ? num_x_rows <= 0 : num_x_rows < num_rows) return MVSD_E_INVALID;
   if (!(greedy_eps >= 0.0f)) return MVSD_E_INVALID;
+  if ((uintptr_t)masks % 16 != 0) return MVSD_E_ALIGN;
   if (!workspace || workspace_bytes < mvsd::sampler_race_workspace_bytes(num_rows, vocab_size))
     return MVSD_E_WORKSPACE;
   return hip_status(mvsd::launch_sampler_race(ids, x, x_dtype, stride, row_index, num_x_rows,
-                                              noise, noise_stride, temperature, greedy_eps,
+                                              noise, noise_stride, temperature, greedy_eps, masks,
                                               num_rows, vocab_size, workspace,
                                               (hipStream_t)stream));
 }
@@ -712,12 +767,18 @@ int mvsd_selftest(int test, uint64_t* failures, mvsd_stream_t stream) {
 }
 
 int mvsd_sampling_masks(const mvsd_rejection_args* a, float* masks, mvsd_stream_t stream) {
-  return sampling_masks_impl(a, masks, nullptr, 0, stream);
+  return sampling_masks_impl(a, nullptr, masks, true, nullptr, 0, stream);
 }
 
 int mvsd_sampling_masks_split(const mvsd_rejection_args* a, float* masks, void* scratch,
                               int64_t scratch_bytes, mvsd_stream_t stream) {
-  return sampling_masks_impl(a, masks, scratch, scratch_bytes, stream);
+  return sampling_masks_impl(a, nullptr, masks, false, scratch, scratch_bytes, stream);
+}
+
+int mvsd_step_masks(const mvsd_rejection_args* a, const int32_t* bonus_rows, float* masks,
+                    void* scratch, int64_t scratch_bytes, mvsd_stream_t stream) {
+  if (!bonus_rows) return MVSD_E_INVALID;
+  return sampling_masks_impl(a, bonus_rows, masks, true, scratch, scratch_bytes, stream);
 }
 
 int mvsd_apply_top_k_top_p_split(float* logits, int64_t logits_stride, const int64_t* top_k,
@@ -741,7 +802,7 @@ int mvsd_apply_top_k_top_p_split(float* logits, int64_t logits_stride, const int
   p.V = (int)vocab_size;
   p.top_k = top_k;
   p.top_p = top_p;
-  return hip_status(mvsd::launch_split_constraints(p, MVSD_F32, 0.f, false, true, scratch,
+  return hip_status(mvsd::launch_split_constraints(p, MVSD_F32, nullptr, true, scratch,
                                                    (hipStream_t)stream));
 }
 

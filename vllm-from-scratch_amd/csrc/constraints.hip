@@ -554,16 +554,16 @@ __device__ inline int greedy_tied_top_p(const typename Elem<DT>::storage* __rest
   return 1;
 }
 
-// The row's mask (A, B, J) from its request's top-k / top-p; false when nothing is masked.
+// The mask (A, B, J) of target row xrow from request r's top-k / top-p (r < 0: none); false when
+// nothing is masked.
 template <int DT>
-__device__ __forceinline__ bool row_thresholds(const VerifyParams& p, int row, ConstraintSmem& sm, float& A,
-                               float& Bv, int& J) {
+__device__ __forceinline__ bool row_thresholds(const VerifyParams& p, int r, int64_t xrow,
+                                               ConstraintSmem& sm, float& A, float& Bv, int& J) {
   using S = typename Elem<DT>::storage;
   const int tid = threadIdx.x;
   A = -INFINITY;
   Bv = -INFINITY;
   J = -1;
-  const int r = request_of(p, row);
   if (p.all_greedy || r < 0) return false;
   const int64_t kk = p.top_k ? p.top_k[r] : (int64_t)p.V;
   const float t = p.top_p ? 1.0f - p.top_p[r] : 0.f;
@@ -581,7 +581,7 @@ __device__ __forceinline__ bool row_thresholds(const VerifyParams& p, int row, C
   const float T = req_temperature(p, r);
   const Divider dv = make_divider(T);
   const int V = p.V;
-  const S* x = static_cast<const S*>(p.target) + target_row(p, row) * p.target_stride;
+  const S* x = static_cast<const S*>(p.target) + xrow * p.target_stride;
 
   // ---- pass 1: row maximum and per-thread maxima (ordered keys of the raw values); rows with
   // top-k only also keep each thread's four largest keys ----
@@ -928,7 +928,7 @@ __global__ __launch_bounds__(kCT) void constraints_kernel(VerifyParams p) {
   }
   float A, Bv;
   int J;
-  const bool any = row_thresholds<DT>(p, row, sm, A, Bv, J);
+  const bool any = row_thresholds<DT>(p, request_of(p, row), target_row(p, row), sm, A, Bv, J);
   if constexpr (!WRITE) {
     if (threadIdx.x == 0) p.masks[row] = make_float4(A, Bv, __int_as_float(J), 0.f);
   } else {
@@ -1006,7 +1006,7 @@ struct SplitRow {
   uint32_t mkey;
   unsigned long long ties;
   int count;      // candidates listed by split_mass
-  int pad;
+  int req;        // request of the row
 };
 static_assert(sizeof(SplitRow) == 64, "row descriptor layout");
 
@@ -1017,8 +1017,7 @@ struct SplitHead {
 
 struct SplitParams {
   VerifyParams p;
-  float greedy_eps;  // rows whose temperature is 0 or below this are greedy
-  int skip_greedy;   // greedy rows need no mask
+  const int32_t* bonus_rows;  // [B] target row of each request's bonus row, mask P + r; or null
   int nch;
   SplitHead* head;
   SplitRow* rows;                // [P]
@@ -1040,10 +1039,10 @@ __device__ inline int split_class(const SplitParams& sp, int r, int& k, float& t
   k = kk > 0 && kk < p.V ? (int)kk : 0;
   t = p.top_p ? fmaxf(1.0f - p.top_p[r], 0.f) : 0.f;  // p >= 1 (or NaN) keeps every entry
   const float temp = p.temperature ? p.temperature[r] : 1.f;
-  greedy = p.temperature != nullptr && (temp == 0.f || temp < sp.greedy_eps);
+  greedy = p.temperature != nullptr && temp == 0.f;
   T = p.temperature && p.apply_temperature && !greedy ? temp : 1.f;
   if (k == 0 && !(t > 0.f)) return 0;
-  if (greedy && (sp.skip_greedy || !(t > 0.f))) return 0;
+  if (greedy && !(t > 0.f)) return 0;
   return k > 0 ? 2 : 1;
 }
 
@@ -1066,10 +1065,12 @@ __global__ __launch_bounds__(1024) void split_plan_kernel(SplitParams sp) {
     int begin, end;
     span(r, begin, end);
     const int c = split_class(sp, r, k, t, T, greedy);
+    const int n = max(end - begin, 0) + (sp.bonus_rows ? 1 : 0);
     if (c == 0) {
       for (int j = begin; j < end; ++j) p.masks[j] = neutral;
-    } else if (end > begin) {
-      atomicAdd(&cnt[c], end - begin);
+      if (sp.bonus_rows) p.masks[p.P + r] = neutral;
+    } else if (n > 0) {
+      atomicAdd(&cnt[c], n);
     }
   }
   __syncthreads();
@@ -1085,17 +1086,20 @@ __global__ __launch_bounds__(1024) void split_plan_kernel(SplitParams sp) {
     int begin, end;
     span(r, begin, end);
     const int c = split_class(sp, r, k, t, T, greedy);
-    if (c == 0 || end <= begin) continue;
-    const int at = atomicAdd(&cnt[c], end - begin);
-    for (int j = begin; j < end; ++j) {
+    const int n = max(end - begin, 0) + (sp.bonus_rows ? 1 : 0);
+    if (c == 0 || n == 0) continue;
+    const int at = atomicAdd(&cnt[c], n);
+    for (int u = 0; u < n; ++u) {
+      const int j = begin + u;
       SplitRow d{};
-      d.row = j;
-      d.xrow = target_row(p, j);
+      d.row = j < end ? j : p.P + r;
+      d.xrow = j < end ? target_row(p, j) : clamped_row(p, sp.bonus_rows[r]);
+      d.req = r;
       d.k = k;
       d.t = t;
       d.T = T;
       d.greedy = greedy;
-      sp.rows[at + (j - begin)] = d;
+      sp.rows[at + u] = d;
     }
   }
 }
@@ -1767,7 +1771,7 @@ __global__ __launch_bounds__(kCT) void split_finish_kernel(SplitParams sp) {
   float A, Bv;
   int J;
   __syncthreads();
-  row_thresholds<DT>(sp.p, d.row, sm, A, Bv, J);
+  row_thresholds<DT>(sp.p, d.req, d.xrow, sm, A, Bv, J);
   write(A, Bv, J);
 }
 
@@ -1861,8 +1865,8 @@ template <int DT>
 void launch_split_dt(const SplitParams& sp, int chunk, hipStream_t stream) {
   constexpr int kLong = kSplitLong / (kSplitThreads * Elem<DT>::kVec);
   constexpr int kShort = kSplitShort / (kSplitThreads * Elem<DT>::kVec);
-  const int64_t items = (int64_t)sp.p.P * sp.nch;
-  const dim3 rows((unsigned)sp.p.P), slots((unsigned)(items < kSplitGrid ? items : kSplitGrid));
+  const int64_t n = sp.p.P + (sp.bonus_rows ? sp.p.B : 0), items = n * sp.nch;
+  const dim3 rows((unsigned)n), slots((unsigned)(items < kSplitGrid ? items : kSplitGrid));
   const dim3 block(kSplitThreads), wide(kCT);
   const unsigned lds = (unsigned)sp.nch * (unsigned)(chunk / kSplitGroup) * 2;
   if (chunk == kSplitLong) {
@@ -1883,19 +1887,19 @@ int64_t split_constraints_bytes(int64_t rows, int64_t V) {
   return rows > 0 && V > 0 && split_rows(rows, V) ? split_layout(rows, V).total : 0;
 }
 
-hipError_t launch_split_constraints(const VerifyParams& params, int target_dtype, float greedy_eps,
-                                    bool skip_greedy, bool apply, void* scratch,
+hipError_t launch_split_constraints(const VerifyParams& params, int target_dtype,
+                                    const int32_t* bonus_rows, bool apply, void* scratch,
                                     hipStream_t stream) {
-  if (params.P == 0) return hipSuccess;
-  const SplitLayout l = split_layout(params.P, params.V);
+  const int64_t n = params.P + (bonus_rows ? params.B : 0);
+  if (n == 0) return hipSuccess;
+  const SplitLayout l = split_layout(n, params.V);
   char* ws = static_cast<char*>(scratch);
   SplitParams sp;
   memset(&sp, 0, sizeof(sp));
   sp.p = params;
   sp.p.order = nullptr;
   if (!sp.p.masks) sp.p.masks = reinterpret_cast<float4*>(ws + l.masks);
-  sp.greedy_eps = greedy_eps;
-  sp.skip_greedy = skip_greedy ? 1 : 0;
+  sp.bonus_rows = bonus_rows;
   sp.nch = l.nch;
   sp.head = reinterpret_cast<SplitHead*>(ws + l.head);
   sp.rows = reinterpret_cast<SplitRow*>(ws + l.rows);

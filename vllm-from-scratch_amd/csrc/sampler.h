@@ -25,10 +25,12 @@ int64_t sampler_race_workspace_bytes(int64_t rows, int64_t V);
 // (or x_r[i] when temperature is null), evaluated as argmax of v log2(e) - log2(noise[r][i]);
 // rows whose temperature is below greedy_eps, and every row when noise is null, take the
 // argmax of the raw row.  x_r = x + row_index[r] * stride (clamped to [0, num_x_rows)) or
-// x + r * stride; x is x_dtype (MVSD_F32 / MVSD_BF16 / MVSD_F16).
+// x + r * stride; x is x_dtype (MVSD_F32 / MVSD_BF16 / MVSD_F16).  masks (null: none): row r's
+// entries that masks[r] (verify.h) masks score -inf, unless the row takes its argmax.
 hipError_t launch_sampler_race(int32_t* ids, const void* x, int x_dtype, int64_t stride,
                                const int32_t* row_index, int64_t num_x_rows, const float* noise,
                                int64_t noise_stride, const float* temperature, float greedy_eps,
-                               int64_t rows, int64_t V, void* workspace, hipStream_t stream);
+                               const float* masks, int64_t rows, int64_t V, void* workspace,
+                               hipStream_t stream);
 
 }  // namespace mvsd

@@ -6,14 +6,15 @@
 // one 256-thread workgroup per row; and the exponential race of random_sample (argmax of
 // softmax(x / T) / E per row) in one pass over 8192-column chunks of every row:
 //   race_kernel  each chunk's best key of v log2(e) - log2(E), v = fl(x / T) or x (the
-//                argmax of softmax(v) / E, whose max and sum are common to the row), or of x
-//                for greedy rows
+//                argmax of softmax(v) / E, whose max and sum are common to the row) over the
+//                entries its constraint mask keeps, or of x for greedy rows
 //   race_pick    one wavefront per row takes the best chunk key
 // Rows are fp32 (or, for the race, bf16 / fp16 upcast in the kernel) with unit column stride.
 #include <type_traits>
 
 #include "mvsd_device.h"
 #include "sampler.h"
+#include "verify.h"
 
 namespace mvsd {
 
@@ -108,11 +109,12 @@ __device__ inline float4 f32x4_of(u32x4 q) {
                      __uint_as_float(q[3]));
 }
 
-template <int DT>
-using RaceQuad = std::conditional_t<Elem<DT>::kVec == 4, u32x4, u32x2>;
+typedef u32x2 u32x2_align2 __attribute__((aligned(2)));
 
-// 4 consecutive columns of a DT row starting at column i (16-byte aligned for fp32, 8-byte
-// for 16-bit types), as fp32.
+template <int DT>
+using RaceQuad = std::conditional_t<Elem<DT>::kVec == 4, u32x4_align4, u32x2_align2>;
+
+// 4 consecutive columns of a DT row starting at column i (any alignment), as fp32.
 template <int DT>
 __device__ inline void race_load4(const typename Elem<DT>::storage* row, int i, float (&v)[4]) {
   using S = typename Elem<DT>::storage;
@@ -122,27 +124,54 @@ __device__ inline void race_load4(const typename Elem<DT>::storage* row, int i, 
   for (int j = 0; j < 4; ++j) v[j] = Elem<DT>::cvt(s[j]);
 }
 
-template <int DT, int MODE, bool VEC>
+// The chunk's best key.  Bound by reading the row and its noise (56 us for 256 fp32 rows of
+// 151936 columns, 5.6 TB/s); for a few rows by the round trips.  MASKED: entries masked by the row's constraints (m) take no part, and a
+// quad of which the whole wave has only masked entries reads no noise (on a top-k row, nearly all).
+template <int DT, int MODE, bool MASKED>
 __device__ inline uint64_t race_chunk(const typename Elem<DT>::storage* row, const float* e,
-                                      int begin, int end, const Divider& dv) {
+                                      int begin, int end, const Divider& dv, const float4& m) {
   uint64_t best = 0;
   bool nan_row = false;
   auto score = [&](float xv, float ev, int i) {
     if constexpr (MODE == kRaceGreedy) {
       best = umax64(best, argmax_key(xv, i));
     } else {
+      if (MASKED && row_masked(m, xv, i)) return;
       const float v = MODE == kRaceDivide ? divide(dv, xv) : xv;
       nan_row |= (v != v) | (v == INFINITY);
       const float key = fmaf(v, kLog2e, -__builtin_amdgcn_logf(ev));
       best = umax64(best, argmax_key(key, i));
     }
   };
+  // 4 columns per lane and step: one 16-byte (fp32) or 8-byte (16-bit) load of the row and one
+  // 16-byte load of the noise
+  constexpr int kStep = 4 * kSmpThreads;
+  const int vend = begin + ((end - begin) & ~(kStep - 1));
   int i = begin;
-  if (VEC) {
-    // 4 columns per lane and step: one 16-byte (fp32) or 8-byte (16-bit) load of the row and
-    // one 16-byte load of the noise
-    constexpr int kStep = 4 * kSmpThreads;
-    const int vend = begin + ((end - begin) & ~(kStep - 1));
+  if constexpr (MASKED && MODE != kRaceGreedy) {
+    constexpr int U = kRaceChunk / kStep;  // the whole chunk: one round trip, then the noise's
+    for (; i < vend; i += U * kStep) {
+      float xv[U][4];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        race_load4<DT>(row, min(i + u * kStep, vend - kStep) + 4 * threadIdx.x, xv[u]);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (i + u * kStep >= vend) break;
+        const int j = i + u * kStep + 4 * threadIdx.x;
+        bool live = false;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) live |= !row_masked(m, xv[u][q], j + q);
+        if (!live) continue;
+        const float4 ev = f32x4_of(*reinterpret_cast<const u32x4_align4*>(e + j));
+        score(xv[u][0], ev.x, j);
+        score(xv[u][1], ev.y, j + 1);
+        score(xv[u][2], ev.z, j + 2);
+        score(xv[u][3], ev.w, j + 3);
+      }
+    }
+    i = vend;
+  } else {
 #pragma unroll 4
     for (; i < vend; i += kStep) {
       const int j = i + 4 * threadIdx.x;
@@ -150,7 +179,7 @@ __device__ inline uint64_t race_chunk(const typename Elem<DT>::storage* row, con
       race_load4<DT>(row, j, xv);
       float4 ev = make_float4(1.f, 1.f, 1.f, 1.f);  // greedy rows read no noise
       if constexpr (MODE != kRaceGreedy)
-        ev = f32x4_of(__builtin_nontemporal_load(reinterpret_cast<const u32x4*>(e + j)));
+        ev = f32x4_of(__builtin_nontemporal_load(reinterpret_cast<const u32x4_align4*>(e + j)));
       score(xv[0], ev.x, j);
       score(xv[1], ev.y, j + 1);
       score(xv[2], ev.z, j + 2);
@@ -166,12 +195,13 @@ __device__ inline uint64_t race_chunk(const typename Elem<DT>::storage* row, con
 
 // One workgroup per (row r, chunk c of kRaceChunk columns): keys[r * nch + c] = the chunk's
 // best key.  Row r is x + row_index[r] * stride, the index clamped to [0, num_x_rows) (or
-// x + r * stride).  Without noise every row is greedy.
-template <int DT, bool VEC>
+// x + r * stride).  Without noise every row is greedy.  masks (or null): the row masks of the
+// sampling constraints, which greedy rows ignore.
+template <int DT>
 __global__ __launch_bounds__(kSmpThreads) void race_kernel(
     uint64_t* keys, const void* x, int64_t stride, const int32_t* row_index, int64_t num_x_rows,
-    const float* noise, int64_t noise_stride, const float* temperature, float greedy_eps, int V,
-    int nch) {
+    const float* noise, int64_t noise_stride, const float* temperature, float greedy_eps,
+    const float4* masks, int V, int nch) {
   using S = typename Elem<DT>::storage;
   __shared__ uint64_t s_k[kSmpWaves];
   const int r = blockIdx.x / nch, c = blockIdx.x % nch;
@@ -182,11 +212,17 @@ __global__ __launch_bounds__(kSmpThreads) void race_kernel(
   const int begin = c * kRaceChunk, end = min(V, begin + kRaceChunk);
   const float T = temperature ? temperature[r] : 1.f;
   const Divider dv = make_divider(T);
+  const float4 m = masks ? masks[r] : make_float4(-INFINITY, -INFINITY, 0.f, 0.f);
+  const bool masked = m.x != -INFINITY || m.y != -INFINITY;
   uint64_t best;
   if (!noise || (temperature && T < greedy_eps))
-    best = race_chunk<DT, kRaceGreedy, VEC>(row, e, begin, end, dv);
-  else if (!temperature) best = race_chunk<DT, kRaceMode, VEC>(row, e, begin, end, dv);
-  else best = race_chunk<DT, kRaceDivide, VEC>(row, e, begin, end, dv);
+    best = race_chunk<DT, kRaceGreedy, false>(row, e, begin, end, dv, m);
+  else if (!temperature)
+    best = masked ? race_chunk<DT, kRaceMode, true>(row, e, begin, end, dv, m)
+                  : race_chunk<DT, kRaceMode, false>(row, e, begin, end, dv, m);
+  else
+    best = masked ? race_chunk<DT, kRaceDivide, true>(row, e, begin, end, dv, m)
+                  : race_chunk<DT, kRaceDivide, false>(row, e, begin, end, dv, m);
   const uint64_t w = wave_max_u64(best);
   if (lane_id() == 0) s_k[wave_id()] = w;
   __syncthreads();
@@ -256,17 +292,11 @@ int64_t sampler_race_workspace_bytes(int64_t rows, int64_t V) {
 template <int DT>
 static void launch_race_dt(int32_t* ids, const void* x, int64_t stride, const int32_t* row_index,
                            int64_t num_x_rows, const float* noise, int64_t noise_stride,
-                           const float* temperature, float greedy_eps, int64_t rows, int V,
-                           int nch, uint64_t* keys, bool vec, hipStream_t stream) {
+                           const float* temperature, float greedy_eps, const float4* masks,
+                           int64_t rows, int V, int nch, uint64_t* keys, hipStream_t stream) {
   const dim3 grid((unsigned)(rows * nch)), block(kSmpThreads);
-  if (vec)
-    hipLaunchKernelGGL((race_kernel<DT, true>), grid, block, 0, stream, keys, x, stride,
-                       row_index, num_x_rows, noise, noise_stride, temperature, greedy_eps, V,
-                       nch);
-  else
-    hipLaunchKernelGGL((race_kernel<DT, false>), grid, block, 0, stream, keys, x, stride,
-                       row_index, num_x_rows, noise, noise_stride, temperature, greedy_eps, V,
-                       nch);
+  hipLaunchKernelGGL((race_kernel<DT>), grid, block, 0, stream, keys, x, stride, row_index,
+                     num_x_rows, noise, noise_stride, temperature, greedy_eps, masks, V, nch);
   hipLaunchKernelGGL(race_pick_kernel, dim3((unsigned)((rows + kSmpWaves - 1) / kSmpWaves)),
                      block, 0, stream, ids, keys, rows, nch, V);
 }
@@ -274,27 +304,24 @@ static void launch_race_dt(int32_t* ids, const void* x, int64_t stride, const in
 hipError_t launch_sampler_race(int32_t* ids, const void* x, int x_dtype, int64_t stride,
                                const int32_t* row_index, int64_t num_x_rows, const float* noise,
                                int64_t noise_stride, const float* temperature, float greedy_eps,
-                               int64_t rows, int64_t V, void* workspace, hipStream_t stream) {
+                               const float* masks, int64_t rows, int64_t V, void* workspace,
+                               hipStream_t stream) {
   if (rows <= 0) return hipSuccess;
   const int nch = (int)((V + kRaceChunk - 1) / kRaceChunk);
   uint64_t* keys = static_cast<uint64_t*>(workspace);
-  const int esize = x_dtype == MVSD_F32 ? 4 : 2;
-  // every 4-column quad of every row is aligned (16 bytes for fp32 rows, 8 for 16-bit rows)
-  // and so is every noise quad; greedy-only calls may pass no noise
-  const bool vec = (reinterpret_cast<uintptr_t>(x) & (4 * esize - 1)) == 0 && stride % 4 == 0 &&
-                   (reinterpret_cast<uintptr_t>(noise) & 15) == 0 && noise_stride % 4 == 0;
+  const float4* mk = reinterpret_cast<const float4*>(masks);
   switch (x_dtype) {
     case MVSD_F32:
       launch_race_dt<MVSD_F32>(ids, x, stride, row_index, num_x_rows, noise, noise_stride,
-                               temperature, greedy_eps, rows, (int)V, nch, keys, vec, stream);
+                               temperature, greedy_eps, mk, rows, (int)V, nch, keys, stream);
       break;
     case MVSD_BF16:
       launch_race_dt<MVSD_BF16>(ids, x, stride, row_index, num_x_rows, noise, noise_stride,
-                                temperature, greedy_eps, rows, (int)V, nch, keys, vec, stream);
+                                temperature, greedy_eps, mk, rows, (int)V, nch, keys, stream);
       break;
     case MVSD_F16:
       launch_race_dt<MVSD_F16>(ids, x, stride, row_index, num_x_rows, noise, noise_stride,
-                               temperature, greedy_eps, rows, (int)V, nch, keys, vec, stream);
+                               temperature, greedy_eps, mk, rows, (int)V, nch, keys, stream);
       break;
     default:
       return hipErrorInvalidValue;

@@ -86,10 +86,11 @@ struct VerifyParams {
 };
 
 // Verify row j's row in the target tensor: target_rows[j] clamped to the tensor, or j.
-__device__ inline int64_t target_row(const VerifyParams& p, int row) {
-  if (!p.target_rows) return row;
-  const int64_t t = p.target_rows[row];
+__device__ inline int64_t clamped_row(const VerifyParams& p, int64_t t) {
   return t < 0 ? 0 : (t >= p.target_num_rows ? p.target_num_rows - 1 : t);
+}
+__device__ inline int64_t target_row(const VerifyParams& p, int row) {
+  return p.target_rows ? clamped_row(p, p.target_rows[row]) : row;
 }
 
 __device__ inline bool req_is_greedy(const VerifyParams& p, int r) {
@@ -138,11 +139,12 @@ hipError_t launch_constraints(const VerifyParams& params, int target_dtype, hipS
 // The same masks (params.masks, or scratch of its own when that is null) with each row split over
 // workgroups.  The scratch holds split_constraints_bytes(rows, V) bytes, 256-byte aligned; 0 where
 // the split path does not apply (above 128 rows).  Without top-p, launch_constraints is as fast.  params.cu null: one row per request; params.temperature null:
-// no divide, no greedy row.  Rows whose temperature is 0 or below greedy_eps are greedy;
-// skip_greedy leaves them unmasked.  apply: masked entries of the (fp32) rows become -inf.
+// no divide, no greedy row.  bonus_rows (or null) adds request r's bonus row, target row
+// bonus_rows[r], as row P + r of the masks (P + B rows in all).  apply: masked entries of the
+// (fp32) rows become -inf.
 int64_t split_constraints_bytes(int64_t rows, int64_t V);
-hipError_t launch_split_constraints(const VerifyParams& params, int target_dtype, float greedy_eps,
-                                    bool skip_greedy, bool apply, void* scratch,
+hipError_t launch_split_constraints(const VerifyParams& params, int target_dtype,
+                                    const int32_t* bonus_rows, bool apply, void* scratch,
                                     hipStream_t stream);
 // Top-k / top-p masking in place on fp32 rows logits + r * stride, r < num_rows (one request
 // per row, no temperature): masked entries become -inf.  top_k [num_rows] int64 or null;

@@ -136,6 +136,16 @@ SIGNATURES = {
                                           c_int64, c_void_p]),
     "mvsd_apply_top_k_top_p_split": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64,
                                              c_int64, c_void_p, c_int64, c_void_p]),
+    "mvsd_step_masks": (c_int, [ctypes.POINTER(RejectionArgs), c_void_p, c_void_p, c_void_p,
+                                c_int64, c_void_p]),
+    "mvsd_rejection_sample_masked": (c_int, [ctypes.POINTER(RejectionArgs), c_void_p, c_void_p]),
+    "mvsd_sampler_race_rows_masked": (c_int, [c_void_p, c_void_p, c_int, c_int64, c_void_p,
+                                              c_int64, c_void_p, c_int64, c_void_p, c_float,
+                                              c_void_p, c_int64, c_int64, c_void_p, c_int64,
+                                              c_void_p]),
+    "mvsd_row_logprobs_split": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int64,
+                                        c_void_p, c_int64, c_int64, c_int64, c_int, c_void_p,
+                                        c_int64, c_void_p]),
     "mvsd_logprobs_workspace_bytes": (c_int64, [c_int64, c_int64, c_int64]),
     "mvsd_spec_logprobs_split": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int64,
                                          c_void_p, c_void_p, c_int64, c_void_p, c_void_p,

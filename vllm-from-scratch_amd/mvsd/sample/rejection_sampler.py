@@ -180,15 +180,15 @@ class RejectionSampler:
 
     def _bonus_rows_race_only(self, sm: SamplingMetadata, logits: torch.Tensor) -> bool:
         """True when the caller's sampler is mvsd.sample.Sampler itself and, for this batch,
-        it would only take each bonus row's argmax or exponential race: no logprobs, no
-        penalty or active min_tokens, no min_p, top-k or top-p; and the recovered-token seam
-        is the module's own."""
+        it would only take each bonus row's argmax or exponential race under its top-k / top-p:
+        no penalty or active min_tokens, no min_p, and no logprobs but raw ones; and the
+        recovered-token seam is the module's own."""
         from .sampler import Sampler as DeviceSampler
 
-        return (type(self.sampler) is DeviceSampler and sm.max_num_logprobs is None
-                and sm.no_penalties and not _has_active_min_tokens(sm)
-                and sm.min_p is None and sm.top_k is None and sm.top_p is None
+        return (type(self.sampler) is DeviceSampler and not self.is_processed_logprobs_mode
+                and sm.no_penalties and not _has_active_min_tokens(sm) and sm.min_p is None
                 and sample_recovered_tokens is _SAMPLE_RECOVERED_TOKENS
+                and (sm.all_greedy or sm.temperature is not None)
                 and logits.dtype in (torch.float32, torch.bfloat16, torch.float16)
                 and logits.stride(1) == 1)
 
@@ -200,10 +200,11 @@ class RejectionSampler:
         The randomness is drawn exactly as the reference draws it, in its order: the bonus
         rows' Exp(1) noise (Sampler.sample's random_sample, for every row unless the batch is
         all greedy), the uniforms (generate_uniform_probs), the recovered tokens' noise
-        (generate_exponential_noise).  Then one race launch reads the bonus rows in place
-        (greedy rows: their argmax) and the verify kernel reads the verify rows in place, so
-        neither the [B, V] gather of the bonus rows nor its fp32 upcast is written, and the
-        race runs between the noise writes and the verification."""
+        (generate_exponential_noise).  Then the top-k / top-p masks of the verify and bonus rows
+        are found in one call, one race launch reads the bonus rows in place (greedy rows:
+        their argmax) and the verify kernel reads the verify rows in place, so neither the
+        [B, V] gather of the bonus rows nor its fp32 upcast is written, and the race runs
+        between the noise writes and the verification."""
         from ..outputs import SamplerOutput
         from . import sampler as smp
 
@@ -221,16 +222,28 @@ class RejectionSampler:
         if not all_greedy and num_tokens > 0:
             exp_noise = generate_exponential_noise(B, V, metadata.num_draft_tokens,
                                                    sm.generators, device)
+        constrained = not all_greedy and (sm.top_k is not None or sm.top_p is not None)
+        masks = bonus_masks = None
+        if constrained:
+            masks = _step_masks(logits, metadata, sm, B, num_tokens)
+            bonus_masks = (smp.constraint_masks(logits, metadata.bonus_logits_indices, sm)
+                           if masks is None else masks[num_tokens:])
         bonus = smp.race_rows(logits, metadata.bonus_logits_indices, bonus_noise,
-                              None if all_greedy else sm.temperature)
-        output_token_ids = rejection_sample(
+                              None if all_greedy else sm.temperature, masks=bonus_masks)
+        output_token_ids = _rejection_sample(
             metadata.draft_token_ids, metadata.num_draft_tokens, metadata.max_spec_len,
             metadata.cu_num_draft_tokens, draft_probs, logits, bonus.view(B, 1), sm,
             synthetic_mode=self.synthetic_mode,
             synthetic_conditional_rates=self.synthetic_conditional_rates,
             uniform_probs=uniforms, exp_noise=exp_noise,
-            target_rows=metadata.target_logits_indices, apply_temperature=True)
-        return SamplerOutput(sampled_token_ids=output_token_ids, logprobs_tensors=None)
+            target_rows=metadata.target_logits_indices, apply_temperature=True,
+            apply_top_k_top_p=constrained, row_masks=masks)
+        logprobs_tensors = None
+        if sm.max_num_logprobs is not None:
+            logprobs_tensors = self._get_logprobs_tensors(sm.max_num_logprobs, metadata, logits,
+                                                          None, None, output_token_ids)
+        return SamplerOutput(sampled_token_ids=output_token_ids,
+                             logprobs_tensors=logprobs_tensors)
 
     def _get_logprobs_tensors(self, max_num_logprobs: int, metadata: "SpecDecodeMetadata",
                               logits: torch.Tensor, target_logits: torch.Tensor | None,
@@ -549,6 +562,22 @@ def rejection_sample(
         row of a random request, the kernel's row maximum M, sum S of exp((x - M) / T) and the
         fp32 p[d] its acceptance test compared.
     """
+    return _rejection_sample(
+        draft_token_ids, num_draft_tokens, max_spec_len, cu_num_draft_tokens, draft_probs,
+        target_logits, bonus_token_ids, sampling_metadata, synthetic_mode,
+        synthetic_conditional_rates, uniform_probs=uniform_probs, exp_noise=exp_noise,
+        target_rows=target_rows, apply_temperature=apply_temperature,
+        apply_top_k_top_p=apply_top_k_top_p, debug_row_stats=debug_row_stats)
+
+
+def _rejection_sample(draft_token_ids, num_draft_tokens, max_spec_len, cu_num_draft_tokens,
+                      draft_probs, target_logits, bonus_token_ids, sampling_metadata,
+                      synthetic_mode=False, synthetic_conditional_rates=None, *,
+                      uniform_probs=None, exp_noise=None, target_rows=None,
+                      apply_temperature=False, apply_top_k_top_p=False, debug_row_stats=None,
+                      row_masks=None) -> torch.Tensor:
+    """rejection_sample; ``row_masks`` (None: find them) holds the verify rows' constraint masks
+    in its first P rows, which the call clears."""
     assert draft_token_ids.ndim == 1
     assert draft_probs is None or draft_probs.ndim == 2
     assert cu_num_draft_tokens.ndim == 1
@@ -683,12 +712,48 @@ def rejection_sample(
     )
     if top_k is None and top_p is None:
         nat.check(handle.mvsd_rejection_sample(args, stream), "mvsd_rejection_sample")
+    elif row_masks is not None:
+        nat.check(handle.mvsd_rejection_sample_masked(args, row_masks.data_ptr(), stream),
+                  "mvsd_rejection_sample_masked")
     else:
         scratch = _constraints_scratch(num_tokens, vocab_size, top_p, device)
         nat.check(handle.mvsd_rejection_sample_split(
             args, nat.ptr(scratch), 0 if scratch is None else scratch.numel(), stream),
             "mvsd_rejection_sample_split")
     return output_token_ids
+
+
+def _step_masks(logits: torch.Tensor, metadata: "SpecDecodeMetadata", sm: SamplingMetadata,
+                batch_size: int, num_tokens: int) -> torch.Tensor | None:
+    """The constraint masks [P + B, 4] of the verify rows and of the bonus rows from one
+    ``mvsd_step_masks`` call; None where its split path does not apply."""
+    device = logits.device
+    V = logits.shape[-1]
+    n = num_tokens + batch_size
+    scratch = _constraints_scratch(n, V, sm.top_p, device)
+    if scratch is None:
+        return None
+    temperature = _as(sm.temperature, torch.float32, device)
+    top_k = None if sm.top_k is None else _as(sm.top_k, torch.int64, device)
+    top_p = _as(sm.top_p, torch.float32, device)
+    cu = _as(metadata.cu_num_draft_tokens, torch.int32, device)
+    rows = _as(metadata.target_logits_indices, torch.int32, device)
+    bonus_rows = _as(metadata.bonus_logits_indices, torch.int32, device)
+    for values in (temperature, top_k, top_p, cu, bonus_rows):
+        assert values is None or values.shape == (batch_size,)
+    assert rows.shape == (num_tokens,)
+    masks = torch.empty((n, 4), dtype=torch.float32, device=device)
+    args = nat.RejectionArgs(
+        target_logits=logits.data_ptr(), target_dtype=nat.dtype_code(logits.dtype),
+        target_stride=logits.stride(0), target_rows=rows.data_ptr(),
+        target_num_rows=logits.shape[0], cu_num_draft_tokens=cu.data_ptr(),
+        temperature=temperature.data_ptr(), all_greedy=0, apply_temperature=1,
+        batch_size=batch_size, num_tokens=num_tokens, vocab_size=V, top_k=nat.ptr(top_k),
+        top_p=top_p.data_ptr())
+    nat.check(nat.lib().mvsd_step_masks(args, bonus_rows.data_ptr(), masks.data_ptr(),
+                                        scratch.data_ptr(), scratch.numel(),
+                                        nat.stream_of(device)), "mvsd_step_masks")
+    return masks
 
 
 def _constraints_scratch(num_rows: int, vocab_size: int, top_p, device) -> torch.Tensor | None:

@@ -12,15 +12,17 @@ The rejection sampler takes its bonus tokens from a sampler object (rejection_sa
     -> logprobs of the raw (before any processing) or processed rows on request
 
 Every row operation is a HIP kernel (``mvsd_apply_logits_processors``,
-``mvsd_apply_top_k_top_p``, ``mvsd_sampler_rows``, ``mvsd_sampler_race(_rows)``,
-``mvsd_spec_logprobs``).  The temperature divide is a tensor divide, as in the reference,
-except where nothing reads the divided rows (no min_p, top-k or top-p, and no processed_*
-logprobs mode): there one race launch divides each value as it reads it (the same IEEE fp32
-quotient) and gives the rows under SAMPLING_EPS their argmax, and the caller's logits are
-left undivided.  The race's token is the argmax of softmax(v) / E, evaluated as that of
-v log2(e) - log2(E) (the row's max and sum are common to its entries), so only near-ties
-within a few fp32 ulps of the keys' magnitudes can differ from the reference's fp32
-arithmetic.  The exponential noise is drawn by
+``mvsd_apply_top_k_top_p(_split)``, ``mvsd_sampling_masks_split``, ``mvsd_sampler_rows``,
+``mvsd_sampler_race(_rows_masked)``, ``mvsd_row_logprobs_split``).  Where nothing needs written
+rows (no penalty, min_tokens or min_p, raw logprobs; ``_reads_rows_in_place``), the rows are read
+as they arrive, in their own dtype: top-k / top-p become row masks, one race launch divides each
+value by the temperature as it reads it (the same IEEE fp32 quotient), applies the masks and gives
+the rows under SAMPLING_EPS their argmax, and the logprobs read the raw rows.  Otherwise the
+temperature divide is a tensor divide and the constraints mask the fp32 rows in place, as in the
+reference (so too for a caller's own contiguous fp32 rows with top-k or top-p).  The race's token
+is the argmax of softmax(v) / E, evaluated as that of v log2(e) - log2(E) (the row's max and sum
+are common to its entries), so only near-ties within a few fp32 ulps of the keys' magnitudes can
+differ from the reference's fp32 arithmetic.  The exponential noise is drawn by
 ``generate_sampler_noise`` in the reference's order (the whole block from the global RNG when
 some row has no generator, then each seeded row from its generator), so a given RNG state
 gives the same noise; the function is a seam that tests may replace.
@@ -36,7 +38,7 @@ from ..outputs import LogprobsTensors, SamplerOutput
 from .metadata import SAMPLING_EPS, SamplingMetadata
 from .ops.topk_topp_sampler import apply_top_k_top_p
 
-_ARGMAX, _MIN_P, _LOG_SOFTMAX = 0, 1, 3
+_MIN_P, _LOG_SOFTMAX = 1, 3
 _PROCESSED_MODES = ("processed_logits", "processed_logprobs")
 
 
@@ -88,11 +90,13 @@ def random_sample(probs_logits: torch.Tensor, generators: dict[int, torch.Genera
 
 def race_rows(logits: torch.Tensor, row_index: torch.Tensor | None,
               noise: torch.Tensor | None, temperature: torch.Tensor | None,
-              greedy_eps: float = SAMPLING_EPS) -> torch.Tensor:
+              greedy_eps: float = SAMPLING_EPS,
+              masks: torch.Tensor | None = None) -> torch.Tensor:
     """Sampled ids (int32 [n]) of the rows ``logits[row_index]`` (fp32, bf16 or fp16, read in
     place) in one ``mvsd_sampler_race_rows`` call: rows whose temperature is below
     ``greedy_eps`` take the argmax of the raw row (greedy_sample), the others the exponential
-    race of softmax(row / T) with ``noise`` [n, V]; without noise every row is greedy."""
+    race of softmax(row / T) with ``noise`` [n, V], over the entries that ``masks`` [n, 4] (as
+    ``sampling_masks`` writes them; None: all) keeps; without noise every row is greedy."""
     nat.require_device_tensor(logits, "logits")
     assert logits.ndim == 2 and logits.stride(1) == 1
     device = logits.device
@@ -111,12 +115,70 @@ def race_rows(logits: torch.Tensor, row_index: torch.Tensor | None,
     lib = nat.lib()
     ws = torch.empty(max(1, lib.mvsd_sampler_race_workspace_bytes(n, V)), dtype=torch.uint8,
                      device=device)
-    nat.check(lib.mvsd_sampler_race_rows(
+    nat.check(lib.mvsd_sampler_race_rows_masked(
         ids.data_ptr(), logits.data_ptr(), nat.dtype_code(logits.dtype), logits.stride(0),
         nat.ptr(rows), logits.shape[0], nat.ptr(noise), 0 if noise is None else noise.stride(0),
-        nat.ptr(temperature), float(greedy_eps), n, V, ws.data_ptr(), ws.numel(),
-        nat.stream_of(device)), "mvsd_sampler_race_rows")
+        nat.ptr(temperature), float(greedy_eps), nat.ptr(masks), n, V, ws.data_ptr(),
+        ws.numel(), nat.stream_of(device)), "mvsd_sampler_race_rows_masked")
     return ids
+
+
+def constraint_masks(logits: torch.Tensor, row_index: torch.Tensor | None,
+                     sm: SamplingMetadata) -> torch.Tensor | None:
+    """The top-k / top-p masks [n, 4] of the rows ``logits[row_index]`` (every row when None),
+    one request each, for ``race_rows``; None when no request has either."""
+    if sm.all_greedy or (sm.top_k is None and sm.top_p is None):
+        return None
+    device = logits.device
+
+    def on_device(values, dtype):
+        return None if values is None else values.to(device=device, dtype=dtype).contiguous()
+
+    rows = on_device(row_index, torch.int32)
+    temperature = on_device(sm.temperature, torch.float32)
+    top_k, top_p = on_device(sm.top_k, torch.int64), on_device(sm.top_p, torch.float32)
+    n, V = logits.shape[0] if rows is None else rows.shape[0], logits.shape[1]
+    for values in (temperature, top_k, top_p):
+        assert values is None or values.numel() == n
+    masks = torch.empty((n, 4), dtype=torch.float32, device=device)
+    handle = nat.lib()
+    size = 0 if top_p is None else handle.mvsd_constraints_scratch_bytes(n, V)
+    scratch = torch.empty(size, dtype=torch.uint8, device=device) if size > 0 else None
+    args = nat.RejectionArgs(
+        target_logits=logits.data_ptr(), target_dtype=nat.dtype_code(logits.dtype),
+        target_stride=logits.stride(0), target_rows=nat.ptr(rows),
+        target_num_rows=logits.shape[0], temperature=temperature.data_ptr(), all_greedy=0,
+        apply_temperature=1, batch_size=n, num_tokens=n, vocab_size=V, top_k=nat.ptr(top_k),
+        top_p=nat.ptr(top_p))
+    nat.check(handle.mvsd_sampling_masks_split(args, masks.data_ptr(), nat.ptr(scratch), size,
+                                               nat.stream_of(device)),
+              "mvsd_sampling_masks_split")
+    return masks
+
+
+def row_logprobs(rows: torch.Tensor, num_logprobs: int, token_ids: torch.Tensor,
+                 logits_mode: bool) -> LogprobsTensors | None:
+    """Each row's token first, then its top ``num_logprobs`` (value, then index), as the row's
+    log-softmax or (``logits_mode``) its values, and the token's rank: one
+    ``mvsd_row_logprobs_split`` call on rows of any float dtype.  None where that path does not
+    apply (above 128 logprobs)."""
+    n, V = rows.shape
+    device = rows.device
+    handle = nat.lib()
+    size = handle.mvsd_logprobs_workspace_bytes(n, V, num_logprobs)
+    if size <= 0:
+        return None
+    ids = torch.empty((n, num_logprobs + 1), dtype=torch.int32, device=device)
+    lps = torch.empty((n, num_logprobs + 1), dtype=torch.float32, device=device)
+    ranks = torch.empty((n,), dtype=torch.int32, device=device)
+    workspace = torch.empty(size, dtype=torch.uint8, device=device)
+    tokens = token_ids.to(device=device, dtype=torch.int32).contiguous()
+    nat.check(handle.mvsd_row_logprobs_split(
+        ids.data_ptr(), lps.data_ptr(), ranks.data_ptr(), rows.data_ptr(),
+        nat.dtype_code(rows.dtype), rows.stride(0), tokens.data_ptr(), n, V, num_logprobs,
+        int(logits_mode), workspace.data_ptr(), size, nat.stream_of(device)),
+        "mvsd_row_logprobs_split")
+    return LogprobsTensors(ids, lps, ranks)
 
 
 class TopKTopPSampler:
@@ -147,6 +209,8 @@ class Sampler:
         logprobs_mode = logprobs_mode_override or self.logprobs_mode
         assert not (sampling_metadata.all_greedy and sampling_metadata.all_random)
         num_logprobs = sampling_metadata.max_num_logprobs
+        if self._reads_rows_in_place(logits, sampling_metadata, logprobs_mode):
+            return self._forward_in_place(logits, sampling_metadata, logprobs_mode)
         raw_logprobs = None
         if num_logprobs is not None:
             if logprobs_mode == "raw_logprobs":
@@ -168,6 +232,46 @@ class Sampler:
             tensors = self.gather_logprobs(raw_logprobs, num_logprobs, sampled)
         return SamplerOutput(sampled_token_ids=sampled.to(torch.int32).unsqueeze(dim=1),
                              logprobs_tensors=tensors)
+
+    def _reads_rows_in_place(self, logits: torch.Tensor, sm: SamplingMetadata,
+                             logprobs_mode: str) -> bool:
+        """True when this batch needs no row written: no penalty or active min_tokens, no min_p,
+        and only raw logprobs, up to the 128 of the split path.  (With top-k or top-p, the
+        caller's own contiguous fp32 rows are to be divided and masked in place; other rows are
+        copied before that, so there it does not show.)"""
+        from .rejection_sampler import _has_active_min_tokens
+
+        return (type(self) is Sampler and type(self.topk_topp_sampler) is TopKTopPSampler
+                and self.topk_topp_sampler.logprobs_mode not in _PROCESSED_MODES
+                and logprobs_mode in ("raw_logprobs", "raw_logits")
+                and sm.no_penalties and not _has_active_min_tokens(sm) and sm.min_p is None
+                and (sm.max_num_logprobs is None or sm.max_num_logprobs >= 0)
+                and (sm.all_greedy or sm.temperature is not None)
+                and logits.is_cuda and logits.ndim == 2 and logits.shape[0] > 0
+                and logits.dtype in (torch.float32, torch.bfloat16, torch.float16)
+                and logits.stride(1) == 1
+                and (sm.all_greedy or (sm.top_k is None and sm.top_p is None)
+                     or logits.dtype != torch.float32 or not logits.is_contiguous())
+                and (sm.max_num_logprobs is None
+                     or nat.lib().mvsd_logprobs_workspace_bytes(
+                         logits.shape[0], logits.shape[1], sm.max_num_logprobs) > 0))
+
+    def _forward_in_place(self, logits: torch.Tensor, sm: SamplingMetadata,
+                          logprobs_mode: str) -> SamplerOutput:
+        """forward on rows read in place in their own dtype: the constraints as row masks, one
+        race that applies them (rows under SAMPLING_EPS take their argmax), the logprobs of the
+        raw rows.  The same tokens as the general path, which writes the rows' fp32 copy, its
+        quotient by the temperature and its masked entries."""
+        noise = None
+        if not sm.all_greedy:
+            noise = generate_sampler_noise(tuple(logits.shape), sm.generators, logits.device)
+        ids = race_rows(logits, None, noise, None if sm.all_greedy else sm.temperature,
+                        masks=constraint_masks(logits, None, sm))
+        tensors = None
+        if sm.max_num_logprobs is not None:
+            tensors = row_logprobs(logits, sm.max_num_logprobs, ids,
+                                   logprobs_mode == "raw_logits")
+        return SamplerOutput(sampled_token_ids=ids.unsqueeze(dim=1), logprobs_tensors=tensors)
 
     # -------- logits processors --------
 
@@ -293,10 +397,7 @@ class Sampler:
 
     @staticmethod
     def greedy_sample(logits: torch.Tensor) -> torch.Tensor:
-        x = logits.contiguous()
-        ids = torch.empty(x.shape[0], dtype=torch.int32, device=x.device)
-        _rows(_ARGMAX, x, ids=ids)
-        return ids.to(torch.int64)
+        return race_rows(logits.contiguous(), None, None, None).to(torch.int64)
 
     # -------- logprobs --------
 
@@ -316,10 +417,13 @@ class Sampler:
     def gather_logprobs(logprobs: torch.Tensor, num_logprobs: int,
                         token_ids: torch.Tensor) -> LogprobsTensors:
         """Sampled token first, then the top ``num_logprobs`` (value, then index), and the
-        sampled token's rank (sampler.py:330-349); one ``mvsd_spec_logprobs`` launch with each
-        row its own position."""
+        sampled token's rank (sampler.py:330-349); ``row_logprobs``, or one
+        ``mvsd_spec_logprobs`` launch with each row its own position."""
         assert token_ids.dtype == torch.int64
         x = logprobs.to(torch.float32).contiguous()
+        split = row_logprobs(x, num_logprobs, token_ids, True)
+        if split is not None:
+            return split
         n, V = x.shape
         device = x.device
         ids = torch.empty((n, num_logprobs + 1), dtype=torch.int32, device=device)
