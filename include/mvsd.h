@@ -323,6 +323,20 @@ int mvsd_ngram_propose(int32_t* drafts, int32_t* num_valid, int32_t* token_ids,
                        int32_t min_n, int32_t max_n, int32_t k, int cap_by_model_len,
                        int64_t max_model_len, mvsd_stream_t stream);
 
+/* mvsd_ngram_propose with long histories split over workgroups.  workspace:                */
+/* mvsd_ngram_workspace_bytes() bytes, 256-byte aligned, caller-owned, cleared once with     */
+/* mvsd_ngram_workspace_init and left cleared by every call (calls that may overlap need      */
+/* workspaces of their own); NULL: one workgroup per history.                                */
+int64_t mvsd_ngram_workspace_bytes(void);
+int mvsd_ngram_workspace_init(void* workspace, int64_t workspace_bytes, mvsd_stream_t stream);
+int mvsd_ngram_propose_split(int32_t* drafts, int32_t* num_valid, int32_t* token_ids,
+                       int64_t row_stride, int64_t max_seq_len, const int32_t* num_tokens,
+                       const int32_t* new_tokens, int64_t new_tokens_stride,
+                       int64_t max_new_tokens, const int32_t* new_counts,
+                       const uint8_t* active, int gate_on_new_counts, int64_t num_reqs,
+                       int32_t min_n, int32_t max_n, int32_t k, int cap_by_model_len,
+                       int64_t max_model_len, void* workspace, int64_t workspace_bytes, mvsd_stream_t stream);
+
 /* ------------------------------------------------------------------------------------ */
 /* apply_logits_processors — penalties and min_tokens of the verify rows, in place.        */
 /* Replaces: RejectionSampler.apply_logits_processors / apply_penalties /                  */

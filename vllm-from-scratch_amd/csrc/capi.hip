@@ -879,6 +879,29 @@ int mvsd_ngram_propose(int32_t* drafts, int32_t* num_valid, int32_t* token_ids,
                        const uint8_t* active, int gate_on_new_counts, int64_t num_reqs,
                        int32_t min_n, int32_t max_n, int32_t k, int cap_by_model_len,
                        int64_t max_model_len, mvsd_stream_t stream) {
+  return mvsd_ngram_propose_split(drafts, num_valid, token_ids, row_stride, max_seq_len, num_tokens,
+                                  new_tokens, new_tokens_stride, max_new_tokens, new_counts, active,
+                                  gate_on_new_counts, num_reqs, min_n, max_n, k, cap_by_model_len,
+                                  max_model_len, nullptr, 0, stream);
+}
+
+int64_t mvsd_ngram_workspace_bytes(void) { return mvsd::ngram_workspace_bytes(); }
+
+int mvsd_ngram_workspace_init(void* workspace, int64_t workspace_bytes, mvsd_stream_t stream) {
+  if (!workspace || workspace_bytes < mvsd::ngram_workspace_bytes()) return MVSD_E_WORKSPACE;
+  if ((uintptr_t)workspace % 256 != 0) return MVSD_E_ALIGN;
+  return hip_status(mvsd::launch_zero_fill(workspace, mvsd::ngram_workspace_bytes(),
+                                           (hipStream_t)stream));
+}
+
+int mvsd_ngram_propose_split(int32_t* drafts, int32_t* num_valid, int32_t* token_ids,
+                             int64_t row_stride, int64_t max_seq_len, const int32_t* num_tokens,
+                             const int32_t* new_tokens, int64_t new_tokens_stride,
+                             int64_t max_new_tokens, const int32_t* new_counts,
+                             const uint8_t* active, int gate_on_new_counts, int64_t num_reqs,
+                             int32_t min_n, int32_t max_n, int32_t k, int cap_by_model_len,
+                             int64_t max_model_len, void* workspace, int64_t workspace_bytes,
+                             mvsd_stream_t stream) {
   if (num_reqs < 0) return MVSD_E_INVALID;
   if (min_n < 1 || max_n < min_n || k < 1) return MVSD_E_INVALID;
   if (max_n > mvsd::kNgramMaxN || k > 256) return MVSD_E_RANGE;
@@ -889,7 +912,10 @@ int mvsd_ngram_propose(int32_t* drafts, int32_t* num_valid, int32_t* token_ids,
   if (new_tokens && (max_new_tokens < 0 || new_tokens_stride < max_new_tokens))
     return MVSD_E_INVALID;
   if (gate_on_new_counts && !new_counts) return MVSD_E_INVALID;
-  mvsd::NgramParams p;
+  if (workspace && (workspace_bytes < mvsd::ngram_workspace_bytes() ||
+                    ((uintptr_t)workspace & 255) != 0))
+    return MVSD_E_WORKSPACE;
+  mvsd::NgramParams p{};
   p.drafts = drafts;
   p.num_valid = num_valid;
   p.tokens = token_ids;
@@ -907,7 +933,7 @@ int mvsd_ngram_propose(int32_t* drafts, int32_t* num_valid, int32_t* token_ids,
   p.k = k;
   p.cap_by_model_len = cap_by_model_len ? 1 : 0;
   p.max_model_len = max_model_len;
-  return hip_status(mvsd::launch_ngram(p, num_reqs, (hipStream_t)stream));
+  return hip_status(mvsd::launch_ngram(p, num_reqs, workspace, (hipStream_t)stream));
 }
 
 }  // extern "C"

@@ -39,9 +39,15 @@ struct NgramParams {
   int k;
   int cap_by_model_len;
   int64_t max_model_len;
+  int parts;          // workgroups per request (set by the launch)
+  int* shared_first;  // [requests, kNgramMaxN + 1], zero between calls (set by the launch)
 };
 
-hipError_t launch_ngram(const NgramParams& p, int64_t num_reqs, hipStream_t stream);
+// With a workspace (ngram_workspace_bytes, zero between calls), long histories are split over
+// workgroups.
+int64_t ngram_workspace_bytes();
+hipError_t launch_ngram(const NgramParams& p, int64_t num_reqs, void* workspace,
+                        hipStream_t stream);
 
 hipError_t launch_ngram_valid_sampled(int32_t* next_token_ids, int32_t* counts,
                                       int32_t* valid_ids, int64_t valid_stride,

@@ -116,6 +116,12 @@ SIGNATURES = {
                                    c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int,
                                    c_int64, c_int32, c_int32, c_int32, c_int, c_int64,
                                    c_void_p]),
+    "mvsd_ngram_propose_split": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_void_p,
+                                   c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int,
+                                   c_int64, c_int32, c_int32, c_int32, c_int, c_int64,
+                                   c_void_p, c_int64, c_void_p]),
+    "mvsd_ngram_workspace_bytes": (c_int64, []),
+    "mvsd_ngram_workspace_init": (c_int, [c_void_p, c_int64, c_void_p]),
     "mvsd_v2_workspace_bytes": (c_int64, [c_int64, c_int64, c_int64]),
     "mvsd_v2_rejection_sample": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int, c_int64,
                                          c_int64, c_void_p, c_int, c_int64, c_int64, c_void_p,
