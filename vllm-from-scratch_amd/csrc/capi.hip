@@ -27,10 +27,6 @@ int hip_status(hipError_t err) {
   return MVSD_E_HIP;
 }
 
-bool aligned16(const void* ptr, int64_t stride_bytes) {
-  return ((uintptr_t)ptr % 16 == 0) && (stride_bytes % 16 == 0);
-}
-
 int elem_size(int dtype) {
   switch (dtype) {
     case MVSD_F32: return 4;
@@ -55,12 +51,12 @@ std::atomic<int> g_wait_limit{mvsd::kSpinLimitDefault};
 // Resident-workgroup capacity of the verify kernel variant per device (CUs x occupancy).
 int verify_capacity(int device, int dtype, int draft_dtype, bool masked) {
   static std::mutex mu;
-  static int cache[kMaxDevices][3][4][2];
-  if (device < 0 || device >= kMaxDevices || dtype < 0 || dtype > 2 || draft_dtype < -1 ||
-      draft_dtype > 2)
+  static int cache[kMaxDevices][3][5][2];
+  if (device < 0 || device >= kMaxDevices || dtype < 0 || dtype > 2 ||
+      draft_dtype < mvsd::kGreedyOnly || draft_dtype > 2)
     return 0;
   std::lock_guard<std::mutex> lock(mu);
-  int& slot = cache[device][dtype][draft_dtype + 1][masked ? 1 : 0];
+  int& slot = cache[device][dtype][draft_dtype - mvsd::kGreedyOnly][masked ? 1 : 0];
   if (slot > 0) return slot;
   int cus = 0;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
@@ -234,7 +230,8 @@ int rejection_sample_impl(const mvsd_rejection_args* a, void* ws_ptr, int64_t ws
   int device = 0;
   hipError_t err = hipGetDevice(&device);
   if (err != hipSuccess) return hip_status(err);
-  const int draft_dtype = a->draft_probs ? a->draft_dtype : -1;
+  const int draft_dtype = a->all_greedy ? mvsd::kGreedyOnly
+                          : a->draft_probs ? a->draft_dtype : -1;
   const int cap = verify_capacity(device, a->target_dtype, draft_dtype, masked);
   if (cap <= 0) return hip_status(hipErrorInvalidDevice);
 
@@ -268,11 +265,6 @@ int rejection_sample_impl(const mvsd_rejection_args* a, void* ws_ptr, int64_t ws
   p.max_spec_len = (int)a->max_spec_len;
   p.G = size_plan.g;
   p.spin_limit = g_wait_limit.load();
-  const int esz = elem_size(a->target_dtype);
-  p.target_aligned = aligned16(a->target_logits, a->target_stride * esz);
-  p.draft_aligned =
-      a->draft_probs ? aligned16(a->draft_probs, a->draft_stride * elem_size(draft_dtype)) : false;
-  p.noise_aligned = a->exp_noise ? aligned16(a->exp_noise, a->noise_stride * 4) : false;
   p.ctrl = reinterpret_cast<int*>(ws + lay.ctrl);
   p.req_cnt = reinterpret_cast<int*>(ws + lay.req_cnt);
   p.score_cnt = reinterpret_cast<int*>(ws + lay.score_cnt);

@@ -107,10 +107,6 @@ __device__ inline void for_each_vector(const P* xv, int nvec, G&& g) {
   for (int v = nfull * step + tid; v < nvec; v += kCT) g(v, xv[v]);
 }
 
-// The row's vectors at its element alignment.
-template <int DT>
-using RowVec = std::conditional_t<sizeof(typename Elem<DT>::storage) == 4, u32x4_align4, u32x4_align2>;
-
 // Calls f(i0, v, n) for every group of consecutive entries: v[0, n) are entries i0, i0 + 1,
 // ...; a group is one 16-byte vector (n = VEC), or one of the row's last entries that fill none
 // (n = 1).  Per-group work lets a pass test a whole vector with one branch.  Rows of any alignment
@@ -121,7 +117,7 @@ __device__ inline void for_each_group(const typename Elem<DT>::storage* __restri
                                       F&& f) {
   constexpr int VEC = Elem<DT>::kVec;
   const int nvec = V / VEC;
-  for_each_vector(reinterpret_cast<const RowVec<DT>*>(x), nvec, [&](int vi, const u32x4& r) {
+  for_each_vector(reinterpret_cast<const Vec16<DT>*>(x), nvec, [&](int vi, const u32x4& r) {
     float v[VEC];
 #pragma unroll
     for (int j = 0; j < VEC; ++j) v[j] = vec_elem<DT>(r, j);

@@ -12,6 +12,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "../../include/mvsd.h"
 
 namespace mvsd {
@@ -49,19 +51,36 @@ struct Elem<MVSD_F16> {
   __device__ static inline _Float16 ninf() { return static_cast<_Float16>(-INFINITY); }
 };
 
-// Load kVec consecutive elements starting at p[idx] and convert them to fp32.  Elements at
-// or beyond `limit` are replaced by `fill`.  `aligned` (wave-uniform) says p + idx is 16-byte
-// aligned whenever idx is a multiple of kVec; otherwise scalar loads are used.
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
+// Rows start at any element (an odd vocabulary, a view), so vector loads promise the compiler
+// element alignment only.  gfx950's global loads take any alignment: it emits the same
+// global_load_dwordx4 / dwordx2 as for aligned rows.
+typedef u32x4 u32x4_align4 __attribute__((aligned(4)));
+typedef u32x4 u32x4_align2 __attribute__((aligned(2)));
+typedef u32x2 u32x2_align4 __attribute__((aligned(4)));
+typedef u32x2 u32x2_align2 __attribute__((aligned(2)));
+template <int DT>
+using Vec16 = std::conditional_t<sizeof(typename Elem<DT>::storage) == 4, u32x4_align4, u32x4_align2>;
+template <int DT>
+using Vec8 = std::conditional_t<sizeof(typename Elem<DT>::storage) == 4, u32x2_align4, u32x2_align2>;
+
+// The 16-byte vector holding elements p[0 .. kVec), which must be in bounds.
+template <int DT>
+__device__ inline u32x4 load_vec_any(const typename Elem<DT>::storage* p) {
+  return *reinterpret_cast<const Vec16<DT>*>(p);
+}
+
+// Load kVec consecutive elements starting at p[idx] and convert them to fp32.  Elements at
+// or beyond `limit` are replaced by `fill`.
 template <int DT>
 __device__ inline void load_vec(const typename Elem<DT>::storage* __restrict__ p, int64_t idx,
-                                int64_t limit, bool aligned, float fill,
-                                float (&out)[Elem<DT>::kVec]) {
+                                int64_t limit, float fill, float (&out)[Elem<DT>::kVec]) {
   constexpr int V = Elem<DT>::kVec;
   using S = typename Elem<DT>::storage;
-  if (aligned && idx + V <= limit) {
-    const u32x4 raw = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p + idx));
+  if (idx + V <= limit) {
+    const u32x4 raw = __builtin_nontemporal_load(reinterpret_cast<const Vec16<DT>*>(p + idx));
     const S* s = reinterpret_cast<const S*>(&raw);
 #pragma unroll
     for (int j = 0; j < V; ++j) out[j] = Elem<DT>::cvt(s[j]);
@@ -69,20 +88,6 @@ __device__ inline void load_vec(const typename Elem<DT>::storage* __restrict__ p
 #pragma unroll
     for (int j = 0; j < V; ++j) out[j] = (idx + j < limit) ? Elem<DT>::cvt(p[idx + j]) : fill;
   }
-}
-
-// The 16-byte vector holding elements p[0 .. kVec) at any element alignment.  The type tells
-// the compiler that only element alignment holds; gfx950's global loads take any alignment, so
-// it emits one global_load_dwordx4 for rows of odd length too.  p[0 .. kVec) must be in bounds.
-typedef u32x4 u32x4_align4 __attribute__((aligned(4)));
-typedef u32x4 u32x4_align2 __attribute__((aligned(2)));
-
-template <int DT>
-__device__ inline u32x4 load_vec_any(const typename Elem<DT>::storage* p) {
-  if constexpr (sizeof(typename Elem<DT>::storage) == 4)
-    return *reinterpret_cast<const u32x4_align4*>(p);
-  else
-    return *reinterpret_cast<const u32x4_align2*>(p);
 }
 
 // Element j of a 16-byte vector, as fp32.

@@ -102,14 +102,10 @@ constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kRaceMode = 0, kRaceDivide = 1, kRaceGreedy = 2;
 constexpr uint64_t kRaceNaNRow = ~0ull;  // chunk key of a row whose probabilities are NaN: index 0
 
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-
 __device__ inline float4 f32x4_of(u32x4 q) {
   return make_float4(__uint_as_float(q[0]), __uint_as_float(q[1]), __uint_as_float(q[2]),
                      __uint_as_float(q[3]));
 }
-
-typedef u32x2 u32x2_align2 __attribute__((aligned(2)));
 
 template <int DT>
 using RaceQuad = std::conditional_t<Elem<DT>::kVec == 4, u32x4_align4, u32x2_align2>;

@@ -192,7 +192,6 @@ struct V2Params {
   int32_t num_reqs, num_states, vocab, K, nchunks;
   int use_fp64;
   int use_block;  // block verification (Sun et al. 2024) instead of the per-token test
-  bool target_aligned, draft_aligned;
   // workspace
   float *tmax, *tsum, *dmax, *dsum;  // [num_logits, nchunks] chunk partials
   int32_t* targ;
@@ -212,7 +211,7 @@ __device__ inline int clamp_state(int s, int n) { return s < 0 ? 0 : (s >= n ? n
 // columns at or past `limit` read -inf.
 template <int DT, int NT = kThreads>
 __device__ inline void load_chunk(const void* base, int64_t row_off, int c0, int limit,
-                                  bool aligned, float (&x)[kV2Chunk / NT]) {
+                                  float (&x)[kV2Chunk / NT]) {
   using S = typename Elem<DT>::storage;
   constexpr int VEC = Elem<DT>::kVec;
   const S* p = reinterpret_cast<const S*>(base) + row_off;
@@ -220,7 +219,7 @@ __device__ inline void load_chunk(const void* base, int64_t row_off, int c0, int
   for (int j = 0; j < kV2Chunk / NT / VEC; ++j) {
     const int col = c0 + (j * NT + (int)threadIdx.x) * VEC;
     float v[VEC];
-    load_vec<DT>(p, col, limit, aligned, -INFINITY, v);
+    load_vec<DT>(p, col, limit, -INFINITY, v);
 #pragma unroll
     for (int e = 0; e < VEC; ++e) x[j * VEC + e] = v[e];
   }
@@ -302,13 +301,13 @@ __global__ __launch_bounds__(kThreads) void v2_stats_kernel(V2Params p) {
   float x[G][kV2PerThread];
   // the target loads go out before the temperature is known; the draft loads (random rows
   // only) right after, so both rows are in flight together
-  load_chunk<TDT>(p.target, row * p.target_stride, c0, p.vocab, p.target_aligned, x[0]);
+  load_chunk<TDT>(p.target, row * p.target_stride, c0, p.vocab, x[0]);
   const int st = clamp_state(st_raw, p.num_states);
   const float temp = p.temperature[st];
   if constexpr (HAS_DRAFT) {
     if (temp != 0.f)
       load_chunk<DDT>(p.draft, (int64_t)st * p.draft_stride0 + (int64_t)step * p.draft_stride1,
-                      c0, p.vocab, p.draft_aligned, x[1]);
+                      c0, p.vocab, x[1]);
   }
   if (temp == 0.f) {
     double bv = -INFINITY;
@@ -448,9 +447,9 @@ __global__ __launch_bounds__(kThreads) void v2_residual_kernel(V2Params p) {
   const float t_lse = p.rtl[row], d_lse = p.rdl[row];
   const int c0 = c * kV2Chunk;
   float x[kV2PerThread], q[kV2PerThread];
-  load_chunk<TDT>(p.target, row * p.target_stride, c0, p.vocab, p.target_aligned, x);
+  load_chunk<TDT>(p.target, row * p.target_stride, c0, p.vocab, x);
   load_chunk<DDT>(p.draft, (int64_t)st * p.draft_stride0 + (int64_t)step * p.draft_stride1, c0,
-                  p.vocab, p.draft_aligned, q);
+                  p.vocab, q);
   float part[1] = {0.f};
   const Divider dv = make_divider(temp);
 #pragma unroll
@@ -634,12 +633,12 @@ __global__ __launch_bounds__(kResThreads) void v2_resample_kernel(V2Params p) {
   if (d.mode == kResampleNone) return;
   const int c0 = c * kV2Chunk;
   float x[kResPer];
-  load_chunk<TDT, kResThreads>(p.target, d.row * p.target_stride, c0, p.vocab, p.target_aligned, x);
+  load_chunk<TDT, kResThreads>(p.target, d.row * p.target_stride, c0, p.vocab, x);
   constexpr int TV = Elem<TDT>::kVec;
   if constexpr (HAS_DRAFT) {
     if (d.mode == kResampleResidual) {
       float q[kResPer];
-      load_chunk<DDT, kResThreads>(p.draft, d.draft, c0, p.vocab, p.draft_aligned, q);
+      load_chunk<DDT, kResThreads>(p.draft, d.draft, c0, p.vocab, q);
       const Divider dv = make_divider(d.temp);
 #pragma unroll
       for (int k = 0; k < kResPer; ++k) {
@@ -922,11 +921,6 @@ int mvsd_v2_rejection_sample(
   p.nchunks = nch;
   p.use_fp64 = use_fp64 != 0;
   p.use_block = use_block_verification != 0;
-  const int tsz = target_dtype == MVSD_F32 ? 4 : 2;
-  const int dsz = draft_dtype == MVSD_F32 ? 4 : 2;
-  p.target_aligned = ((uintptr_t)target_logits % 16 == 0) && ((target_stride * tsz) % 16 == 0);
-  p.draft_aligned = draft_logits && ((uintptr_t)draft_logits % 16 == 0) &&
-                    ((draft_stride0 * dsz) % 16 == 0) && ((draft_stride1 * dsz) % 16 == 0);
   char* w = static_cast<char*>(workspace);
   const int64_t rows = num_logits * nch, reqs = num_reqs * (int64_t)nch;
   auto take = [&](int64_t bytes) {

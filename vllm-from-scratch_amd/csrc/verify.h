@@ -60,9 +60,6 @@ struct VerifyParams {
   int lag;         // stats units between a request's last stats unit and its score unit
   int tail_groups;  // stats groups at the end of the launch run in half-chunk tasks
   int spin_limit;  // polls before a wait gives up (0: every wait gives up at once)
-  bool target_aligned;
-  bool draft_aligned;
-  bool noise_aligned;
   // workspace (every array is zero between calls)
   int* ctrl;             // [kCtrlTicket] ticket, [kCtrlFlag] wait-failure flag, [kCtrlExit] exits
   int* req_cnt;          // [B] started stats tasks per request
@@ -126,8 +123,9 @@ struct VerifyPlan {
 VerifyPlan verify_plan(int target_dtype, int64_t vocab_size, int64_t units, int cap,
                        int64_t batch_rows, bool score_units);
 
-// The verify kernel variant for a target dtype, draft dtype (-1: point-mass drafts) and
-// sampling constraints.
+// The verify kernel variant for a target dtype, draft dtype (-1: point-mass drafts, kGreedyOnly:
+// all requests greedy) and sampling constraints.
+constexpr int kGreedyOnly = -2;
 const void* verify_kernel_ptr(int target_dtype, int draft_dtype, bool masked);
 hipError_t launch_zero_fill(void* p, int64_t bytes, hipStream_t stream);
 hipError_t launch_verify(const VerifyParams& params, int target_dtype, int grid,

@@ -129,9 +129,9 @@ __device__ inline int64_t vec_col(int64_t s0, int i) {
 // Target loads.  The stats tasks' loads are temporal, so that a row a score task reads again
 // shortly afterwards is still in the Infinity Cache; the score tasks' loads are the last use
 // and stream non-temporally.
-template <bool NT>
-__device__ inline u32x4 load16(const void* p) {
-  const u32x4* q = static_cast<const u32x4*>(p);
+template <int DT, bool NT>
+__device__ inline u32x4 load16(const typename Elem<DT>::storage* p) {
+  const Vec16<DT>* q = reinterpret_cast<const Vec16<DT>*>(p);
   if constexpr (NT) return __builtin_nontemporal_load(q);
   else return *q;
 }
@@ -160,39 +160,39 @@ __device__ inline u32x4 load_vec_checked(const typename Elem<DT>::storage* __res
   return v;
 }
 
-// DT row sub-chunk, full and aligned.
+// DT row sub-chunk, full.
 template <int DT, int EPT, bool NT>
 __device__ inline void load_raw(const typename Elem<DT>::storage* __restrict__ base, int64_t s0,
                                 u32x4 (&out)[EPT / Elem<DT>::kVec]) {
 #pragma unroll
-  for (int i = 0; i < EPT / Elem<DT>::kVec; ++i) out[i] = load16<NT>(base + vec_col<DT>(s0, i));
+  for (int i = 0; i < EPT / Elem<DT>::kVec; ++i) out[i] = load16<DT, NT>(base + vec_col<DT>(s0, i));
 }
 
 // DT row sub-chunk, bounds-checked: elements at or beyond vend read as `fill`.
 template <int DT, int EPT, bool NT>
 __device__ inline void load_raw_checked(const typename Elem<DT>::storage* __restrict__ base,
-                                        int64_t s0, int64_t vend, bool aligned,
+                                        int64_t s0, int64_t vend,
                                         typename Elem<DT>::storage fill,
                                         u32x4 (&out)[EPT / Elem<DT>::kVec]) {
   constexpr int VEC = Elem<DT>::kVec;
 #pragma unroll
   for (int i = 0; i < EPT / VEC; ++i) {
     const int64_t col = vec_col<DT>(s0, i);
-    if (aligned && col + VEC <= vend) out[i] = load16<NT>(base + col);
+    if (col + VEC <= vend) out[i] = load16<DT, NT>(base + col);
     else out[i] = load_vec_checked<DT>(base, col, vend, fill);
   }
 }
 
-// fp32 row sub-chunk in DT layout; FAST: full and aligned, else bounds-checked with `fill`.
+// fp32 row sub-chunk in DT layout; FAST: full, else bounds-checked with `fill`.
 template <int DT, int EPT, bool FAST>
 __device__ inline void load_raw_f32(const float* __restrict__ base, int64_t s0, int64_t vend,
-                                    bool aligned, float fill, u32x4 (&out)[EPT / 4]) {
+                                    float fill, u32x4 (&out)[EPT / 4]) {
   constexpr int VEC = Elem<DT>::kVec;
 #pragma unroll
   for (int m = 0; m < EPT / 4; ++m) {
     const int64_t col = vec_col<DT>(s0, m / (VEC / 4)) + (m % (VEC / 4)) * 4;
-    if (FAST || (aligned && col + 4 <= vend))
-      out[m] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(base + col));
+    if (FAST || col + 4 <= vend)
+      out[m] = __builtin_nontemporal_load(reinterpret_cast<const Vec16<MVSD_F32>*>(base + col));
     else
       out[m] = load_vec_checked<MVSD_F32>(base, col, vend, fill);
   }
@@ -200,8 +200,6 @@ __device__ inline void load_raw_f32(const float* __restrict__ base, int64_t s0, 
 
 // Draft probabilities of a thread's EPT elements in one sub-chunk, in the target's column
 // layout: fp32 (one word per element) or bf16 / fp16 (two per word), upcast when consumed.
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-
 template <int DD, int EPT>
 struct DraftBuf {
   static constexpr int kWords = DD == MVSD_F32 ? EPT : EPT / 2;
@@ -218,15 +216,15 @@ __device__ inline float draft_elem(const uint32_t* w, int k) {
   }
 }
 
-// Draft sub-chunk for the columns of the DT layout; FAST: full and aligned, else
+// Draft sub-chunk for the columns of the DT layout; FAST: full, else
 // bounds-checked (columns at or past vend read as 0).
 template <int DT, int DD, int EPT, bool FAST>
-__device__ inline void load_draft(const void* base_v, int64_t s0, int64_t vend, bool aligned,
+__device__ inline void load_draft(const void* base_v, int64_t s0, int64_t vend,
                                   DraftBuf<DD, EPT>& q) {
   constexpr int VEC = Elem<DT>::kVec;
   if constexpr (DD == MVSD_F32) {
     u32x4 raw[EPT / 4];
-    load_raw_f32<DT, EPT, FAST>(static_cast<const float*>(base_v), s0, vend, aligned, 0.f, raw);
+    load_raw_f32<DT, EPT, FAST>(static_cast<const float*>(base_v), s0, vend, 0.f, raw);
 #pragma unroll
     for (int m = 0; m < EPT / 4; ++m)
 #pragma unroll
@@ -237,13 +235,13 @@ __device__ inline void load_draft(const void* base_v, int64_t s0, int64_t vend, 
 #pragma unroll
     for (int i = 0; i < EPT / VEC; ++i) {
       const int64_t col = vec_col<DT>(s0, i);
-      if (FAST || (aligned && col + VEC <= vend)) {
+      if (FAST || col + VEC <= vend) {
         if constexpr (VEC == 4) {
-          const u32x2 v = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(base + col));
+          const u32x2 v = __builtin_nontemporal_load(reinterpret_cast<const Vec8<DD>*>(base + col));
           q.w[2 * i] = v[0];
           q.w[2 * i + 1] = v[1];
         } else {
-          const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(base + col));
+          const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const Vec16<DD>*>(base + col));
 #pragma unroll
           for (int j = 0; j < 4; ++j) q.w[4 * i + j] = v[j];
         }
@@ -261,15 +259,14 @@ __device__ inline void load_draft(const void* base_v, int64_t s0, int64_t vend, 
 
 // Walk [v0, vend) in SUB-column sub-chunks: load(buf, s0, Fast<bool>) issues a sub-chunk's
 // loads, body(buf, s0, Fast<bool>) consumes them.  hook() runs once, after the first loads
-// are issued.  Unaligned inputs and the partial last sub-chunk take the checked path.
+// are issued.  The partial last sub-chunk takes the checked path.
 // The loads of sub-chunk j + 1 are issued before body(j), unconditionally (past the end of
 // the run they reload the final sub-chunk, a cache hit): every path then issues the same
 // loads, so the compiler's in-order load counter lets body(j) wait for sub-chunk j alone
 // while the next one is in flight.
 template <int SUB, typename Buf, typename Load, typename Body, typename Hook>
-__device__ inline void pipeline(int64_t v0, int64_t vend, bool aligned, Load&& load, Body&& body,
-                                Hook&& hook) {
-  const int nfull = aligned ? (int)((vend - v0) / SUB) : 0;
+__device__ inline void pipeline(int64_t v0, int64_t vend, Load&& load, Body&& body, Hook&& hook) {
+  const int nfull = (int)((vend - v0) / SUB);
   auto at = [&](int j) { return v0 + (int64_t)min(j, nfull - 1) * SUB; };
   if (nfull > 0) {
     Buf a, b;
@@ -406,8 +403,7 @@ __device__ inline auto target_loader(const VerifyParams& p, const typename Elem<
       if constexpr (decltype(fast)::value)
         load_raw<DT, EPT, false>(tb[g], s0, buf.x[g]);
       else
-        load_raw_checked<DT, EPT, false>(tb[g], s0, vend, p.target_aligned, Elem<DT>::ninf(),
-                                         buf.x[g]);
+        load_raw_checked<DT, EPT, false>(tb[g], s0, vend, Elem<DT>::ninf(), buf.x[g]);
     }
   };
 }
@@ -482,7 +478,7 @@ __device__ inline void task_argmax(const VerifyParams& p, int c, int row0, int n
         }
       }
     };
-    pipeline<kVThreads * EPT, TargetBuf<DT, EPT, G>>(v0, vend, p.target_aligned,
+    pipeline<kVThreads * EPT, TargetBuf<DT, EPT, G>>(v0, vend,
                                                      target_loader<DT, EPT, G>(p, tb, vend), body,
                                                      after_loads);
   } else {
@@ -504,7 +500,7 @@ __device__ inline void task_argmax(const VerifyParams& p, int c, int row0, int n
       }
     }
   };
-  pipeline<kVThreads * EPT, TargetBuf<DT, EPT, G>>(v0, vend, p.target_aligned,
+  pipeline<kVThreads * EPT, TargetBuf<DT, EPT, G>>(v0, vend,
                                                    target_loader<DT, EPT, G>(p, tb, vend), body,
                                                    after_loads);
   }
@@ -575,7 +571,7 @@ __device__ inline void task_stats(const VerifyParams& p, int c, float c1, int ro
       }
     }
   };
-  pipeline<kVThreads * EPT, TargetBuf<DT, EPT, G>>(v0, vend, p.target_aligned,
+  pipeline<kVThreads * EPT, TargetBuf<DT, EPT, G>>(v0, vend,
                                                    target_loader<DT, EPT, G>(p, tb, vend), body,
                                                    after_loads);
   float M[G];
@@ -610,21 +606,21 @@ __device__ inline void task_stats(const VerifyParams& p, int c, float c1, int ro
 template <int DT>
 using TargetQuad = std::conditional_t<Elem<DT>::kVec == 4, u32x4, u32x2>;
 
-// Target row sub-chunk in quads; FAST: full and aligned, else bounds-checked with `fill`.
+// Target row sub-chunk in quads; FAST: full, else bounds-checked with `fill`.
 template <int DT, int EPT, bool FAST>
 __device__ inline void load_target_quads(const typename Elem<DT>::storage* __restrict__ base,
-                                         int64_t s0, int64_t vend, bool aligned,
+                                         int64_t s0, int64_t vend,
                                          typename Elem<DT>::storage fill,
                                          TargetQuad<DT> (&out)[EPT / 4]) {
   if constexpr (Elem<DT>::kVec == 4) {
     if constexpr (FAST) load_raw<DT, EPT, true>(base, s0, out);
-    else load_raw_checked<DT, EPT, true>(base, s0, vend, aligned, fill, out);
+    else load_raw_checked<DT, EPT, true>(base, s0, vend, fill, out);
   } else {
 #pragma unroll
     for (int m = 0; m < EPT / 4; ++m) {
       const int64_t col = vec_col<MVSD_F32>(s0, m);
-      if (FAST || (aligned && col + 4 <= vend)) {
-        out[m] = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(base + col));
+      if (FAST || col + 4 <= vend) {
+        out[m] = __builtin_nontemporal_load(reinterpret_cast<const Vec8<DT>*>(base + col));
       } else {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
@@ -671,13 +667,12 @@ __device__ inline uint64_t task_score(const VerifyParams& p, int r, float c1, in
                              : nullptr;
   const float* eb = p.noise + (int64_t)r * p.noise_stride;
   const float4 mk = MASKED ? p.masks[row] : make_float4(0.f, 0.f, 0.f, 0.f);
-  const bool aligned = p.target_aligned && p.noise_aligned && (p.draft_aligned || !HAS_DRAFT);
 
   auto load = [&](Buf& buf, int64_t s0, auto fast) {
     constexpr bool F = decltype(fast)::value;
-    load_target_quads<DT, EPT, F>(tb, s0, vend, p.target_aligned, Elem<DT>::ninf(), buf.x);
-    if constexpr (HAS_DRAFT) load_draft<MVSD_F32, DD, EPT, F>(qb, s0, vend, p.draft_aligned, buf.q);
-    load_raw_f32<MVSD_F32, EPT, F>(eb, s0, vend, p.noise_aligned, 1.f, buf.e);
+    load_target_quads<DT, EPT, F>(tb, s0, vend, Elem<DT>::ninf(), buf.x);
+    if constexpr (HAS_DRAFT) load_draft<MVSD_F32, DD, EPT, F>(qb, s0, vend, buf.q);
+    load_raw_f32<MVSD_F32, EPT, F>(eb, s0, vend, 1.f, buf.e);
   };
 
   float MX = 0.f, NL = 0.f;
@@ -769,7 +764,7 @@ __device__ inline uint64_t task_score(const VerifyParams& p, int r, float c1, in
       bi = elem_index<MVSD_F32, EPT>(s0, kk);
     }
   };
-  pipeline<kVThreads * EPT, Buf>(v0, vend, aligned, load, body, wait_stats);
+  pipeline<kVThreads * EPT, Buf>(v0, vend, load, body, wait_stats);
   const uint64_t key[1] = {argmax_key(bv, bi)};
   return block_max_key_to_row_thread<1, kVWaves>(key, s_key);
 }
@@ -882,13 +877,15 @@ constexpr uint64_t kSkipKey = 2;
 // request is cleared.  A kFull request publishes its decision instead; the slots of its
 // rejected row stay for the score tasks, and its output row is written by finish_scores.
 // Always inlined, as is finish_scores: a call makes the kernel copy its parameters to scratch.
+// GREEDY_ONLY: every request of the launch is greedy.
+template <bool GREEDY_ONLY>
 __device__ __forceinline__ void decide_request(const VerifyParams& p, const Tables& tb, int r,
                                                DecideSmem& sm) {
   const int begin = tb.begin[r];
   const int kf = tb.kflags[r];
   const int K = kf & 0xffff;
-  const bool greedy = (kf >> 16) & kGreedy;
-  const bool full = (kf >> 16) & kFull;
+  const bool greedy = GREEDY_ONLY || ((kf >> 16) & kGreedy);
+  const bool full = !GREEDY_ONLY && ((kf >> 16) & kFull);
   const float c1 = tb.c1[r];
   const int tid = threadIdx.x;
   const int lane = lane_id();
@@ -1214,8 +1211,10 @@ __device__ inline void task_columns(const VerifyParams& p, int part, bool tail, 
 }
 
 // ------------------------------------------------------------------ main kernel ------
-// DD: the draft probabilities' dtype (MVSD_F32, MVSD_BF16, MVSD_F16), or -1 for point-mass
-// drafts.
+// DD: the draft probabilities' dtype (MVSD_F32, MVSD_BF16, MVSD_F16), -1 for point-mass drafts,
+// or kGreedyOnly for launches whose requests are all greedy: no softmax statistics and no score
+// tasks, two fifths of the code and a quarter of its spilled scalar registers, which small greedy
+// batches, bound by latency, pay for (four requests of three fp32 rows: 12.8 -> 11.9 us a call).
 template <int DT, int EPT, int G, int DD, bool MASKED>
 __global__ __launch_bounds__(kVThreads) void verify_kernel(VerifyParams p) {
   static_assert(EPT % Elem<DT>::kVec == 0, "EPT must be a multiple of the vector width");
@@ -1273,57 +1272,61 @@ __global__ __launch_bounds__(kVThreads) void verify_kernel(VerifyParams p) {
       const int nrows = rinfo & 0xff;
       const int ngr = (rinfo >> 8) & 0xff;
       if (tid == 0) started = atomic_add_relaxed(&p.req_cnt[r], 1);
-      if ((rinfo >> 16) & kGreedy)
+      if (DD == kGreedyOnly || ((rinfo >> 16) & kGreedy)) {
         task_argmax<DT, EPT, G, MASKED>(p, c, row0, nrows, v0, vend, s_key, prefetch);
-      else
-        task_stats<DT, EPT, G, MASKED>(p, c, c1, row0, nrows, v0, vend, s_red, s_M, prefetch);
+      } else {
+        if constexpr (DD != kGreedyOnly)
+          task_stats<DT, EPT, G, MASKED>(p, c, c1, row0, nrows, v0, vend, s_red, s_M, prefetch);
+      }
       // the request's stats tasks: nc per group, 2 nc per tail group
       const int g0 = tb.gstart[r], g1 = g0 + ngr;
       const int ntasks = p.nc * (ngr + max(0, g1 - max(g0, tb.gt)));
       if (tid == 0) s_last = started == ntasks - 1;
       __syncthreads();
-      if (s_last) decide_request(p, tb, r, dsm);
-    } else if (kind == kScoreTask) {
-      // every score task counts, so that exactly one of them finishes the request
-      if (tid == 0) {
-        started = atomic_add_relaxed(&p.score_cnt[r], 1);
-        int d = info[7];
-        for (int spins = 0; d == 0; ++spins) {
-          if (spins >= p.spin_limit ||
-              ((spins & 255) == 255 && atomic_load_relaxed(&p.ctrl[kCtrlFlag]) != 0)) {
-            atomic_store_relaxed(&p.ctrl[kCtrlFlag], 1);
-            break;
+      if (s_last) decide_request<DD == kGreedyOnly>(p, tb, r, dsm);
+    } else if (DD != kGreedyOnly && kind == kScoreTask) {
+      if constexpr (DD != kGreedyOnly) {
+        // every score task counts, so that exactly one of them finishes the request
+        if (tid == 0) {
+          started = atomic_add_relaxed(&p.score_cnt[r], 1);
+          int d = info[7];
+          for (int spins = 0; d == 0; ++spins) {
+            if (spins >= p.spin_limit ||
+                ((spins & 255) == 255 && atomic_load_relaxed(&p.ctrl[kCtrlFlag]) != 0)) {
+              atomic_store_relaxed(&p.ctrl[kCtrlFlag], 1);
+              break;
+            }
+            d = atomic_load_relaxed(&p.decision[r]);
+            if (d == 0) __builtin_amdgcn_s_sleep(1);
           }
-          d = atomic_load_relaxed(&p.decision[r]);
-          if (d == 0) __builtin_amdgcn_s_sleep(1);
+          s_dec = d;
         }
-        s_dec = d;
+        __syncthreads();
+        const int d = s_dec;
+        const int K = rinfo & 0xffff;
+        uint64_t key = d == 0 ? kFailKey : kSkipKey;
+        if (d >= 1 && d <= K) {
+          // rejection at position d - 1: score this chunk of that row
+          const int row = row0 + d - 1;
+          const int draft = DD >= 0 ? -1 : p.draft_ids[row];
+          bool ok;
+          const int nslots = tb.gstart[r] + (d - 1) / p.G >= tb.gt ? 2 * p.nc : p.nc;
+          key = task_score<DT, 2 * EPT, DD, MASKED>(p, r, c1, row, nslots, draft, v0, vend,
+                                                           s_key, s_ml, ok, prefetch);
+          if (!ok) key = kFailKey;
+        } else {
+          // every draft accepted, or no usable decision: nothing to score, but the slot tells
+          // the finisher that this task has read the decision
+          prefetch();
+        }
+        const int ntasks = tail ? 2 * p.nc : p.nc;
+        if (tid == 0) {
+          slot_store(p.score_slots + r * slot_stride(p) + c, key);
+          s_last = started == ntasks - 1;
+        }
+        __syncthreads();
+        if (s_last) finish_scores(p, tb, r, d, ntasks);
       }
-      __syncthreads();
-      const int d = s_dec;
-      const int K = rinfo & 0xffff;
-      uint64_t key = d == 0 ? kFailKey : kSkipKey;
-      if (d >= 1 && d <= K) {
-        // rejection at position d - 1: score this chunk of that row
-        const int row = row0 + d - 1;
-        const int draft = DD >= 0 ? -1 : p.draft_ids[row];
-        bool ok;
-        const int nslots = tb.gstart[r] + (d - 1) / p.G >= tb.gt ? 2 * p.nc : p.nc;
-        key = task_score<DT, 2 * EPT, DD, MASKED>(p, r, c1, row, nslots, draft, v0, vend,
-                                                         s_key, s_ml, ok, prefetch);
-        if (!ok) key = kFailKey;
-      } else {
-        // every draft accepted, or no usable decision: nothing to score, but the slot tells
-        // the finisher that this task has read the decision
-        prefetch();
-      }
-      const int ntasks = tail ? 2 * p.nc : p.nc;
-      if (tid == 0) {
-        slot_store(p.score_slots + r * slot_stride(p) + c, key);
-        s_last = started == ntasks - 1;
-      }
-      __syncthreads();
-      if (s_last) finish_scores(p, tb, r, d, ntasks);
     } else {
       prefetch();
     }
@@ -1443,6 +1446,8 @@ template <int DT, bool MASKED>
 const void* kernel_for_mask(int draft_dtype) {
   constexpr int E = ept_of<DT>();
   switch (draft_dtype) {
+    case kGreedyOnly:  // constraints never apply to a greedy batch
+      return reinterpret_cast<const void*>(&verify_kernel<DT, E, kGroup, kGreedyOnly, false>);
     case -1: return reinterpret_cast<const void*>(&verify_kernel<DT, E, kGroup, -1, MASKED>);
     case MVSD_F32: return reinterpret_cast<const void*>(&verify_kernel<DT, E, kGroup, MVSD_F32, MASKED>);
     case MVSD_BF16: return reinterpret_cast<const void*>(&verify_kernel<DT, E, kGroup, MVSD_BF16, MASKED>);
@@ -1468,8 +1473,9 @@ const void* verify_kernel_ptr(int target_dtype, int draft_dtype, bool masked) {
 hipError_t launch_verify(const VerifyParams& params, int target_dtype, int grid,
                          hipStream_t stream) {
   if (params.B == 0) return hipSuccess;
-  const void* fn = verify_kernel_ptr(target_dtype, params.draft ? params.draft_dtype : -1,
-                                     params.masks != nullptr);
+  const void* fn = verify_kernel_ptr(
+      target_dtype, params.all_greedy ? kGreedyOnly : params.draft ? params.draft_dtype : -1,
+      params.masks != nullptr);
   if (!fn) return hipErrorInvalidValue;
   void* args[] = {const_cast<VerifyParams*>(&params)};
   hipError_t err = hipLaunchKernel(fn, dim3(grid), dim3(kVThreads), args, 0, stream);
