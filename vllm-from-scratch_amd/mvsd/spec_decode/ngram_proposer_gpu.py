@@ -1,11 +1,12 @@
 """Device-resident ngram proposer (drop-in for minivllm/spec_decode/ngram_proposer_gpu.py).
 
 ``NgramGPUKernel.forward`` and the match inside ``NgramProposerGPU.propose`` are one HIP
-launch (``mvsd_ngram_propose_split``): one workgroup per request, or several where histories may
-be longer than 4096 tokens, stages the history through LDS, computes for every window end the common-suffix length with the history's tail, and keeps the
-earliest end per n-gram length.  ``propose`` also folds the in-place scatter of this step's
-sampled tokens into that launch.  Results are ``drafts [B, k]`` int32 (-1 padded) and
-``num_valid [B]`` int32 (leading valid count).
+launch (``mvsd_ngram_propose``, or ``mvsd_ngram_propose_split`` where histories may be longer than
+8192 tokens): one workgroup per request, or several, stages the history through LDS, computes for
+every window end the common-suffix length with the history's tail, and keeps the earliest end per
+n-gram length.  ``propose`` also folds the in-place scatter of this step's sampled tokens into
+that launch.  Results are ``drafts [B, k]`` int32 (-1 padded) and ``num_valid [B]`` int32
+(leading valid count).
 
 Semantics follow the reference (:56-148, :204-245): largest n in [min_n, max_n] with a match,
 earliest window among equals, at least one token after the window, no max_model_len cap.
@@ -20,24 +21,21 @@ from ..outputs import DraftTokenIds
 from .utils import TargetRows, update_scheduler_for_invalid_drafts  # noqa: F401
 
 
-# Buffers no longer than one tile hold histories that one workgroup covers in one step.
-_SPLIT_FROM = 4096 + 1
+# Up to two tiles of 4096 tokens, one workgroup is done before the host has the next call ready.
+_SPLIT_FROM = 2 * 4096 + 1
 
-# One cleared workspace per (device, stream), of one fixed size (67 kB): calls on a stream run one
-# after another and leave it cleared, calls on different streams have their own.
+# One cleared workspace per (device, stream), of one fixed size (mvsd_ngram_workspace_bytes fits
+# it): calls on a stream run one after another and leave it cleared, calls on different streams
+# have their own.
 _WORKSPACES: dict[tuple[int, int], torch.Tensor] = {}
+_WORKSPACE_BYTES = 1 << 17
 
 
 def _workspace(device: torch.device, stream: int) -> torch.Tensor:
-    key = (device.index if device.index is not None else torch.cuda.current_device(), stream)
-    ws = _WORKSPACES.get(key)
-    if ws is None:
-        handle = nat.lib()
-        ws = torch.empty(handle.mvsd_ngram_workspace_bytes(), dtype=torch.uint8, device=device)
-        nat.check(handle.mvsd_ngram_workspace_init(ws.data_ptr(), ws.numel(), stream),
-                  "mvsd_ngram_workspace_init")
-        ws = _WORKSPACES.setdefault(key, ws)
-    return ws
+    ws = torch.empty(_WORKSPACE_BYTES, dtype=torch.uint8, device=device)
+    nat.check(nat.lib().mvsd_ngram_workspace_init(ws.data_ptr(), ws.numel(), stream),
+              "mvsd_ngram_workspace_init")
+    return _WORKSPACES.setdefault((device.index, stream), ws)
 
 
 def ngram_propose_device(token_ids: torch.Tensor, num_tokens: torch.Tensor, *, min_n: int,
@@ -77,23 +75,26 @@ def ngram_propose_device(token_ids: torch.Tensor, num_tokens: torch.Tensor, *, m
         new_stride, max_new = new.stride(0), new.shape[1]
         counts = new_counts[:num_reqs].to(torch.int32).contiguous()
     width = token_ids.shape[1]
+    out_ptr = out.data_ptr()
     if width <= _SPLIT_FROM or torch.cuda.is_current_stream_capturing():
         # (a captured launch could be replayed beside a later call on this stream, so it gets no
         # workspace)
         status = nat.lib().mvsd_ngram_propose(
-            drafts.data_ptr(), num_valid.data_ptr(), token_ids.data_ptr(), token_ids.stride(0),
+            out_ptr, out_ptr + 4 * num_reqs * k, token_ids.data_ptr(), token_ids.stride(0),
             width, lengths.data_ptr(), None if new is None else new.data_ptr(), new_stride,
             max_new, None if counts is None else counts.data_ptr(),
             None if act is None else act.data_ptr(), int(gate_on_new_counts), num_reqs, min_n,
             max_n, k, int(cap_by_model_len), max_model_len, nat.stream_of(device))
     else:
         stream = nat.stream_of(device)
-        workspace = _workspace(device, stream)
+        workspace = _WORKSPACES.get((device.index, stream))
+        if workspace is None:
+            workspace = _workspace(device, stream)
         status = nat.lib().mvsd_ngram_propose_split(
-            drafts.data_ptr(), num_valid.data_ptr(), token_ids.data_ptr(), token_ids.stride(0),
+            out_ptr, out_ptr + 4 * num_reqs * k, token_ids.data_ptr(), token_ids.stride(0),
             width, lengths.data_ptr(), nat.ptr(new), new_stride, max_new, nat.ptr(counts),
             nat.ptr(act), int(gate_on_new_counts), num_reqs, min_n, max_n, k,
-            int(cap_by_model_len), max_model_len, workspace.data_ptr(), workspace.numel(), stream)
+            int(cap_by_model_len), max_model_len, workspace.data_ptr(), _WORKSPACE_BYTES, stream)
     if status:
         nat.check(status, "mvsd_ngram_propose")
     return drafts, num_valid
