@@ -364,6 +364,20 @@ int mvsd_apply_logits_processors(float* logits, int64_t stride, int64_t num_toke
                                  const int32_t* n_mask, const int32_t* stop_off,
                                  const int32_t* stop_tok, mvsd_stream_t stream);
 
+/* The penalties of a whole step's compact rows in one call: request r has                   */
+/* cu_num_sampled_tokens[r] - cu_num_sampled_tokens[r-1] = K_r + 1 rows, its verify rows      */
+/* (logits rows target_rows[verify row]) and its bonus row (logits row bonus_rows[r]), whose  */
+/* history holds all K_r drafts; spec_tokens [num_rows] lists each request's drafts and one   */
+/* filler (-1).  The entries and penalties as for mvsd_apply_logits_processors.               */
+int mvsd_apply_step_penalties(float* logits, int64_t stride, int64_t num_rows, int64_t vocab_size,
+                              int64_t batch_size, const int32_t* cu_num_sampled_tokens,
+                              const int32_t* target_rows, const int32_t* bonus_rows,
+                              const int32_t* spec_tokens, const int32_t* ent_off,
+                              const int32_t* ent_tok, const int32_t* ent_info,
+                              const float* presence, const float* frequency,
+                              const float* repetition, mvsd_stream_t stream);
+
+
 /* ------------------------------------------------------------------------------------ */
 /* spec_logprobs — logprobs of every output position of a verification step.              */
 /* Replaces: RejectionSampler._get_logprobs_tensors, minivllm/sample/rejection_sampler.py: */

@@ -1,0 +1,54 @@
+"""The penalties' host summaries (csrc/hostops.c) against numpy's distinct values and counts."""
+
+import numpy as np
+import pytest
+
+from mvsd import _hostops
+from mvsd.sample.rejection_sampler import _penalty_entries
+
+
+def check(prompts, outputs, specs):
+    off, tok, info = _penalty_entries(prompts, outputs, specs)
+    assert off.dtype == tok.dtype == info.dtype == np.int32
+    assert off.shape == (len(specs) + 1,) and off[0] == 0 and tok.size == info.size == off[-1]
+    for r, spec in enumerate(specs):
+        prompt = list(prompts[r]) if r < len(prompts) else []
+        output = list(outputs[r]) if r < len(outputs) else []
+        got = {int(t): int(i) for t, i in zip(tok[off[r]:off[r + 1]], info[off[r]:off[r + 1]])}
+        assert len(got) == off[r + 1] - off[r]  # distinct
+        want = {t: output.count(t) | (-2 ** 31 if t in prompt else 0)
+                for t in {*prompt, *output, *spec}}
+        assert got == want
+
+
+@pytest.mark.parametrize("n", [0, 1, 7, 8, 9, 300])
+@pytest.mark.parametrize("vocab", [1, 5, 150000])
+def test_counts(n, vocab):
+    rng = np.random.default_rng(n + vocab)
+    lists = lambda scale: [rng.integers(0, vocab, rng.integers(0, scale * n + 1)).tolist()
+                           for _ in range(9)]
+    check(lists(3), lists(1), [s[:6] for s in lists(1)])
+
+
+def test_forms_of_input():
+    check([], [], [])
+    check([], [[5]], [[1, 2], [], [-1]])                       # missing tail requests
+    check([(1, 2, 1)], [np.array([2, 2, 9])], [range(3)])      # any sequence of integers
+    check([[np.int64(7), 7, True]], [[0]], [[7]])
+    check([[2 ** 31 - 1, -1, -2 ** 31]], [[2 ** 31 - 1]], [[]])
+    off, tok, info = _penalty_entries([[1.0, 2.0]], [[2.0]], [[3]])  # as np.asarray reads them
+    assert sorted(zip(tok.tolist(), info.tolist())) == [(1, -2 ** 31), (2, 1 - 2 ** 31), (3, 0)]
+
+
+def test_errors():
+    room = np.empty(64, dtype=np.int32)
+    with pytest.raises(TypeError):
+        _hostops.penalty_entries([["a"]], [[]], [[]], room)
+    with pytest.raises(TypeError):
+        _hostops.penalty_entries([3], [[]], [[]], room)
+    with pytest.raises(OverflowError):
+        _hostops.penalty_entries([[2 ** 70]], [[]], [[]], room)
+    with pytest.raises(ValueError):
+        _hostops.penalty_entries([[1, 2, 3]], [[4]], [[5]], room[:8])
+    with pytest.raises(ValueError):
+        _hostops.penalty_entries([], [], [[]] * 9, room[:4])

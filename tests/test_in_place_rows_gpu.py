@@ -82,3 +82,33 @@ def test_forward(device, dtype, limits, V, B, greedy):
         torch.manual_seed(11)
         outs.append(rs.RejectionSampler(cls()).forward(meta, probs, logits.clone(), sm))
     same(*outs, LP_ATOL)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("limits", ["", "kp"])
+@pytest.mark.parametrize("V,B,greedy", [(500, 7, 0), (65600, 6, 2), (3001, 5, 4), (700, 1, 0)])
+def test_forward_with_penalties(device, dtype, limits, V, B, greedy):
+    """Verify and bonus rows penalised in one launch against the general path's two."""
+    g = torch.Generator(device=device).manual_seed(V + B)
+    host = torch.Generator().manual_seed(V)
+    tokens = lambda n: torch.randint(0, min(V, 60), (n,), generator=host).tolist()
+    drafts = [tokens((i + 1) % 5) for i in range(B)]
+    meta = make_metadata(drafts, device=device)
+    P = sum(len(d) for d in drafts)
+    logits = (torch.randn(P + B, V, device=device, generator=g) * 2.5).to(dtype)
+    probs = torch.softmax(torch.randn(P, V, device=device, generator=g) * 2.5, -1)
+    temps, top_k, top_p = params(B, V, limits, greedy, g)
+    sm = sampling_metadata(
+        temps, drafts, device=device, top_k=top_k, top_p=top_p, max_num_logprobs=3,
+        no_penalties=False, prompt_token_ids=[tokens(20 * i) for i in range(B)],
+        output_token_ids=[tokens(9 * (B - i)) for i in range(B)],
+        presence_penalties=[0.3 * (i % 3) for i in range(B)],
+        frequency_penalties=[0.2 * (i % 2) for i in range(B)],
+        repetition_penalties=[1.0 + 0.3 * (i % 4) for i in range(B)])
+    before = logits.clone()
+    outs = []
+    for cls in (Sampler, General):
+        torch.manual_seed(11)
+        outs.append(rs.RejectionSampler(cls()).forward(meta, probs, logits, sm))
+    same(*outs, LP_ATOL)
+    assert torch.equal(logits, before)

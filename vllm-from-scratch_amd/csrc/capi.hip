@@ -475,7 +475,7 @@ int mvsd_apply_logits_processors(float* logits, int64_t stride, int64_t num_toke
   if (!logits || stride < vocab_size || !cu_num_draft_tokens) return MVSD_E_INVALID;
   if (ent_off && (!ent_tok || !ent_info || !spec_tokens)) return MVSD_E_INVALID;
   if (n_mask && (!stop_off || !stop_tok)) return MVSD_E_INVALID;
-  mvsd::ProcessorParams p;
+  mvsd::ProcessorParams p{};
   p.logits = logits;
   p.stride = stride;
   p.P = (int)num_tokens;
@@ -492,6 +492,40 @@ int mvsd_apply_logits_processors(float* logits, int64_t stride, int64_t num_toke
   p.n_mask = n_mask;
   p.stop_off = stop_off;
   p.stop_tok = stop_tok;
+  return hip_status(mvsd::launch_logits_processors(p, (hipStream_t)stream));
+}
+
+int mvsd_apply_step_penalties(float* logits, int64_t stride, int64_t num_rows, int64_t vocab_size,
+                              int64_t batch_size, const int32_t* cu_num_sampled_tokens,
+                              const int32_t* target_rows, const int32_t* bonus_rows,
+                              const int32_t* spec_tokens, const int32_t* ent_off,
+                              const int32_t* ent_tok, const int32_t* ent_info,
+                              const float* presence, const float* frequency,
+                              const float* repetition, mvsd_stream_t stream) {
+  if (num_rows < 0 || batch_size < 0 || vocab_size <= 0) return MVSD_E_INVALID;
+  if (num_rows == 0 || batch_size == 0) return MVSD_OK;
+  if (num_rows > 0x7fffffff || batch_size > 0x7fffffff || vocab_size > 0x7fffffff)
+    return MVSD_E_RANGE;
+  if (!logits || stride < vocab_size || !cu_num_sampled_tokens || !bonus_rows || !spec_tokens ||
+      !ent_off || !ent_tok || !ent_info)
+    return MVSD_E_INVALID;
+  if (num_rows > batch_size && !target_rows) return MVSD_E_INVALID;
+  mvsd::ProcessorParams p{};
+  p.logits = logits;
+  p.stride = stride;
+  p.P = (int)num_rows;
+  p.V = (int)vocab_size;
+  p.B = (int)batch_size;
+  p.cu = cu_num_sampled_tokens;
+  p.target_rows = target_rows;
+  p.bonus_rows = bonus_rows;
+  p.spec = spec_tokens;
+  p.ent_off = ent_off;
+  p.ent_tok = ent_tok;
+  p.ent_info = ent_info;
+  p.presence = presence;
+  p.frequency = frequency;
+  p.repetition = repetition;
   return hip_status(mvsd::launch_logits_processors(p, (hipStream_t)stream));
 }
 

@@ -14,6 +14,11 @@ struct ProcessorParams {
   int B;
   const int32_t* cu;    // [B] cumulative draft counts, no leading 0
   const int32_t* spec;  // [P] draft token of each row (request r's drafts, in order)
+  // A step's compact rows (both null: the rows are verify rows, in place): cu counts K_r + 1 rows
+  // per request, row j < K_r of request r is logits row target_rows[verify row], its last row
+  // logits row bonus_rows[r] (each clamped to [0, P)).
+  const int32_t* target_rows;
+  const int32_t* bonus_rows;
   // penalties (ent_off null: none)
   const int32_t* ent_off;   // [B + 1] offsets into ent_tok / ent_info
   const int32_t* ent_tok;   // distinct tokens of each request's prompt, output and drafts

@@ -36,7 +36,13 @@ __global__ __launch_bounds__(kProcThreads) void logits_processors_kernel(Process
   const int r = lo;
   const int begin = r == 0 ? 0 : p.cu[r - 1];
   const int j = row - begin;  // position of the row in its request's draft block
-  float* x = p.logits + (int64_t)row * p.stride;
+  int64_t at = row;
+  if (p.bonus_rows) {
+    // verify rows before compact row `row`: all rows before it but r bonus rows
+    at = row == p.cu[r] - 1 ? p.bonus_rows[r] : p.target_rows[row - r];
+    at = min(max(at, (int64_t)0), (int64_t)p.P - 1);
+  }
+  float* x = p.logits + at * p.stride;
 
   if (p.ent_off) {
     const float rep = p.repetition ? p.repetition[r] : 1.f;

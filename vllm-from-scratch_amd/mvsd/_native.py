@@ -97,6 +97,8 @@ SIGNATURES = {
     "mvsd_sample_recovered_tokens": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64,
                                              c_void_p, c_int64, c_void_p, c_int64, c_int64,
                                              c_int64, c_int64, c_int64, c_void_p]),
+    "mvsd_apply_step_penalties": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_int64]
+                                  + [c_void_p] * 11),
     "mvsd_apply_logits_processors": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_int64,
                                              c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                              c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,

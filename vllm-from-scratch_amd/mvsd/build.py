@@ -1,4 +1,5 @@
-"""Build recipe for libmvsd.so (the HIP kernels + C ABI declared in include/mvsd.h).
+"""Build recipe for libmvsd.so (the HIP kernels + C ABI declared in include/mvsd.h) and for the
+host extension module _hostops.so (csrc/hostops.c, compiled by the C compiler).
 
 Compiles every ``csrc/*.hip`` for gfx950 with hipcc (one object per source, in parallel) and
 links them into one shared library next to this file.  Flags:
@@ -26,6 +27,7 @@ CSRC_DIR = PACKAGE_DIR.parent / "csrc"
 INCLUDE_DIR = PACKAGE_DIR.parent.parent / "include"
 LIB_NAME = "libmvsd.so"
 LIB_PATH = PACKAGE_DIR / LIB_NAME
+HOSTOPS_PATH = PACKAGE_DIR / "_hostops.so"  # CPython extension module, host code only
 
 OFFLOAD_ARCH = os.environ.get("MVSD_OFFLOAD_ARCH", "gfx950")
 
@@ -60,8 +62,24 @@ def _run(cmd: list[str]) -> str:
     noise = "packed-fp32-ops"
     stderr = "\n".join(line for line in proc.stderr.splitlines() if noise not in line)
     if proc.returncode != 0:
-        raise RuntimeError(f"hipcc failed ({proc.returncode}): {' '.join(cmd)}\n{stderr}")
+        raise RuntimeError(f"{cmd[0]} failed ({proc.returncode}): {' '.join(cmd)}\n{stderr}")
     return stderr
+
+
+def build_hostops() -> list[str]:
+    """Compile csrc/hostops.c into mvsd/_hostops.so and return the command."""
+    import sysconfig
+
+    cc = next((c for c in (os.environ.get("CC"), shutil.which("gcc"), shutil.which("cc"))
+               if c and shutil.which(c)), None)
+    if cc is None:
+        raise RuntimeError("no C compiler found: set CC")
+    tmp = HOSTOPS_PATH.with_suffix(".so.tmp")
+    cmd = [cc, "-O2", "-Wall", "-shared", "-fPIC", f"-I{sysconfig.get_paths()['include']}", "-o",
+           str(tmp), str(CSRC_DIR / "hostops.c")]
+    _run(cmd)
+    tmp.replace(HOSTOPS_PATH)
+    return cmd
 
 
 def build(verbose: bool = False) -> Path:
@@ -72,6 +90,7 @@ def build(verbose: bool = False) -> Path:
     import tempfile
     from concurrent.futures import ThreadPoolExecutor
 
+    hostops = build_hostops()
     srcs = sources()
     if not srcs:
         raise RuntimeError(f"no HIP sources under {CSRC_DIR}")
@@ -88,7 +107,7 @@ def build(verbose: bool = False) -> Path:
                 *map(str, objs)]
         logs.append(_run(link))
     if verbose:
-        for cmd in cmds + [link]:
+        for cmd in [hostops, *cmds, link]:
             print(" ".join(cmd), flush=True)
         for log in logs:
             if log.strip():

@@ -109,7 +109,7 @@ class RejectionSampler:
                 "speculative decoding with logprobs=-1 (the whole vocabulary) is not supported; "
                 "request logprobs=k with k >= 1")
 
-        if self._bonus_rows_race_only(sampling_metadata, logits):
+        if self._bonus_rows_race_only(metadata, sampling_metadata, logits):
             return self._forward_race_only(metadata, draft_probs, logits, sampling_metadata)
 
         # 1) bonus tokens from the bonus rows with the regular sampler (:169-181); their
@@ -178,24 +178,31 @@ class RejectionSampler:
         return SamplerOutput(sampled_token_ids=output_token_ids,
                              logprobs_tensors=logprobs_tensors)
 
-    def _bonus_rows_race_only(self, sm: SamplingMetadata, logits: torch.Tensor) -> bool:
+    def _bonus_rows_race_only(self, metadata: "SpecDecodeMetadata", sm: SamplingMetadata,
+                              logits: torch.Tensor) -> bool:
         """True when the caller's sampler is mvsd.sample.Sampler itself and, for this batch,
-        it would only take each bonus row's argmax or exponential race under its top-k / top-p:
-        no penalty or active min_tokens, no min_p, and no logprobs but raw ones; and the
-        recovered-token seam is the module's own."""
+        it would only take each bonus row's argmax or exponential race under its penalties and
+        top-k / top-p: no active min_tokens, no min_p, and no logprobs but raw ones; with
+        penalties, compact rows of this batch alone and every request's drafts in the sampling
+        metadata; and the recovered-token seam is the module's own."""
         from .sampler import Sampler as DeviceSampler
 
         return (type(self.sampler) is DeviceSampler and not self.is_processed_logprobs_mode
-                and sm.no_penalties and not _has_active_min_tokens(sm) and sm.min_p is None
+                and not _has_active_min_tokens(sm) and sm.min_p is None
                 and sample_recovered_tokens is _SAMPLE_RECOVERED_TOKENS
                 and (sm.all_greedy or sm.temperature is not None)
                 and logits.dtype in (torch.float32, torch.bfloat16, torch.float16)
-                and logits.stride(1) == 1)
+                and logits.stride(1) == 1
+                and (sm.no_penalties
+                     or (logits.shape[0] == sum(metadata.num_draft_tokens) + len(
+                         metadata.num_draft_tokens)
+                         and list(map(len, sm.spec_token_ids)) == metadata.num_draft_tokens)))
 
     def _forward_race_only(self, metadata: "SpecDecodeMetadata",
                            draft_probs: torch.Tensor | None, logits: torch.Tensor,
                            sm: SamplingMetadata):
-        """forward when the bonus rows only need the race (``_bonus_rows_race_only``).
+        """forward when the bonus rows only need the race (``_bonus_rows_race_only``), after one
+        launch that penalises an fp32 copy of the rows where the batch has penalties.
 
         The randomness is drawn exactly as the reference draws it, in its order: the bonus
         rows' Exp(1) noise (Sampler.sample's random_sample, for every row unless the batch is
@@ -222,6 +229,9 @@ class RejectionSampler:
         if not all_greedy and num_tokens > 0:
             exp_noise = generate_exponential_noise(B, V, metadata.num_draft_tokens,
                                                    sm.generators, device)
+        raw_logits = logits
+        if not sm.no_penalties:
+            logits = self._penalised_rows(logits, metadata, sm)
         constrained = not all_greedy and (sm.top_k is not None or sm.top_p is not None)
         masks = bonus_masks = None
         if constrained:
@@ -240,10 +250,26 @@ class RejectionSampler:
             apply_top_k_top_p=constrained, row_masks=masks)
         logprobs_tensors = None
         if sm.max_num_logprobs is not None:
-            logprobs_tensors = self._get_logprobs_tensors(sm.max_num_logprobs, metadata, logits,
-                                                          None, None, output_token_ids)
+            logprobs_tensors = self._get_logprobs_tensors(
+                sm.max_num_logprobs, metadata, raw_logits, None, None, output_token_ids)
         return SamplerOutput(sampled_token_ids=output_token_ids,
                              logprobs_tensors=logprobs_tensors)
+
+    @staticmethod
+    def _penalised_rows(logits: torch.Tensor, metadata: "SpecDecodeMetadata",
+                        sm: SamplingMetadata) -> torch.Tensor:
+        """The step's rows as fp32 with every verify and bonus row penalised in one launch: a
+        bonus row's history, committed output and all drafts, is that of a verify row after the
+        last draft."""
+        device = logits.device
+        rows = (logits.clone() if logits.dtype == torch.float32 else logits.to(torch.float32))
+        _launch_logits_processors(
+            rows, metadata.cu_num_sampled_tokens, [k + 1 for k in metadata.num_draft_tokens],
+            [[*spec, -1] for spec in sm.spec_token_ids],
+            _penalty_entries(sm.prompt_token_ids, sm.output_token_ids, sm.spec_token_ids), sm,
+            None, target_rows=_as(metadata.target_logits_indices, torch.int32, device),
+            bonus_rows=_as(metadata.bonus_logits_indices, torch.int32, device))
+        return rows
 
     def _get_logprobs_tensors(self, max_num_logprobs: int, metadata: "SpecDecodeMetadata",
                               logits: torch.Tensor, target_logits: torch.Tensor | None,
@@ -421,25 +447,19 @@ class RejectionSampler:
 def _penalty_entries(prompts, outputs, specs):
     """Per request: the distinct tokens of prompt, committed output and drafts, each with
     its committed output count and prompt flag, as (ent_off [B+1], ent_tok, ent_info) int32
-    arrays with ent_info = count | in_prompt << 31."""
-    offs = [0]
-    toks: list[np.ndarray] = []
-    infos: list[np.ndarray] = []
-    for i, spec in enumerate(specs):
-        prompt = np.asarray(prompts[i] if i < len(prompts) else [], dtype=np.int64)
-        out = np.asarray(outputs[i] if i < len(outputs) else [], dtype=np.int64)
-        union = np.unique(np.concatenate([prompt, out, np.asarray(spec, dtype=np.int64)]))
-        out_vals, out_counts = np.unique(out, return_counts=True)
-        counts = np.zeros(union.shape[0], dtype=np.int64)
-        counts[np.searchsorted(union, out_vals)] = out_counts
-        in_prompt = np.isin(union, prompt)
-        toks.append(union)
-        infos.append(counts | (in_prompt.astype(np.int64) << 31))
-        offs.append(offs[-1] + union.shape[0])
-    tok = np.concatenate(toks) if toks else np.zeros(0, np.int64)
-    info = np.concatenate(infos) if infos else np.zeros(0, np.int64)
-    return (np.asarray(offs, dtype=np.int32), tok.astype(np.int32),
-            info.astype(np.uint32).view(np.int32))
+    arrays with ent_info = count | in_prompt << 31 (csrc/hostops.c)."""
+    from .. import _hostops
+
+    B = len(specs)
+    room = sum(sum(map(len, lists[:B])) for lists in (prompts, outputs, specs))
+    buffer = np.empty(B + 1 + 2 * room, dtype=np.int32)
+    try:
+        n = _hostops.penalty_entries(prompts, outputs, specs, buffer)
+    except TypeError:  # tokens that are no integers: as an array conversion reads them
+        whole = [[np.asarray(tokens, dtype=np.int64).tolist() for tokens in lists]
+                 for lists in (prompts, outputs, specs)]
+        n = _hostops.penalty_entries(*whole, buffer)
+    return buffer[:B + 1], buffer[B + 1:B + 1 + n], buffer[B + 1 + n:B + 1 + 2 * n]
 
 
 def _min_tokens_rows(sm: SamplingMetadata, num_draft: list[int]):
@@ -468,8 +488,20 @@ def _expand_opt(values: torch.Tensor | None, cu: torch.Tensor, num_rows: int):
     return None if values is None else expand_batch_to_tokens(values, cu, num_rows)
 
 
-def _launch_logits_processors(logits, cu, num_draft, specs, entries, penalties, masks):
-    """One mvsd_apply_logits_processors launch on fp32 rows ``logits`` (request-major)."""
+def _upload(arrays, device) -> list[torch.Tensor]:
+    """int32 device copies of host arrays, through one pinned buffer and one copy that the host
+    does not wait for."""
+    arrays = [np.asarray(a, dtype=np.int32) for a in arrays]
+    host = torch.empty(sum(a.size for a in arrays), dtype=torch.int32, pin_memory=True)
+    np.concatenate(arrays, out=host.numpy())
+    return list(host.to(device, non_blocking=True).split([a.size for a in arrays]))
+
+
+def _launch_logits_processors(logits, cu, num_draft, specs, entries, penalties, masks,
+                              target_rows=None, bonus_rows=None):
+    """One mvsd_apply_logits_processors launch on fp32 rows ``logits`` (request-major), or, with
+    ``target_rows`` and ``bonus_rows``, on a step's compact rows: num_draft[i] = K_i + 1 rows of
+    request i, the K_i verify rows at ``target_rows`` and its bonus row at ``bonus_rows``."""
     assert logits.ndim == 2 and logits.dtype == torch.float32, "fp32 [P, V] logits expected"
     nat.require_device_tensor(logits, "logits")
     if logits.stride(1) != 1:
@@ -479,11 +511,6 @@ def _launch_logits_processors(logits, cu, num_draft, specs, entries, penalties, 
         raise ValueError(f"{num_rows} verify rows but {sum(num_draft)} draft tokens")
     device = logits.device
     keep = []
-
-    def dev(array, dtype=torch.int32):
-        t = torch.as_tensor(np.ascontiguousarray(array)).to(device=device, dtype=dtype)
-        keep.append(t)
-        return t.data_ptr()
 
     def dev_opt(values):
         if values is None:
@@ -498,21 +525,30 @@ def _launch_logits_processors(logits, cu, num_draft, specs, entries, penalties, 
         return
     cu_t = _as(cu, torch.int32, device)
     spec = np.asarray([t for row in specs for t in row], dtype=np.int32)
+    host = [spec, *(entries or ()), *(masks or ())]
+    on_device = iter(_upload(host, device))
+    spec_t = next(on_device)
     ent_off = ent_tok = ent_info = None
     presence = frequency = repetition = None
     if entries is not None:
-        ent_off, ent_tok, ent_info = (dev(a) for a in entries)
+        ent_off, ent_tok, ent_info = (next(on_device).data_ptr() for _ in range(3))
         presence = dev_opt(penalties.presence_penalties)
         frequency = dev_opt(penalties.frequency_penalties)
         repetition = dev_opt(penalties.repetition_penalties)
     n_mask = stop_off = stop_tok = None
     if masks is not None:
-        n_mask, stop_off, stop_tok = (dev(a) for a in masks)
-    nat.check(nat.lib().mvsd_apply_logits_processors(
-        logits.data_ptr(), logits.stride(0), num_rows, V, len(num_draft), cu_t.data_ptr(),
-        dev(spec) if spec.size else None, ent_off, ent_tok, ent_info, presence, frequency,
-        repetition, n_mask, stop_off, stop_tok, nat.stream_of(device)),
-        "mvsd_apply_logits_processors")
+        n_mask, stop_off, stop_tok = (next(on_device).data_ptr() for _ in range(3))
+    spec_ptr = spec_t.data_ptr() if spec.size else None
+    if bonus_rows is None:
+        nat.check(nat.lib().mvsd_apply_logits_processors(
+            logits.data_ptr(), logits.stride(0), num_rows, V, len(num_draft), cu_t.data_ptr(),
+            spec_ptr, ent_off, ent_tok, ent_info, presence, frequency, repetition, n_mask,
+            stop_off, stop_tok, nat.stream_of(device)), "mvsd_apply_logits_processors")
+    else:
+        nat.check(nat.lib().mvsd_apply_step_penalties(
+            logits.data_ptr(), logits.stride(0), num_rows, V, len(num_draft), cu_t.data_ptr(),
+            target_rows.data_ptr(), bonus_rows.data_ptr(), spec_ptr, ent_off, ent_tok, ent_info,
+            presence, frequency, repetition, nat.stream_of(device)), "mvsd_apply_step_penalties")
 
 
 def _has_active_min_tokens(sm: SamplingMetadata) -> bool:
