@@ -180,14 +180,18 @@ class RejectionSampler:
 
     def _bonus_rows_race_only(self, metadata: "SpecDecodeMetadata", sm: SamplingMetadata,
                               logits: torch.Tensor) -> bool:
-        """True when the caller's sampler is mvsd.sample.Sampler itself and, for this batch,
-        it would only take each bonus row's argmax or exponential race under its penalties and
-        top-k / top-p: no active min_tokens, no min_p, and no logprobs but raw ones; with
-        penalties, compact rows of this batch alone and every request's drafts in the sampling
-        metadata; and the recovered-token seam is the module's own."""
+        """True when the caller's sampler is mvsd.sample.Sampler itself (with its own top-k /
+        top-p sampler) and, for this batch, it would only take each bonus row's argmax or
+        exponential race under its penalties and top-k / top-p: no active min_tokens, no min_p,
+        and no logprobs but raw ones; with penalties, compact rows of this batch alone and every
+        request's drafts in the sampling metadata; and the recovered-token seam is the module's
+        own."""
         from .sampler import Sampler as DeviceSampler
+        from .sampler import TopKTopPSampler
 
-        return (type(self.sampler) is DeviceSampler and not self.is_processed_logprobs_mode
+        return (type(self.sampler) is DeviceSampler
+                and type(self.sampler.topk_topp_sampler) is TopKTopPSampler
+                and not self.is_processed_logprobs_mode
                 and not _has_active_min_tokens(sm) and sm.min_p is None
                 and sample_recovered_tokens is _SAMPLE_RECOVERED_TOKENS
                 and (sm.all_greedy or sm.temperature is not None)
