@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from mvsd import _native as nat
+from mvsd.spec_decode import ngram_proposer_gpu as ngram
 from mvsd.spec_decode.ngram_proposer_gpu import ngram_propose_device
 from oracle import ngram as oracle_ngram
 
@@ -60,3 +61,23 @@ def test_appended_tokens_equal_one_workgroup(device):
         nat.stream_of(device)), "mvsd_ngram_propose")
     assert torch.equal(a, b)
     assert torch.equal(drafts, want) and torch.equal(valid, want_valid)
+
+
+def test_kept_workspaces_are_bounded(device, monkeypatch):
+    """One workspace per stream, the oldest given back; each stream's results as before."""
+    monkeypatch.setattr(ngram, "_WORKSPACES", {})
+    monkeypatch.setattr(ngram, "_MAX_WORKSPACES", 2)
+    rng = np.random.default_rng(5)
+    lens = np.array([20000, 12290, 4097], dtype=np.int32)
+    tokens = histories(rng, lens, 20000, 50000)
+    want, counts = oracle_ngram.brute_device_batch(tokens, lens, 2, 5, 5)
+    t, n = torch.from_numpy(tokens).to(device), torch.from_numpy(lens).to(device)
+    torch.cuda.synchronize()
+    for _ in range(2):
+        for stream in [torch.cuda.Stream(device) for _ in range(4)]:
+            with torch.cuda.stream(stream):
+                drafts, valid = ngram_propose_device(t, n, min_n=2, max_n=5, k=5)
+            stream.synchronize()
+            assert len(ngram._WORKSPACES) <= 2
+            assert np.array_equal(drafts.cpu().numpy(), want)
+            assert np.array_equal(valid.cpu().numpy(), counts)

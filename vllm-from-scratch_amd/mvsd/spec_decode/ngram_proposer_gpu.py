@@ -26,7 +26,9 @@ _SPLIT_FROM = 2 * 4096 + 1
 
 # One cleared workspace per (device, stream), of one fixed size (mvsd_ngram_workspace_bytes fits
 # it): calls on a stream run one after another and leave it cleared, calls on different streams
-# have their own.
+# have their own.  At most _MAX_WORKSPACES are kept; the oldest goes back to the allocator, which
+# hands it out again in its stream's order only, after the launches that use it.
+_MAX_WORKSPACES = 64
 _WORKSPACES: dict[tuple[int, int], torch.Tensor] = {}
 _WORKSPACE_BYTES = 1 << 17
 
@@ -35,7 +37,10 @@ def _workspace(device: torch.device, stream: int) -> torch.Tensor:
     ws = torch.empty(_WORKSPACE_BYTES, dtype=torch.uint8, device=device)
     nat.check(nat.lib().mvsd_ngram_workspace_init(ws.data_ptr(), ws.numel(), stream),
               "mvsd_ngram_workspace_init")
-    return _WORKSPACES.setdefault((device.index, stream), ws)
+    ws = _WORKSPACES.setdefault((device.index, stream), ws)
+    while len(_WORKSPACES) > _MAX_WORKSPACES:
+        _WORKSPACES.pop(list(_WORKSPACES)[0], None)
+    return ws
 
 
 def ngram_propose_device(token_ids: torch.Tensor, num_tokens: torch.Tensor, *, min_n: int,
