@@ -125,3 +125,16 @@ def test_rows_in_place_equal_gathered_rows(device, dtype):
     # a 16-bit row's chunks sum in another order than the fp32 row's, which can move the log-sum
     # and each value (magnitude below 32) by one rounding: 2 * 2^-20
     assert (here.logprobs - there.logprobs).abs().max() <= 2 * 2.0 ** -20
+
+
+@pytest.mark.parametrize("V", [33, 2049, 50257, 151936])
+@pytest.mark.parametrize("k", [31, 32, 33])
+def test_bound_of_64_or_256_unions(device, V, k):
+    """The bound on the k-th largest comes from 64 unions of groups up to k = 32, from 256 above."""
+    g = torch.Generator(device=device).manual_seed(V + k)
+    x = torch.randn(5, V, device=device, generator=g) * 2.5
+    x[1] = x[1].sort(descending=True).values  # the largest side by side in one chunk
+    x[2, V // 2:] = -math.inf
+    x[3] = x[3].round()
+    check(x, k, torch.arange(5, device=device) * 5 % V)
+    check(x, k, torch.arange(5, device=device) * 5 % V, logits_mode=True)

@@ -271,23 +271,27 @@ __global__ __launch_bounds__(kLpThreads) void spec_logprobs_kernel(LogprobParams
 //   - M and S from the chunks, hence lp;
 //   - the rank: the count of entries x >= x_token, plus, where lp merges values (the largest entry
 //     below the token's value has the token's lp), those entries of the chunk counted again;
-//   - theta, the k-th largest of 256 disjoint unions of groups' maxima: at least k entries reach
-//     it, so the top-k are among the entries whose order value reaches theta's, and these lie in
-//     the groups whose maximum does (about k of them).  Their entries are gathered into LDS and
-//     ranked by counting.
+//   - theta, the k-th largest of the maxima of 256 disjoint unions of groups (64 for k <= 32, found
+//     by one wave: a sixteenth of the compares, and a few more candidates): at least k entries
+//     reach it, so the top-k are among the entries whose order value reaches theta's, and these lie in
+//     the groups whose maximum does (about k of them).  Their entries are gathered into LDS (one
+//     float compare passes over the positions where no lane holds a candidate) and ranked by
+//     counting.
 //   - More candidates than LDS holds: the entries strictly above theta, then as many entries equal
 //     to it as are missing, lowest index first; or, if even those above do not fit, the lists.
 // What bounds it: the scan is one read of the rows with about 12 VALU operations per entry
 // (127 us for 1280 fp32 rows of 151936 columns, 6.1 TB/s); the finish is a chain of a few small
-// loads and barriers (25 us for those rows, 10 us for 24).  The lists path spends about 40
+// loads and barriers (about 22 us for those rows, 27 before the 64 unions and the compare; 10 us
+// for 24).  The lists path spends about 40
 // operations on every entry (64-bit keys, serial insertion) and reads rows twice with 4-byte
-// loads: it took 2908 us for those 1280 rows with k = 20 (now 155 us in all), and 236 us for 24
+// loads: it took 2908 us for those 1280 rows with k = 20 (now 149 us in all), and 236 us for 24
 // bf16 rows with k = 5 (now 17 us).
 
 constexpr int kSplitMaxK = 128;       // theta is read off 256 keys
 constexpr int kGroupsPerChunk = 16;   // of 16 lanes each
 constexpr int kMaxGroups = 4096;      // LDS for the groups of one row
 constexpr int kLpCap = 1024;          // gathered candidates
+constexpr int kThetaWaveK = 32;       // largest k whose theta is read off 64 keys
 constexpr float kLpLog2e = 1.44269504088896340736f;
 
 // Columns per chunk: 8192, or 2048 where rows of 8192-column chunks would leave compute units
@@ -405,6 +409,7 @@ __global__ __launch_bounds__(kThreads) void lp_scan_kernel(LogprobParams p) {
 struct FinishSmem {
   uint64_t cand[kLpCap];
   __align__(16) uint32_t tkey[kThreads];
+  __align__(16) uint32_t theta_key[kWave];
   ListSmem<8, kWaves> lists;
   float red[kWaves];
   int wave_cnt[kWaves];
@@ -488,9 +493,27 @@ __global__ __launch_bounds__(kThreads) void lp_finish_kernel(LogprobParams p) {
   }
   if (k == 0) return;
 
-  // ---- theta: the k-th largest of the 256 threads' keys ----
-  {
-    // fewer than k keys are above the k-th largest, and it is the smallest such key
+  // ---- theta: the k-th largest of the 256 threads' keys, or of 64 maxima of four of them ----
+  // (fewer than k keys are above the k-th largest, and it is the smallest such key)
+  if (k <= kThetaWaveK) {  // block-uniform
+    uint32_t own = 0;
+    if (wid == 0) {
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) own = max(own, sm.tkey[w * kWave + lane]);
+      sm.theta_key[lane] = own;
+    }
+    __syncthreads();
+    if (wid == 0) {
+      int above = 0;
+      const uint4* keys = reinterpret_cast<const uint4*>(sm.theta_key);
+#pragma unroll
+      for (int j = 0; j < kWave / 4; ++j) {
+        const uint4 o = keys[j];
+        above += (o.x > own) + (o.y > own) + (o.z > own) + (o.w > own);
+      }
+      if (above < k) atomicMin(&sm.theta, own);
+    }
+  } else {
     int above = 0;
     const uint4* keys = reinterpret_cast<const uint4*>(sm.tkey);
 #pragma unroll 8
@@ -515,6 +538,7 @@ __global__ __launch_bounds__(kThreads) void lp_finish_kernel(LogprobParams p) {
 
   // ---- the entries of those groups whose order value is at or above `floor` ----
   auto gather = [&](uint32_t floor) {
+    const float floor_v = key_float(floor);
     for (int b = 0; b < nl; b += kThreads / 16) {
       const int li = b + tid / 16;
       const bool on = li < nl;
@@ -528,8 +552,11 @@ __global__ __launch_bounds__(kThreads) void lp_finish_kernel(LogprobParams p) {
       for (int j = 0; j < NV; ++j) {
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
+          const float v = vec_elem<DT>(q[j], e);
+          // most positions of the group hold no candidate (a NaN on either side goes on)
+          if (__ballot(!(ord(v) < floor_v)) == 0) continue;
           const int col = inside_col<DT>(c0 + j * kThreads * VEC, e, V);
-          const uint32_t key = ord_key(vec_elem<DT>(q[j], e));
+          const uint32_t key = ord_key(v);
           const bool take = on && col >= 0 && key >= floor;
           const uint64_t mask = __ballot(take);
           if (mask == 0) continue;
