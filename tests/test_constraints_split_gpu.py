@@ -98,3 +98,26 @@ def test_apply_in_place_equals_general_path(device, n, V):
         nat.stream_of(device)), "mvsd_apply_top_k_top_p")
     apply_top_k_top_p(wide[:, 1:V + 1], k, p)
     assert torch.equal(wide, want)
+
+
+def test_decreasing_counts_stay_inside_the_scratch(device):
+    """Cumulative draft counts that decrease list rows more than once: the plan keeps to its
+    room.  (The masks of such a batch mean nothing; the call reads and writes in bounds.)"""
+    P, V, guard = 64, 65536, 1 << 20
+    x = torch.randn(P, V, device=device)
+    cu = torch.tensor([P if r % 2 == 0 else 0 for r in range(P)], dtype=torch.int32, device=device)
+    ones = torch.ones(P, device=device)
+    top_p, top_k = ones * 0.9, torch.full((P,), V, device=device)
+    top_k[::3] = 20
+    need = nat.lib().mvsd_constraints_scratch_bytes(P, V)
+    buffer = torch.full((need + guard,), 0xA5, dtype=torch.uint8, device=device)
+    masks = torch.empty(P + 64, 4, device=device).fill_(7.0)
+    args = nat.RejectionArgs(
+        target_logits=x.data_ptr(), target_dtype=nat.F32, target_stride=V, target_num_rows=P,
+        cu_num_draft_tokens=cu.data_ptr(), temperature=ones.data_ptr(), all_greedy=0,
+        apply_temperature=1, batch_size=P, num_tokens=P, vocab_size=V, top_k=top_k.data_ptr(),
+        top_p=top_p.data_ptr())
+    nat.check(nat.lib().mvsd_sampling_masks_split(args, masks.data_ptr(), buffer.data_ptr(), need,
+                                                  nat.stream_of(x.device)),
+              "mvsd_sampling_masks_split")
+    assert (buffer[need:] == 0xA5).all() and (masks[P:] == 7.0).all()

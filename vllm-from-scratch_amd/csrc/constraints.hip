@@ -488,7 +488,8 @@ __global__ __launch_bounds__(1024) void constraint_plan_kernel(VerifyParams p) {
     const int c = request_class(p, r);
     if (c != 0 && end > begin) {
       const int at = base[c] + atomicAdd(&cnt[c], end - begin);
-      for (int j = begin; j < end; ++j) p.order[at + (j - begin)] = j + 1;
+      // (cumulative counts that decrease would list a row more than once: only P places)
+      for (int j = begin; j < min(end, p.P - at + begin); ++j) p.order[at + (j - begin)] = j + 1;
     }
   }
 }
@@ -1070,10 +1071,12 @@ __global__ __launch_bounds__(1024) void split_plan_kernel(SplitParams sp) {
     }
   }
   __syncthreads();
+  // the descriptors' room; cumulative counts that decrease would list a row more than once
+  const int room = p.P + (sp.bonus_rows ? p.B : 0);
   const int exact = cnt[1];
   if (tid == 0) {
-    sp.head->rows = exact + cnt[2];
-    sp.head->exact = exact;
+    sp.head->rows = min(exact + cnt[2], room);
+    sp.head->exact = min(exact, room);
   }
   __syncthreads();
   if (tid < 3) cnt[tid] = tid == 2 ? exact : 0;
@@ -1085,7 +1088,7 @@ __global__ __launch_bounds__(1024) void split_plan_kernel(SplitParams sp) {
     const int n = max(end - begin, 0) + (sp.bonus_rows ? 1 : 0);
     if (c == 0 || n == 0) continue;
     const int at = atomicAdd(&cnt[c], n);
-    for (int u = 0; u < n; ++u) {
+    for (int u = 0; u < n && at + u < room; ++u) {
       const int j = begin + u;
       SplitRow d{};
       d.row = j < end ? j : p.P + r;
