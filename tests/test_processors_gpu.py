@@ -14,6 +14,7 @@ import numpy as np
 import pytest
 import torch
 
+from mvsd import _native as nat
 from mvsd.outputs import SamplerOutput
 from mvsd.sample import rejection_sampler as rs
 from mvsd.sample.metadata import SamplingMetadata
@@ -207,3 +208,21 @@ def test_forward_with_penalties_and_min_tokens(device, monkeypatch):
     assert not rep_.unexplained, rep_.unexplained[:5]
     # the processors changed something the sampler saw
     assert not np.array_equal(processed, verify_rows)
+
+
+def test_step_penalties_of_counts_that_do_not_match_the_rows(device):
+    """mvsd_apply_step_penalties reads its target rows inside the P - B it was given, whatever the
+    cumulative counts say: the rows that the neighbouring entries name stay as they are."""
+    rows, B, V = 6, 4, 64
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=device)
+    x = torch.ones(rows, V, device=device)
+    around = i32([5, 5, 5, 5, 1, 2, 5, 5, 5, 5])
+    target_rows, bonus_rows, cu = around[4:6], i32([0, 0, 0, 0]), i32([0, 0, 0, rows])
+    spec, off = i32([-1] * rows), i32([0, 0, 0, 0, 1])
+    tok, info = i32([7]), i32([1])
+    presence = torch.ones(B, device=device)
+    nat.check(nat.lib().mvsd_apply_step_penalties(
+        x.data_ptr(), V, rows, V, B, cu.data_ptr(), target_rows.data_ptr(), bonus_rows.data_ptr(),
+        spec.data_ptr(), off.data_ptr(), tok.data_ptr(), info.data_ptr(), presence.data_ptr(),
+        None, None, nat.stream_of(x.device)), "mvsd_apply_step_penalties")
+    assert (x[3:] == 1.0).all() and (x[1:3, 7] == 0.0).all()

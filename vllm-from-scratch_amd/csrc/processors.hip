@@ -38,8 +38,10 @@ __global__ __launch_bounds__(kProcThreads) void logits_processors_kernel(Process
   const int j = row - begin;  // position of the row in its request's draft block
   int64_t at = row;
   if (p.bonus_rows) {
-    // verify rows before compact row `row`: all rows before it but r bonus rows
-    at = row == p.cu[r] - 1 ? p.bonus_rows[r] : p.target_rows[row - r];
+    // verify rows before compact row `row`: all rows before it but r bonus rows (out of the P - B
+    // verify rows only where the counts do not match the rows)
+    const int v = row - r;
+    at = row == p.cu[r] - 1 || v < 0 || v >= p.P - p.B ? p.bonus_rows[r] : p.target_rows[v];
     at = min(max(at, (int64_t)0), (int64_t)p.P - 1);
   }
   float* x = p.logits + at * p.stride;
