@@ -409,14 +409,16 @@ int mvsd_spec_logprobs(int32_t* ids, float* lps, int32_t* ranks, const float* ta
 /* * width, or num_rows.  That function returns 0 where this path does not apply; the calls */
 /* then return MVSD_E_RANGE.  Rows are MVSD_F32 / MVSD_BF16 / MVSD_F16 (dtype, common to     */
 /* target and bonus), upcast exactly, at any element alignment; bonus_rows [batch_size]     */
-/* selects request q's bonus row (NULL: row q).  topk_scores_split reads int64 tokens and   */
+/* selects request q's bonus row (NULL: row q).  target and bonus have target_num_rows and   */
+/* bonus_num_rows rows; a row index outside them reads the nearest row.  topk_scores_split reads int64 tokens and   */
 /* writes int64 ids and ranks.                                                              */
 /* ------------------------------------------------------------------------------------ */
 int64_t mvsd_logprobs_workspace_bytes(int64_t positions, int64_t vocab_size, int64_t k);
 
 int mvsd_spec_logprobs_split(int32_t* ids, float* lps, int32_t* ranks, const void* target,
-                             int dtype, int64_t target_stride, const int32_t* target_rows,
-                             const void* bonus, int64_t bonus_stride, const int32_t* bonus_rows,
+                             int dtype, int64_t target_stride, int64_t target_num_rows,
+                             const int32_t* target_rows, const void* bonus, int64_t bonus_stride,
+                             int64_t bonus_num_rows, const int32_t* bonus_rows,
                              const int32_t* cu_num_sampled_tokens,
                              const int32_t* sampled_token_ids, int64_t sampled_stride,
                              int64_t batch_size, int64_t num_tokens, int64_t vocab_size,

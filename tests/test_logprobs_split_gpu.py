@@ -138,3 +138,19 @@ def test_bound_of_64_or_256_unions(device, V, k):
     x[3] = x[3].round()
     check(x, k, torch.arange(5, device=device) * 5 % V)
     check(x, k, torch.arange(5, device=device) * 5 % V, logits_mode=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_row_indices_outside_the_logits_read_the_nearest_row(device, dtype):
+    V = 4100
+    meta = make_metadata([[1, 2], [], [3]], device=device)
+    logits = (torch.randn(6, V, device=device) * 2.5).to(dtype)
+    sampled = torch.tensor([[5, 6, 7], [8, -1, -1], [9, 10, -1]], dtype=torch.int32, device=device)
+    sampler = rs.RejectionSampler(Sampler())
+    tables = []
+    for target, bonus in (([0, 1, 4], [0, 3, 5]), ([-1, 1, 4], [-2 ** 31, 3, 2 ** 31 - 1])):
+        meta.target_logits_indices = torch.tensor(target, dtype=torch.int32, device=device)
+        meta.bonus_logits_indices = torch.tensor(bonus, dtype=torch.int32, device=device)
+        tables.append(sampler._get_logprobs_tensors(4, meta, logits, None, None, sampled))
+    for want, got in zip(*(t[:3] for t in tables)):
+        assert torch.equal(want, got)

@@ -600,8 +600,9 @@ int64_t mvsd_logprobs_workspace_bytes(int64_t positions, int64_t vocab_size, int
 }
 
 int mvsd_spec_logprobs_split(int32_t* ids, float* lps, int32_t* ranks, const void* target,
-                             int dtype, int64_t target_stride, const int32_t* target_rows,
-                             const void* bonus, int64_t bonus_stride, const int32_t* bonus_rows,
+                             int dtype, int64_t target_stride, int64_t target_num_rows,
+                             const int32_t* target_rows, const void* bonus, int64_t bonus_stride,
+                             int64_t bonus_num_rows, const int32_t* bonus_rows,
                              const int32_t* cu_num_sampled_tokens,
                              const int32_t* sampled_token_ids, int64_t sampled_stride,
                              int64_t batch_size, int64_t num_tokens, int64_t vocab_size,
@@ -616,8 +617,10 @@ int mvsd_spec_logprobs_split(int32_t* ids, float* lps, int32_t* ranks, const voi
   if (dtype != MVSD_F32 && dtype != MVSD_BF16 && dtype != MVSD_F16) return MVSD_E_INVALID;
   if (!ids || !lps || !ranks || !bonus || !cu_num_sampled_tokens || !sampled_token_ids)
     return MVSD_E_INVALID;
-  if (num_tokens > 0 && (!target || target_stride < vocab_size)) return MVSD_E_INVALID;
-  if (bonus_stride < vocab_size || sampled_stride < width) return MVSD_E_INVALID;
+  if (num_tokens > 0 && (!target || target_stride < vocab_size || target_num_rows < 1))
+    return MVSD_E_INVALID;
+  if (bonus_stride < vocab_size || bonus_num_rows < 1 || sampled_stride < width)
+    return MVSD_E_INVALID;
   const int64_t need =
       mvsd::split_logprobs_workspace_bytes(batch_size * width, vocab_size, k);
   if (need == 0) return MVSD_E_RANGE;
@@ -626,9 +629,11 @@ int mvsd_spec_logprobs_split(int32_t* ids, float* lps, int32_t* ranks, const voi
   mvsd::LogprobParams p{};
   p.target = target;
   p.tstride = target_stride;
+  p.target_num_rows = target_num_rows;
   p.target_rows = target_rows;
   p.bonus = bonus;
   p.bstride = bonus_stride;
+  p.bonus_num_rows = bonus_num_rows;
   p.bonus_rows = bonus_rows;
   p.cu_sampled = cu_num_sampled_tokens;
   p.tokens = sampled_token_ids;

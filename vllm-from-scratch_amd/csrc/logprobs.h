@@ -9,9 +9,11 @@ namespace mvsd {
 struct LogprobParams {
   const void* target;          // verify rows, row stride tstride (elements)
   int64_t tstride;
+  int64_t target_num_rows;     // rows of `target` that a row index is clamped to, or 0 (any)
   const int32_t* target_rows;  // [P] row of verify row v in `target`, or null (row v)
   const void* bonus;           // bonus rows, row stride bstride
   int64_t bstride;
+  int64_t bonus_num_rows;      // as target_num_rows
   const int32_t* bonus_rows;   // [B] row of request q's bonus row in `bonus`, or null (row q)
   const int32_t* cu_sampled;   // [B] cumulative K_r + 1, no leading 0
   const void* tokens;          // [B, W] sampled ids (int32, or int64 with tokens64), -1 padded

@@ -46,6 +46,10 @@ __device__ inline int64_t token_at(const LogprobParams& p, int64_t i) {
                     : (int64_t) static_cast<const int32_t*>(p.tokens)[i];
 }
 
+__device__ inline int64_t row_inside(int64_t row, int64_t num_rows) {
+  return num_rows > 0 ? min(max(row, (int64_t)0), num_rows - 1) : row;
+}
+
 template <typename S>
 __device__ inline Position<S> position(const LogprobParams& p, int n) {
   Position<S> at;
@@ -80,12 +84,15 @@ __device__ inline Position<S> position(const LogprobParams& p, int n) {
     }
     const int qstart = q == 0 ? 0 : p.cu_sampled[q - 1];
     const int kq = p.cu_sampled[q] - qstart - 1;  // verify rows of request q
-    if (c - qstart < kq) {
-      const int vrow = c - q;  // verify rows before c: c minus the bonus rows of requests < q
-      const int64_t trow = p.target_rows ? p.target_rows[vrow] : vrow;
+    if (c - qstart < kq && p.P > 0) {
+      // verify rows before c: c minus the bonus rows of requests < q (in bounds whatever
+      // cu_sampled holds)
+      const int vrow = min(max(c - q, 0), p.P - 1);
+      const int64_t trow =
+          row_inside(p.target_rows ? p.target_rows[vrow] : vrow, p.target_num_rows);
       at.row = static_cast<const S*>(p.target) + trow * p.tstride;
     } else {
-      const int64_t brow = p.bonus_rows ? p.bonus_rows[q] : q;
+      const int64_t brow = row_inside(p.bonus_rows ? p.bonus_rows[q] : q, p.bonus_num_rows);
       at.row = static_cast<const S*>(p.bonus) + brow * p.bstride;
     }
   }

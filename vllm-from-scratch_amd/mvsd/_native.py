@@ -156,9 +156,10 @@ SIGNATURES = {
                                         c_int64, c_void_p]),
     "mvsd_logprobs_workspace_bytes": (c_int64, [c_int64, c_int64, c_int64]),
     "mvsd_spec_logprobs_split": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int64,
-                                         c_void_p, c_void_p, c_int64, c_void_p, c_void_p,
-                                         c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64,
-                                         c_int64, c_int, c_void_p, c_int64, c_void_p]),
+                                         c_int64, c_void_p, c_void_p, c_int64, c_int64,
+                                         c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64,
+                                         c_int64, c_int64, c_int64, c_int, c_void_p, c_int64,
+                                         c_void_p]),
     "mvsd_topk_scores_split": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int64,
                                        c_void_p, c_int64, c_int64, c_int64, c_int, c_void_p,
                                        c_int64, c_void_p]),

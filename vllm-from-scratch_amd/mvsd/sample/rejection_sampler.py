@@ -338,9 +338,10 @@ class RejectionSampler:
             nat.check(handle.mvsd_spec_logprobs_split(
                 ids.data_ptr(), lps.data_ptr(), ranks.data_ptr(),
                 target_logits.data_ptr() if num_tokens else None, nat.dtype_code(bonus.dtype),
-                target_logits.stride(0), nat.ptr(rows), bonus.data_ptr(), bonus.stride(0),
-                nat.ptr(bonus_rows), cu.data_ptr(), tokens.data_ptr(), tokens.stride(0), B,
-                num_tokens, V, W, max_num_logprobs, 1 if self.is_logits_logprobs_mode else 0,
+                target_logits.stride(0), target_logits.shape[0], nat.ptr(rows), bonus.data_ptr(),
+                bonus.stride(0), bonus.shape[0], nat.ptr(bonus_rows), cu.data_ptr(),
+                tokens.data_ptr(), tokens.stride(0), B, num_tokens, V, W, max_num_logprobs,
+                1 if self.is_logits_logprobs_mode else 0,
                 workspace.data_ptr(), ws_bytes, nat.stream_of(device)),
                 "mvsd_spec_logprobs_split")
             return LogprobsTensors(ids, lps, ranks)
