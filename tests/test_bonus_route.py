@@ -2,6 +2,7 @@
 
 from types import SimpleNamespace
 
+import pytest
 import torch
 
 from mvsd.sample.metadata import SamplingMetadata
@@ -29,3 +30,9 @@ def test_a_replaced_top_k_top_p_sampler_is_used():
     assert not race_only(own)
     assert not race_only(OwnSampler())
     assert not race_only(plain, min_p=torch.tensor([0.1, 0.0]))
+
+
+@pytest.mark.parametrize("shape", [(1,), (3,), (1, 1), (0,)])
+def test_gather_logprobs_takes_one_token_per_row(shape):
+    with pytest.raises(RuntimeError, match="shape"):
+        Sampler.gather_logprobs(torch.zeros(2, 16), 1, torch.zeros(shape, dtype=torch.int64))

@@ -164,6 +164,7 @@ def row_logprobs(rows: torch.Tensor, num_logprobs: int, token_ids: torch.Tensor,
     apply (above 128 logprobs)."""
     n, V = rows.shape
     device = rows.device
+    token_ids = token_ids.reshape(n)  # one per row, or an error here
     handle = nat.lib()
     size = handle.mvsd_logprobs_workspace_bytes(n, V, num_logprobs)
     if size <= 0:
