@@ -1,10 +1,12 @@
-"""The penalties' host summaries (csrc/hostops.c) against numpy's distinct values and counts."""
+"""The penalties' host side: the summaries (csrc/hostops.c) against numpy's distinct values and
+counts, and their upload."""
 
 import numpy as np
 import pytest
+import torch
 
 from mvsd import _hostops
-from mvsd.sample.rejection_sampler import _penalty_entries
+from mvsd.sample.rejection_sampler import _penalty_entries, _upload
 
 
 def check(prompts, outputs, specs):
@@ -52,3 +54,9 @@ def test_errors():
         _hostops.penalty_entries([[1, 2, 3]], [[4]], [[5]], room[:8])
     with pytest.raises(ValueError):
         _hostops.penalty_entries([], [], [[]] * 9, room[:4])
+
+
+def test_uploads_are_refused_in_a_capture(monkeypatch):
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    with pytest.raises(RuntimeError, match="capture"):
+        _upload([np.zeros(3, np.int32)], torch.device("cpu"))

@@ -495,7 +495,11 @@ def _expand_opt(values: torch.Tensor | None, cu: torch.Tensor, num_rows: int):
 
 def _upload(arrays, device) -> list[torch.Tensor]:
     """int32 device copies of host arrays, through one pinned buffer and one copy that the host
-    does not wait for."""
+    does not wait for.  Refused in a graph capture: a replay would read the pinned buffer again,
+    which by then holds another call's arrays."""
+    if torch.cuda.is_current_stream_capturing():
+        raise RuntimeError("penalties and min_tokens upload host lists, which a graph capture "
+                           "cannot record: apply them outside the graph")
     arrays = [np.asarray(a, dtype=np.int32) for a in arrays]
     host = torch.empty(sum(a.size for a in arrays), dtype=torch.int32, pin_memory=True)
     np.concatenate(arrays, out=host.numpy())
