@@ -6,8 +6,10 @@ import pytest
 import torch
 
 from mvsd.sample import rejection_sampler as rs
+from mvsd.sample import sampler as smp
 from mvsd.sample.sampler import Sampler
 from mvsd.testing.spec_metadata import make_metadata, sampling_metadata
+from mvsd.worker.gpu.sample.logprob import compute_topk_scores
 
 pytestmark = pytest.mark.gpu
 
@@ -112,3 +114,40 @@ def test_forward_with_penalties(device, dtype, limits, V, B, greedy):
         outs.append(rs.RejectionSampler(cls()).forward(meta, probs, logits, sm))
     same(*outs, LP_ATOL)
     assert torch.equal(logits, before)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("limits", ["", "kp"])
+@pytest.mark.parametrize("overlap", ["one row", "shifted"])
+def test_overlapping_rows(device, dtype, limits, overlap):
+    """Rows nearer than a row's length (an expanded row, a sliding view) are copied, not refused."""
+    n, V = 5, 1000
+    base = (torch.randn(2 * V, device=device) * 2.5).to(dtype)
+    logits = (base[:V].expand(n, V) if overlap == "one row" else base.as_strided((n, V), (3, 1)))
+    temps, top_k, top_p = params(n, V, limits, 1, None)
+    sm = sampling_metadata(temps, [[]] * n, device=device, top_k=top_k, top_p=top_p,
+                           max_num_logprobs=4)
+    outs = []
+    for rows in (logits, logits.clone(memory_format=torch.contiguous_format)):
+        torch.manual_seed(3)
+        outs.append(Sampler().forward(rows, sm))
+    same(*outs, LP_ATOL)
+    if dtype != torch.float32:
+        tokens = torch.arange(n, device=device)
+        got, want = (compute_topk_scores(rows, 4, tokens) for rows in (logits, logits.float()))
+        assert torch.equal(got.logprob_token_ids, want.logprob_token_ids)
+        assert torch.equal(got.selected_token_ranks, want.selected_token_ranks)
+        assert (got.logprobs - want.logprobs).abs().max() <= LP_ATOL
+
+
+def test_noise_of_any_layout(device, monkeypatch):
+    """A replaced noise function may return any strides, as random_sample takes them."""
+    n, V = 4, 1000
+    logits = (torch.randn(n, V, device=device) * 2.5).to(torch.bfloat16)
+    sm = sampling_metadata([1.0] * n, [[]] * n, device=device, top_k=[7] * n)
+    noise = torch.empty(V, n, device=device).exponential_()
+    outs = []
+    for given in (noise.t(), noise.t().contiguous()):
+        monkeypatch.setattr(smp, "generate_sampler_noise", lambda *args: given)
+        outs.append(Sampler().forward(logits, sm))
+    same(*outs, 0.0)

@@ -316,7 +316,7 @@ class RejectionSampler:
             bonus = bonus_logits.to(torch.float32)
         in_place = (ws_bytes > 0 and target_logits is bonus
                     and bonus.dtype in (torch.float32, torch.bfloat16, torch.float16)
-                    and bonus.stride(-1) == 1)
+                    and bonus.stride(-1) == 1 and bonus.stride(0) >= V)
         if not in_place:
             if target_logits.dtype != torch.float32 or target_logits.stride(-1) != 1:
                 target_logits = (target_logits if rows is None

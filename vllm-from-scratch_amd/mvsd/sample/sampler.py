@@ -108,7 +108,9 @@ def race_rows(logits: torch.Tensor, row_index: torch.Tensor | None,
     V = logits.shape[1]
     if noise is not None:
         noise = noise.to(device=device, dtype=torch.float32)
-        assert noise.shape == (n, V) and noise.stride(1) == 1
+        assert noise.shape == (n, V)
+        if noise.stride(1) != 1 or noise.stride(0) < V:
+            noise = noise.contiguous()
     if temperature is not None:
         temperature = temperature.to(device=device, dtype=torch.float32).contiguous()
     ids = torch.empty(n, dtype=torch.int32, device=device)
@@ -250,7 +252,7 @@ class Sampler:
                 and (sm.all_greedy or sm.temperature is not None)
                 and logits.is_cuda and logits.ndim == 2 and logits.shape[0] > 0
                 and logits.dtype in (torch.float32, torch.bfloat16, torch.float16)
-                and logits.stride(1) == 1
+                and logits.stride(1) == 1 and logits.stride(0) >= logits.shape[1]
                 and (sm.all_greedy or (sm.top_k is None and sm.top_p is None)
                      or logits.dtype != torch.float32 or not logits.is_contiguous())
                 and (sm.max_num_logprobs is None

@@ -52,7 +52,8 @@ def compute_topk_scores(
         raise ValueError(f"{tokens.numel()} sampled tokens for {num_rows} logits rows")
     handle = lib()
     ws_bytes = handle.mvsd_logprobs_workspace_bytes(num_rows, vocab_size, num_logprobs)
-    if ws_bytes > 0 and logits.dtype in _ROW_DTYPES and logits.stride(-1) == 1:
+    if (ws_bytes > 0 and logits.dtype in _ROW_DTYPES and logits.stride(-1) == 1
+            and logits.stride(0) >= vocab_size):
         tokens = tokens.to(torch.int64).contiguous()
         ids = torch.empty(num_rows, num_logprobs + 1, dtype=torch.int64, device=device)
         scores = torch.empty(num_rows, num_logprobs + 1, dtype=torch.float32, device=device)
