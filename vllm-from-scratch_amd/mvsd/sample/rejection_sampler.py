@@ -93,7 +93,7 @@ class RejectionSampler:
                 logits: torch.Tensor, sampling_metadata: SamplingMetadata):
         """``logits`` is the compact ``[P + B, V]`` tensor in metadata row order (:153-225)."""
         from ..outputs import SamplerOutput
-        from .sampler import Sampler as DeviceSampler
+        from .sampler import runs_own_steps
 
         assert metadata.max_spec_len <= MAX_SPEC_LEN
         if len(sampling_metadata.prompt_token_ids) != len(metadata.num_draft_tokens):
@@ -120,7 +120,7 @@ class RejectionSampler:
         # only hand back as an fp32 copy
         bonus_rows_in_place = (max_num_logprobs is not None
                                and not self.is_processed_logprobs_mode
-                               and type(self.sampler) is DeviceSampler)
+                               and runs_own_steps(self.sampler))
         bonus_out = self.sampler.forward(
             bonus_logits, replace(sampling_metadata, max_num_logprobs=(
                 -1 if max_num_logprobs is not None and not bonus_rows_in_place else None)),
@@ -180,27 +180,38 @@ class RejectionSampler:
 
     def _bonus_rows_race_only(self, metadata: "SpecDecodeMetadata", sm: SamplingMetadata,
                               logits: torch.Tensor) -> bool:
-        """True when the caller's sampler is mvsd.sample.Sampler itself (with its own top-k /
-        top-p sampler) and, for this batch, it would only take each bonus row's argmax or
-        exponential race under its penalties and top-k / top-p: no active min_tokens, no min_p,
-        and no logprobs but raw ones; with penalties, compact rows of this batch alone and every
-        request's drafts in the sampling metadata; and the recovered-token seam is the module's
-        own."""
+        """True when the caller's sampler is mvsd.sample.Sampler itself and, for this batch, it
+        would only take each bonus row's argmax or exponential race under its penalties and top-k /
+        top-p: no active min_tokens, no min_p, and no logprobs but raw ones; with penalties,
+        compact rows of this batch alone and every request's drafts in the sampling metadata; and
+        the recovered-token seam is the module's own.  The steps that a batch with penalties,
+        limits or logprobs would go through are then the modules' own too (none overridden by a
+        subclass or replaced), since this route takes their place."""
         from .sampler import Sampler as DeviceSampler
-        from .sampler import TopKTopPSampler
+        from .sampler import TopKTopPSampler, runs_own_steps
 
-        return (type(self.sampler) is DeviceSampler
+        if not (type(self.sampler) is DeviceSampler
                 and type(self.sampler.topk_topp_sampler) is TopKTopPSampler
                 and not self.is_processed_logprobs_mode
+                and (sm.all_greedy or sm.temperature is not None)
                 and not _has_active_min_tokens(sm) and sm.min_p is None
                 and sample_recovered_tokens is _SAMPLE_RECOVERED_TOKENS
-                and (sm.all_greedy or sm.temperature is not None)
                 and logits.dtype in (torch.float32, torch.bfloat16, torch.float16)
-                and logits.stride(1) == 1
-                and (sm.no_penalties
-                     or (logits.shape[0] == sum(metadata.num_draft_tokens) + len(
-                         metadata.num_draft_tokens)
-                         and list(map(len, sm.spec_token_ids)) == metadata.num_draft_tokens)))
+                and logits.stride(1) == 1):
+            return False
+        if (sm.max_num_logprobs is None and sm.no_penalties and sm.top_k is None
+                and sm.top_p is None):
+            return True
+        if not (runs_own_steps(self.sampler) and rejection_sample is _REJECTION_SAMPLE):
+            return False
+        if sm.no_penalties:
+            return True
+        counts = metadata.num_draft_tokens
+        return (getattr(self.apply_logits_processors, "__func__", None)
+                is _APPLY_LOGITS_PROCESSORS
+                and (apply_sampling_constraints, apply_top_k_top_p) == _CONSTRAINT_FUNCTIONS
+                and logits.shape[0] == sum(counts) + len(counts)
+                and list(map(len, sm.spec_token_ids)) == counts)
 
     def _forward_race_only(self, metadata: "SpecDecodeMetadata",
                            draft_probs: torch.Tensor | None, logits: torch.Tensor,
@@ -244,14 +255,16 @@ class RejectionSampler:
                            if masks is None else masks[num_tokens:])
         bonus = smp.race_rows(logits, metadata.bonus_logits_indices, bonus_noise,
                               None if all_greedy else sm.temperature, masks=bonus_masks)
-        output_token_ids = _rejection_sample(
+        sample = (rejection_sample if masks is None
+                  else functools.partial(_rejection_sample, row_masks=masks))
+        output_token_ids = sample(
             metadata.draft_token_ids, metadata.num_draft_tokens, metadata.max_spec_len,
             metadata.cu_num_draft_tokens, draft_probs, logits, bonus.view(B, 1), sm,
             synthetic_mode=self.synthetic_mode,
             synthetic_conditional_rates=self.synthetic_conditional_rates,
             uniform_probs=uniforms, exp_noise=exp_noise,
             target_rows=metadata.target_logits_indices, apply_temperature=True,
-            apply_top_k_top_p=constrained, row_masks=masks)
+            apply_top_k_top_p=constrained)
         logprobs_tensors = None
         if sm.max_num_logprobs is not None:
             logprobs_tensors = self._get_logprobs_tensors(
@@ -980,6 +993,10 @@ def sample_recovered_tokens(
 
 
 _SAMPLE_RECOVERED_TOKENS = sample_recovered_tokens
+# and the steps that RejectionSampler._forward_race_only takes the place of
+_REJECTION_SAMPLE = rejection_sample
+_APPLY_LOGITS_PROCESSORS = RejectionSampler.apply_logits_processors
+_CONSTRAINT_FUNCTIONS = (apply_sampling_constraints, apply_top_k_top_p)
 
 
 # --------------------------------------------------------------------------- helpers

@@ -244,9 +244,7 @@ class Sampler:
         copied before that, so there it does not show.)"""
         from .rejection_sampler import _has_active_min_tokens
 
-        return (type(self) is Sampler and type(self.topk_topp_sampler) is TopKTopPSampler
-                and self.topk_topp_sampler.logprobs_mode not in _PROCESSED_MODES
-                and logprobs_mode in ("raw_logprobs", "raw_logits")
+        return (runs_own_steps(self) and logprobs_mode in ("raw_logprobs", "raw_logits")
                 and sm.no_penalties and not _has_active_min_tokens(sm) and sm.min_p is None
                 and (sm.max_num_logprobs is None or sm.max_num_logprobs >= 0)
                 and (sm.all_greedy or sm.temperature is not None)
@@ -439,3 +437,26 @@ class Sampler:
             x.stride(0), cu.data_ptr(), tokens.data_ptr(), 1, n, 0, V, 1, num_logprobs, 1,
             nat.stream_of(device)), "mvsd_spec_logprobs")
         return LogprobsTensors(ids, lps, ranks)
+
+
+# The steps that Sampler.forward takes one after another, and the functions that they call.
+_STEPS = {name: Sampler.__dict__[name] for name in (
+    "forward", "apply_logits_processors", "apply_penalties", "_combine_outputs_with_spec_tokens",
+    "apply_min_tokens", "sample", "apply_min_p", "greedy_sample", "compute_logprobs",
+    "gather_logprobs")}
+_TOP_K_TOP_P_CALL = TopKTopPSampler.__call__
+_STEP_FUNCTIONS = (apply_top_k_top_p, random_sample)
+
+
+def runs_own_steps(sampler) -> bool:
+    """True when ``sampler`` is a Sampler whose steps are all this module's own, so that a shorter
+    route may take their place: none overridden by a subclass, set on the object or on the class,
+    or replaced in the module, and no processed rows kept by its top-k / top-p sampler."""
+    if type(sampler) is not Sampler:
+        return False
+    limits = sampler.topk_topp_sampler
+    return (type(limits) is TopKTopPSampler and limits.logprobs_mode not in _PROCESSED_MODES
+            and _STEPS.keys().isdisjoint(vars(sampler))
+            and all(Sampler.__dict__.get(name) is step for name, step in _STEPS.items())
+            and TopKTopPSampler.__call__ is _TOP_K_TOP_P_CALL
+            and (apply_top_k_top_p, random_sample) == _STEP_FUNCTIONS)
