@@ -93,6 +93,18 @@ def test_replaced_processors_are_used(monkeypatch):
     assert race_only(Sampler(), PENALTIES)
 
 
+@pytest.mark.parametrize("specs", [None, []])
+def test_penalties_without_draft_lists(specs):
+    assert not race_only(Sampler(), {**PENALTIES, "spec_token_ids": specs})
+
+
+@pytest.mark.parametrize("counts", [np.array([1, 2]), [np.int64(1), 2], (1, 2)])
+def test_draft_counts_of_any_integer_type(counts):
+    assert race_only(Sampler(), PENALTIES, counts=counts)
+    assert not race_only(Sampler(), {**PENALTIES, "spec_token_ids": [[3], [4]]}, counts=counts)
+    assert not race_only(Sampler(), {**PENALTIES, "spec_token_ids": [[3]]}, counts=counts)
+
+
 @pytest.mark.parametrize("shape", [(1,), (3,), (1, 1), (0,)])
 def test_gather_logprobs_takes_one_token_per_row(shape):
     with pytest.raises(RuntimeError, match="shape"):

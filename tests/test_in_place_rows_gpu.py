@@ -2,6 +2,7 @@
 rows' logprobs) against the general path, which writes the rows' fp32 copy, its quotient by the
 temperature and its masked entries: the same RNG state gives the same tokens, ids and ranks."""
 
+import numpy as np
 import pytest
 import torch
 
@@ -150,4 +151,23 @@ def test_noise_of_any_layout(device, monkeypatch):
     for given in (noise.t(), noise.t().contiguous()):
         monkeypatch.setattr(smp, "generate_sampler_noise", lambda *args: given)
         outs.append(Sampler().forward(logits, sm))
+    same(*outs, 0.0)
+
+
+@pytest.mark.parametrize("form", ["no draft lists", "array of counts"])
+def test_forward_with_penalties_in_other_forms(device, form):
+    V, drafts = 500, [[3, 4], [], [5]]
+    meta = make_metadata(drafts, device=device)
+    logits = torch.randn(6, V, device=device) * 2.5
+    sm = sampling_metadata([1.0, 0.0, 0.7], drafts, device=device, no_penalties=False,
+                           prompt_token_ids=[[1, 2]] * 3, output_token_ids=[[3], [4, 4], []],
+                           presence_penalties=[0.5] * 3)
+    if form == "no draft lists":
+        sm.spec_token_ids = None
+    else:
+        meta.num_draft_tokens = np.array(meta.num_draft_tokens)
+    outs = []
+    for cls in (Sampler, General):
+        torch.manual_seed(11)
+        outs.append(rs.RejectionSampler(cls()).forward(meta, None, logits, sm))
     same(*outs, 0.0)

@@ -206,12 +206,12 @@ class RejectionSampler:
             return False
         if sm.no_penalties:
             return True
-        counts = metadata.num_draft_tokens
+        counts = [int(k) for k in metadata.num_draft_tokens]
         return (getattr(self.apply_logits_processors, "__func__", None)
                 is _APPLY_LOGITS_PROCESSORS
                 and (apply_sampling_constraints, apply_top_k_top_p) == _CONSTRAINT_FUNCTIONS
                 and logits.shape[0] == sum(counts) + len(counts)
-                and list(map(len, sm.spec_token_ids)) == counts)
+                and bool(sm.spec_token_ids) and [len(s) for s in sm.spec_token_ids] == counts)
 
     def _forward_race_only(self, metadata: "SpecDecodeMetadata",
                            draft_probs: torch.Tensor | None, logits: torch.Tensor,
