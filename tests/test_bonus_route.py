@@ -93,6 +93,12 @@ def test_replaced_processors_are_used(monkeypatch):
     assert race_only(Sampler(), PENALTIES)
 
 
+def test_batches_without_limits_race_whatever_the_logprobs_mode():
+    assert race_only(with_own_limits(), {})
+    assert race_only(Sampler("processed_logprobs"), {})
+    assert not race_only(Sampler("processed_logprobs"), LIMITS)
+
+
 @pytest.mark.parametrize("specs", [None, []])
 def test_penalties_without_draft_lists(specs):
     assert not race_only(Sampler(), {**PENALTIES, "spec_token_ids": specs})

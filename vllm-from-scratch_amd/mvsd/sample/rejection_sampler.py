@@ -188,11 +188,9 @@ class RejectionSampler:
         limits or logprobs would go through are then the modules' own too (none overridden by a
         subclass or replaced), since this route takes their place."""
         from .sampler import Sampler as DeviceSampler
-        from .sampler import TopKTopPSampler, runs_own_steps
+        from .sampler import runs_own_steps
 
         if not (type(self.sampler) is DeviceSampler
-                and type(self.sampler.topk_topp_sampler) is TopKTopPSampler
-                and not self.is_processed_logprobs_mode
                 and (sm.all_greedy or sm.temperature is not None)
                 and not _has_active_min_tokens(sm) and sm.min_p is None
                 and sample_recovered_tokens is _SAMPLE_RECOVERED_TOKENS
@@ -202,7 +200,8 @@ class RejectionSampler:
         if (sm.max_num_logprobs is None and sm.no_penalties and sm.top_k is None
                 and sm.top_p is None):
             return True
-        if not (runs_own_steps(self.sampler) and rejection_sample is _REJECTION_SAMPLE):
+        if not (runs_own_steps(self.sampler) and rejection_sample is _REJECTION_SAMPLE
+                and not self.is_processed_logprobs_mode):
             return False
         if sm.no_penalties:
             return True
