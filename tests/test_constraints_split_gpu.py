@@ -100,6 +100,30 @@ def test_apply_in_place_equals_general_path(device, n, V):
     assert torch.equal(wide, want)
 
 
+@pytest.mark.parametrize("ties", [2, 300, 100000, 150000])
+def test_greedy_ties_at_the_limit(device, ties):
+    """Greedy rows of tied maxima whose mass below is within 3e-4 of what 1 - p takes: the first
+    maximum is kept or masked as the exact sums say, also where a float sum of the ties (a multiple
+    of 1/64 at 150000) is off by more."""
+    V, n = 151936, 128
+    # t (ties + below) = below + 1 + e, t = 1 - p a multiple of 2^-24
+    t = (torch.linspace(1.2, 1.9 if ties == 2 else 4.0, n, dtype=torch.float64) / ties * 2 ** 24
+         ).round() / 2 ** 24
+    e = 3e-4 * (1 - 2 * (torch.arange(n) % 2))
+    below = (t * ties - 1 - e) / (1 - t)
+    x = torch.full((n, V), -math.inf, device=device)
+    x[:, 500:500 + ties] = 0.0
+    x[:, :20] = (below / 20).log().float().to(device)[:, None]
+    cu = torch.arange(1, n + 1, dtype=torch.int32, device=device)
+    rows = torch.arange(n, dtype=torch.int32, device=device)
+    sm = SamplingMetadata(temperature=torch.zeros(n, device=device), all_greedy=False,
+                          all_random=False, top_k=None, top_p=(1 - t).float().to(device))
+    want = general_masks(x, cu, rows, sm)
+    assert torch.equal((want[:, 0] > -math.inf).cpu(), e > 0)
+    got = sampling_masks(x, cu, sm, target_rows=rows)
+    assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+
+
 def test_decreasing_counts_stay_inside_the_scratch(device):
     """Cumulative draft counts that decrease list rows more than once: the plan keeps to its
     room.  (The masks of such a batch mean nothing; the call reads and writes in bounds.)"""

@@ -1352,14 +1352,16 @@ __global__ __launch_bounds__(kCT) void split_pick_kernel(SplitParams sp) {
     }
     if (k == 0) {
       // The first maximum stays when the mass up to and including it passes the limit
-      // (split_finish decides that exactly).  The float sums settle it for most rows: they are
-      // within 1e-5, and the fixed-point masses lose less than 2^-40 each.
+      // (split_finish decides that exactly).  The float sums settle it for most rows.  A sum of
+      // positive terms is off by at most 1e-5 of itself (about 60 roundings of 2^-24 in a row,
+      // and those of the exponents), so `below`, the sum less the ties, by 1e-5 of the sum: much of
+      // it where nearly all of the mass is ties.  The fixed-point masses lose below 2^-40 each.
       float sum[1] = {tid < nch && cm > -INFINITY
                           ? sp.csum[slot0 + tid] * __builtin_amdgcn_exp2f((cm - M) * kLog2e)
                           : 0.f};
       block_sum<1, kCW>(sum, reinterpret_cast<float*>(sm.c.part));
-      const float below = sum[0] - (float)ties;
-      if (t * sum[0] * 1.001f < fmaxf(below, 0.f) * 0.999f + 0.999f) {
+      const float below = fmaxf(sum[0] - (float)ties - 1e-5f * sum[0], 0.f);
+      if (t * sum[0] * 1.001f < below * 0.999f + 0.999f) {
         done(-INFINITY, -INFINITY, -1);
         return;
       }
