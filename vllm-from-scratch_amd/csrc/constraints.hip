@@ -1245,7 +1245,7 @@ __global__ __launch_bounds__(kSplitThreads) void split_scan_kernel(SplitParams s
           for (int e = 0; e < VEC; ++e) {
             const float w = __builtin_amdgcn_exp2f((ch.v[j][e] - M) * c1);
             const float b = fminf(base - floorf(ch.v[j][e] * per), (float)(kSplitBins - 1));
-            const uint32_t mass = (uint32_t)(w * 0x1p31f);
+            const uint32_t mass = (uint32_t)fmaxf(w * 0x1p31f, 0.f);  // 0 for a NaN entry
             if (mass)
               atomicAdd(&s_hist[(int)b * kSplitCopies + (tid & (kSplitCopies - 1))],
                         (unsigned long long)mass);
@@ -1546,7 +1546,7 @@ __global__ __launch_bounds__(kSplitThreads) void split_mass_kernel(SplitParams s
     const float x_lo = d.x_lo, x_hi = d.x_hi, vmax = d.vmax;
     const S* x = static_cast<const S*>(sp.p.target) + d.xrow * sp.p.target_stride;
     SplitChunk<DT, NV> ch;
-    // a column past the row holds NaN: its mass converts to 0, and it is in no interval
+    // a column past the row holds NaN: its mass is 0, and it is in no interval
     ch.load(x, c, sp.p.V, NAN);
     int n = 0;  // candidates of this lane
 #pragma unroll
@@ -1586,7 +1586,7 @@ __global__ __launch_bounds__(kSplitThreads) void split_mass_kernel(SplitParams s
       if (__ballot(!(top < 0x1p32f)) == 0) {
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
-          const uint32_t m = (uint32_t)e40[e];
+          const uint32_t m = (uint32_t)fmaxf(e40[e], 0.f);  // 0 for NaN
           total += m;
           below += ch.v[j][e] < x_lo ? m : 0u;
         }
