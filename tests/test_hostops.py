@@ -1,6 +1,9 @@
 """The penalties' host side: the summaries (csrc/hostops.c) against numpy's distinct values and
 counts, and their upload."""
 
+import math
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -40,6 +43,30 @@ def test_forms_of_input():
     check([[2 ** 31 - 1, -1, -2 ** 31]], [[2 ** 31 - 1]], [[]])
     off, tok, info = _penalty_entries([[1.0, 2.0]], [[2.0]], [[3]])  # as np.asarray reads them
     assert sorted(zip(tok.tolist(), info.tolist())) == [(1, -2 ** 31), (2, 1 - 2 ** 31), (3, 0)]
+
+
+@pytest.mark.parametrize("order", [1, -1])
+def test_long_and_short_histories(order):
+    """Each request's table has its own size, whatever came before it."""
+    rng = np.random.default_rng(3)
+    prompts = [rng.integers(0, 1500, n).tolist() for n in (5000, 900, 40, 3, 0)][::order]
+    check(prompts, [p[:50] for p in prompts], [[7, 8]] * 5)
+
+
+def test_a_long_history_costs_no_more_first_than_last():
+    rng = np.random.default_rng(4)
+    short = [rng.integers(0, 150000, 20).tolist() for _ in range(2000)]
+    long = [rng.integers(0, 150000, 200000).tolist()]
+
+    def seconds(prompts):
+        best = math.inf
+        for _ in range(3):
+            start = time.perf_counter()
+            _penalty_entries(prompts, [[]] * 2001, [[]] * 2001)
+            best = min(best, time.perf_counter() - start)
+        return best
+
+    assert seconds(long + short) < 3 * seconds(short + long)
 
 
 def test_errors():

@@ -10,7 +10,8 @@
 // One request's distinct tokens: an open-addressing table of places in the entry arrays.
 typedef struct {
   int32_t* slot;    // place + 1, 0 = free
-  size_t cap;       // power of two
+  size_t cap;       // slots in use for this request, a power of two
+  size_t room;      // slots allocated
 } Table;
 
 static uint64_t mix(uint64_t x) {
@@ -47,7 +48,7 @@ static PyObject* penalty_entries(PyObject* self, PyObject* args) {
   PyObject* result = NULL;
   int64_t* keys = NULL;
   int32_t* info = NULL;
-  Table tb = {NULL, 0};
+  Table tb = {NULL, 0, 0};
   size_t keys_cap = 0;
   for (int s = 0; s < 3; ++s) {
     outer[s] = PySequence_Fast(lists[s], "a sequence of token sequences is expected");
@@ -89,10 +90,11 @@ static PyObject* penalty_entries(PyObject* self, PyObject* args) {
       }
       size_t cap = 16;
       while (cap < 2 * all) cap *= 2;
-      if (ok && cap > tb.cap) {
+      tb.cap = cap;  // its own size: a short history after a long one clears a small table
+      if (ok && cap > tb.room) {
         free(tb.slot);
         tb.slot = (int32_t*)malloc(cap * sizeof(int32_t));
-        tb.cap = tb.slot ? cap : 0;
+        tb.room = tb.slot ? cap : 0;
       }
       if (ok && all > keys_cap) {
         free(keys);
