@@ -3,6 +3,7 @@ counts, and their upload."""
 
 import math
 import time
+from collections import deque
 
 import numpy as np
 import pytest
@@ -43,6 +44,10 @@ def test_forms_of_input():
     check([[2 ** 31 - 1, -1, -2 ** 31]], [[2 ** 31 - 1]], [[]])
     off, tok, info = _penalty_entries([[1.0, 2.0]], [[2.0]], [[3]])  # as np.asarray reads them
     assert sorted(zip(tok.tolist(), info.tolist())) == [(1, -2 ** 31), (2, 1 - 2 ** 31), (3, 0)]
+
+
+def test_sequences_without_slices():
+    check(deque([[1, 2, 1], (3,)]), deque([[2]]), deque([[4], []]))
 
 
 @pytest.mark.parametrize("order", [1, -1])

@@ -39,6 +39,7 @@ from __future__ import annotations
 
 import functools
 from dataclasses import replace
+from itertools import islice
 from typing import TYPE_CHECKING
 
 import numpy as np
@@ -468,7 +469,7 @@ def _penalty_entries(prompts, outputs, specs):
     from .. import _hostops
 
     B = len(specs)
-    room = sum(sum(map(len, lists[:B])) for lists in (prompts, outputs, specs))
+    room = sum(sum(map(len, islice(lists, B))) for lists in (prompts, outputs, specs))
     buffer = np.empty(B + 1 + 2 * room, dtype=np.int32)
     try:
         n = _hostops.penalty_entries(prompts, outputs, specs, buffer)
