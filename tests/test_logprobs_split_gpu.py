@@ -9,6 +9,7 @@ import math
 import pytest
 import torch
 
+from mvsd import _native as nat
 from mvsd.sample import rejection_sampler as rs
 from mvsd.sample.sampler import Sampler
 from mvsd.testing.spec_metadata import make_metadata
@@ -154,3 +155,20 @@ def test_row_indices_outside_the_logits_read_the_nearest_row(device, dtype):
         tables.append(sampler._get_logprobs_tensors(4, meta, logits, None, None, sampled))
     for want, got in zip(*(t[:3] for t in tables)):
         assert torch.equal(want, got)
+
+
+@pytest.mark.parametrize("n,V,k,split", [
+    (3, 1024, 128, True), (3, 1025, 20, False), (257, 1025, 20, True),   # fewer groups than k
+    (5, 2048 * 6, 96, True), (5, 2048 * 6 - 1100, 96, False),             # as many, and one less
+    (15, 16384, 128, True), (16, 16384, 128, False), (16, 17000, 128, True),                        # a sixteenth more
+    (150, 50257, 128, True), (150, 50257, 20, True),                      # short, long chunks
+    (1, 33, 33, True)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_rows_of_few_groups(device, dtype, n, V, k, split):
+    """Where the groups of a row are few beside k: the lists kernel, shorter chunks, or the split
+    path's own lists, all the same answers."""
+    assert (nat.lib().mvsd_logprobs_workspace_bytes(n, V, k) > 0) == split
+    g = torch.Generator(device=device).manual_seed(V + k)
+    x = (torch.randn(n, V, device=device, generator=g) * 2.5).to(dtype)
+    check(x, k, torch.arange(n, device=device) * 7 % V)
+    check(x, k, torch.arange(n, device=device) * 7 % V, logits_mode=True)

@@ -14,7 +14,7 @@
 //   rank = #{i : lp(x_i) >= lp(x_token)}.
 //
 // Two paths, the same results:
-//   split     (a workspace, k <= 128): lp_scan_kernel reads each position's row once, split into
+//   split     (a workspace, k <= 128, rows long enough for k): lp_scan_kernel reads each position's row once, split into
 //             chunks over workgroups; lp_finish_kernel, one workgroup per position, combines the
 //             chunks and finds the top-k in the few places that can hold it.
 //   lists     (any k, no workspace): spec_logprobs_kernel, one 512-thread workgroup per position:
@@ -302,13 +302,36 @@ constexpr int kThetaWaveK = 32;       // largest k whose theta is read off 64 ke
 constexpr float kLpLog2e = 1.44269504088896340736f;
 
 // Columns per chunk: 8192, or 2048 where rows of 8192-column chunks would leave compute units
-// idle (fewer than 4 workgroups each) or give fewer groups than the largest k.
+// idle (fewer than 4 workgroups each) or give fewer than two groups per candidate wanted, so that
+// theta is a poor bound or none: 1000 fp32 rows of 32000 columns took 90 us with long chunks and 45
+// with short ones for k = 64 (64 long groups), 1488 and 53 for k = 128; of 65536 columns 70 and 62
+// for k = 64 (128 groups, where the two meet).
 constexpr int kChunkLong = 8192, kChunkShort = 2048;
 
-static int split_chunk(int64_t positions, int64_t V) {
+// Groups of a row that hold entries (16-bit rows can have a few less in their last chunk).
+static int64_t row_groups(int64_t V, int64_t chunk) {
+  const int64_t rest = (V % chunk + 63) / 64;
+  return V / chunk * kGroupsPerChunk + (rest < kGroupsPerChunk ? rest : kGroupsPerChunk);
+}
+
+static int split_chunk(int64_t positions, int64_t V, int64_t k) {
   const int64_t wgs = positions * ((V + kChunkLong - 1) / kChunkLong);
   const int64_t groups_short = (V + kChunkShort - 1) / kChunkShort * kGroupsPerChunk;
-  return wgs < 1024 && groups_short <= kMaxGroups ? kChunkShort : kChunkLong;
+  const bool want_short = wgs < 1024 || row_groups(V, kChunkLong) < 2 * k;
+  return want_short && groups_short <= kMaxGroups ? kChunkShort : kChunkLong;
+}
+
+// Rows too short to give theta (fewer groups than k, and more entries than the candidate buffer)
+// end in the lists, by 256 threads after the scan, where the lists kernel has 512 and no scan.  Up
+// to one workgroup per compute unit that kernel is the faster one, beyond it the slower (k = 128, V =
+// 8000: 181 us against 276 for 256 rows, 349 against 302 for 320; V = 4096: 143 / 164 and 279 / 196).
+// With as many groups as k = 128, theta is the least of the groups' maxima, which one row in 25 has
+// more than 1024 entries above (V = 16384: 258 us against 522 for 128 rows; below 16 rows most calls
+// meet none); a sixteenth more groups are enough (V = 17000: 261 against 37).
+constexpr int64_t kListPositions = 256, kFewPositions = 16;
+static bool lists_are_faster(int64_t positions, int64_t V, int64_t k) {
+  const int64_t need = k <= 96 || positions < kFewPositions ? k : k + k / 16;
+  return V > kLpCap && row_groups(V, kChunkShort) < need && positions <= kListPositions;
 }
 
 template <int DT, int NV>
@@ -642,8 +665,8 @@ hipError_t launch_spec_logprobs(const LogprobParams& p, hipStream_t stream) {
 }
 
 int64_t split_logprobs_workspace_bytes(int64_t positions, int64_t V, int64_t k) {
-  if (positions <= 0 || k > kSplitMaxK) return 0;
-  const int64_t chunk = split_chunk(positions, V);
+  if (positions <= 0 || k > kSplitMaxK || lists_are_faster(positions, V, k)) return 0;
+  const int64_t chunk = split_chunk(positions, V, k);
   const int64_t nch = (V + chunk - 1) / chunk;
   // a row's groups fit LDS; the scan's threads stay below 2^32
   if (nch * kGroupsPerChunk > kMaxGroups || positions * nch >= (1ll << 24)) return 0;
@@ -669,7 +692,7 @@ static void launch_split_dt(const LogprobParams& p, int chunk, hipStream_t strea
 hipError_t launch_split_logprobs(LogprobParams p, int dtype, void* workspace, hipStream_t stream) {
   const int64_t n = (int64_t)p.B * p.W;
   if (n <= 0) return hipSuccess;
-  const int chunk = split_chunk(n, p.V);
+  const int chunk = split_chunk(n, p.V, p.k);
   p.nchunks = (p.V + chunk - 1) / chunk;
   p.stats = static_cast<float4*>(workspace);
   p.group_keys = reinterpret_cast<uint32_t*>(p.stats + n * p.nchunks);
