@@ -46,19 +46,45 @@ def make_rows(V, dtype, device, g):
                         peak]).to(dtype)
 
 
+def kinds_of(V):
+    """(top-k or 0, top-p, temperature) of every class of row."""
+    return [(0, 0.9, 0.8), (0, 0.3, 1.5), (0, 0.999, 1.0), (0, 1e-6, 0.7), (0, 0.0, 1.0),
+            (1, 1.0, 0.8), (20, 1.0, 1.3), (50, 0.9, 0.8), (300, 0.5, 1.0), (600, 0.9, 1.0),
+            (V - 1, 0.8, 0.9), (0, 0.9, 0.0), (0, 0.2, 0.0), (5, 0.5, 0.0), (5, 1.0, 0.0),
+            (0, 1.0, 0.9), (0, 0.9, 1e-30), (3, 0.9, 1e25)]
+
+
+def long_chunks(rows, V):
+    """Whether a call takes 8192-column chunks (csrc/constraints.hip, split_chunk)."""
+    return rows * -(-V // 8192) >= 300 or -(-V // 2048) > 256
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("V", [65536, 65537, 73727, 151936, 524288])
 def test_masks_equal_general_path(device, dtype, V):
     g = torch.Generator(device=device).manual_seed(V)
     x = make_rows(V, dtype, device, g)
-    kinds = [(0, 0.9, 0.8), (0, 0.3, 1.5), (0, 0.999, 1.0), (0, 1e-6, 0.7), (0, 0.0, 1.0),
-             (1, 1.0, 0.8), (20, 1.0, 1.3), (50, 0.9, 0.8), (300, 0.5, 1.0), (600, 0.9, 1.0),
-             (V - 1, 0.8, 0.9), (0, 0.9, 0.0), (0, 0.2, 0.0), (5, 0.5, 0.0), (5, 1.0, 0.0),
-             (0, 1.0, 0.9), (0, 0.9, 1e-30), (3, 0.9, 1e25)]
+    kinds = kinds_of(V)
     n = x.shape[0]
     # every kind on every row, the rows in another order for each request
     for part in (kinds[:9], kinds[9:]):  # at most 128 rows a call
+        assert long_chunks(n * len(part), V)
         _compare(x, part, g)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("V", [65536, 65537, 73727, 151936, 524288])
+def test_masks_of_few_rows_equal_general_path(device, dtype, V):
+    """The same kinds and rows in calls small enough for the 2048-column chunks; 524288 columns
+    have the most chunks and groups of a row."""
+    g = torch.Generator(device=device).manual_seed(V + 1)
+    x = make_rows(V, dtype, device, g)
+    kinds, n = kinds_of(V), x.shape[0]
+    per_call = min(n, 299 // -(-V // 8192))  # rows
+    for i in range(0, n, per_call):
+        for kind in kinds:
+            assert not long_chunks(per_call, V)
+            _compare(x[i:i + per_call], [kind], g)
 
 
 def _compare(x, kinds, g):
