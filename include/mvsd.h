@@ -245,9 +245,9 @@ int mvsd_apply_top_k_top_p(float* logits, int64_t logits_stride, const int64_t* 
 /* constraints' rows split over workgroups: the same results, from scratch of               */
 /* mvsd_constraints_scratch_bytes(rows, V) bytes (rows = num_tokens or num_rows), 256-byte  */
 /* aligned, caller-owned, no initial contents needed.  That function returns 0 where the    */
-/* split path does not apply (above 128 rows): rejection_sample_split and                   */
-/* sampling_masks_split then (and with scratch or top_p NULL) take the other path,          */
-/* apply_top_k_top_p_split returns MVSD_E_RANGE.                                            */
+/* split path does not apply (above 128 rows, below 65536 columns or above 524288):          */
+/* rejection_sample_split and sampling_masks_split then (and with scratch or top_p NULL)     */
+/* take the other path, step_masks and apply_top_k_top_p_split return MVSD_E_RANGE.          */
 /* ------------------------------------------------------------------------------------ */
 int64_t mvsd_constraints_scratch_bytes(int64_t num_rows, int64_t vocab_size);
 
@@ -402,16 +402,18 @@ int mvsd_spec_logprobs(int32_t* ids, float* lps, int32_t* ranks, const float* ta
                        int64_t width, int64_t k, int logits_mode, mvsd_stream_t stream);
 
 /* ------------------------------------------------------------------------------------ */
-/* spec_logprobs_split / topk_scores_split — mvsd_spec_logprobs and mvsd_topk_scores with   */
-/* each row split over workgroups, for k <= 128.  The same results (the sum of exponentials */
-/* in another order) from a workspace of mvsd_logprobs_workspace_bytes(positions, V, k)     */
-/* bytes, 16-byte aligned, caller-owned, no initial contents needed; positions = batch_size */
-/* * width, or num_rows.  That function returns 0 where this path does not apply; the calls */
-/* then return MVSD_E_RANGE.  Rows are MVSD_F32 / MVSD_BF16 / MVSD_F16 (dtype, common to     */
-/* target and bonus), upcast exactly, at any element alignment; bonus_rows [batch_size]     */
-/* selects request q's bonus row (NULL: row q).  target and bonus have target_num_rows and   */
-/* bonus_num_rows rows; a row index outside them reads the nearest row.  topk_scores_split reads int64 tokens and   */
-/* writes int64 ids and ranks.                                                              */
+/* spec_logprobs_split / topk_scores_split — mvsd_spec_logprobs and mvsd_topk_scores with */
+/* each row split over workgroups, for k <= 128.  The same results (the sum of            */
+/* exponentials in another order) from a workspace of                                     */
+/* mvsd_logprobs_workspace_bytes(positions, V, k) bytes, 16-byte aligned, caller-owned,   */
+/* no initial contents needed; positions = batch_size * width, or num_rows.  That         */
+/* function returns 0 where this path does not apply (k above 128, above 2097152 columns, */
+/* up to 256 rows of fewer than about k groups of 128 columns); the calls then return     */
+/* MVSD_E_RANGE.  Rows are MVSD_F32 / MVSD_BF16 / MVSD_F16 (dtype, common to target and   */
+/* bonus), upcast exactly, at any element alignment; bonus_rows [batch_size] selects      */
+/* request q's bonus row (NULL: row q).  target and bonus have target_num_rows and        */
+/* bonus_num_rows rows; a row index outside them reads the nearest row.                   */
+/* topk_scores_split reads int64 tokens and writes int64 ids and ranks.                   */
 /* ------------------------------------------------------------------------------------ */
 int64_t mvsd_logprobs_workspace_bytes(int64_t positions, int64_t vocab_size, int64_t k);
 

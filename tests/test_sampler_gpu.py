@@ -17,6 +17,7 @@ import numpy as np
 import pytest
 import torch
 
+from mvsd import _native as nat
 from mvsd.sample import Sampler
 from mvsd.sample import rejection_sampler as rs
 from mvsd.sample import sampler as smp
@@ -356,3 +357,22 @@ def test_race_rows_in_place(device, dtype):
         assert got[r] == want or float(scores[got[r]]) >= float(scores[want]) * (1 - 1e-5), r
     greedy = smp.race_rows(table.to(device), idx.to(device), None, temps.to(device))
     assert greedy.cpu().tolist() == [int(torch.argmax(x[r])) for r in range(n)]
+
+
+@pytest.mark.parametrize("V", [1, 255, 257, 50257])
+def test_argmax_rows_of_the_c_entry_point(device, V):
+    """mvsd_sampler_rows op 0, which greedy_sample no longer calls: NaN first, then the largest
+    value, the lowest index on ties (+0 and -0 among them); rows of a wider tensor."""
+    wide = torch.randn(6, V + 3, device=device)
+    x = wide[:, 1:V + 1]
+    x[1], x[2] = 0.0, -math.inf
+    x[1, V // 3] = -0.0
+    x[3, V // 2:] = 7.0
+    x[4, [V // 4, V - 1]] = math.nan
+    ids = torch.empty(6, dtype=torch.int32, device=device)
+    nat.check(nat.lib().mvsd_sampler_rows(0, ids.data_ptr(), None, 0, x.data_ptr(), x.stride(0),
+                                          None, 0, 6, V, nat.stream_of(x.device)),
+              "mvsd_sampler_rows")
+    want = [int(x[0].cpu().argmax()), 0, 0, V // 2, V // 4, int(x[5].cpu().argmax())]
+    assert ids.tolist() == want
+    assert Sampler.greedy_sample(x).tolist() == want

@@ -972,10 +972,12 @@ __global__ __launch_bounds__(kCT) void constraints_kernel(VerifyParams p) {
 //                  the exact sums confirm that the crossing lies in it, and a row where it does
 //                  not, or that does not fit (more than 4096 entries, k above 512), takes
 //                  row_thresholds in this workgroup.
+// (and split_apply where the rows themselves are masked in place).
 // So a top-p row is read twice instead of three times, by as many workgroups as it has chunks.
-// What bounds it: for a few rows the chain of six short kernels (8 bf16 rows of 151936 entries with
-// top-p: plan 4 us, scan 7, pick 17, mass 9, finish 13, where the row kernel takes 76); for many,
-// the exponentials of scan and mass, about 30 VALU operations per entry each.
+// What bounds it: for a few rows the chain of five short kernels (8 bf16 rows of 151936 entries with
+// top-p: 38 us a call, where the row kernel takes 71; the 32 rows of a step of 8 requests, half of
+// them with top-k too, kernel by kernel under the profiler: plan 4 us, scan 8, pick 22, mass 12,
+// finish 14); for many, the exponentials of scan and mass, about 30 VALU operations per entry each.
 
 constexpr int kSplitThreads = 256;
 constexpr int kSplitLong = 8192, kSplitShort = 2048;  // columns per chunk
@@ -1813,8 +1815,11 @@ __global__ __launch_bounds__(kSplitThreads) void split_apply_kernel(SplitParams 
 }
 
 int split_chunk(int64_t rows, int64_t V) {
-  // 2048 columns while chunks of 8192 would be about one workgroup per compute unit (a 2048-column
-  // item takes nearly as long as an 8192-column one: 48 rows took 70 us with short chunks, 49 long)
+  // 2048 columns while chunks of 8192 would be about one workgroup per compute unit.  Top-p bf16 rows
+  // of 151936 entries, short / long chunks: 8 rows 38 / 35 us, 16 rows 44 / 40, 32 rows 56 / 42; of
+  // 65536: 8 rows 28 / 31, 32 rows 33 / 32, 64 rows 41 / 35.  Half greedy, a quarter top-k, a quarter
+  // top-p, of 151936: 40 / 45, 42 / 45, 46 / 46 and 64 rows 55 / 49; of 65536: 36 / 42, 36 / 43 (32
+  // rows) and 39 / 43.
   return rows * ((V + kSplitLong - 1) / kSplitLong) < 300 &&
                  (V + kSplitShort - 1) / kSplitShort <= kSplitMaxChunks
              ? kSplitShort
@@ -1826,11 +1831,15 @@ struct SplitLayout {
   int64_t head, rows, cmax, cties, csum, gkeys, hist, cmass, cand, masks, total;
 };
 
-// Whether a call's rows are split: few of them, with their groups in LDS.  With many rows every
-// compute unit has rows of its own, and the row kernel, which takes one exponential per entry
-// instead of two, is as fast: top-p rows of 151936 bf16 entries took 76 us (row kernel) against 43
-// (split) for 8 rows, 82 / 53 for 64, 87 / 72 for 128, 88 / 89 for 192 and 124 / 175 for 512; half
-// greedy, a quarter top-k, a quarter top-p: 77 / 54 for 128.
+// Whether a call's rows are split: few of them and long ones, with their groups in LDS.  With many
+// rows every compute unit has rows of its own, and the row kernel, which takes one exponential per
+// entry instead of two, is as fast: top-p rows of 151936 bf16 entries took 71 us (row kernel)
+// against 38 (split) for 8 rows, 75 / 49 for 64, 77 / 68 for 128, 78 / 82 for 192 and 112 / 165 for
+// 512; half greedy, a quarter top-k, a quarter top-p: 75 / 60 for 128, 78 / 77 for 256.  On short
+// rows the chain of launches is the longer one for batches of every class: those mixed rows took
+// 42 / 36 us for 16 rows of 65536 entries and 42 / 43 for 64, but 36 / 36 and 37 / 45 of 50257 and 30 /
+// 36 and 30 / 43 of 32000 (top-p rows alone still gain there for few rows: 37 / 30 for 16 of 50257, 30 /
+// 28 of 32000).
 constexpr int64_t kSplitRows = 128, kSplitMinV = 65536;
 bool split_rows(int64_t P, int64_t V) {
   const int64_t chunk = split_chunk(P, V), nch = (V + chunk - 1) / chunk;

@@ -19,7 +19,7 @@ namespace mvsd {
 
 constexpr int kTile = 4096;
 constexpr int kMaxDraft = 256;
-constexpr int kNgThreads = 512;  // 256 histories of 4096 tokens: 6.6 us against 7.8 with 256 threads
+constexpr int kNgThreads = 512;  // 256 histories of 4096 tokens: 6.4 us against 7.8 with 256 threads
 constexpr int kNgramSplitGrid = 1024;  // workgroups of a split launch
 constexpr int kNgramSplitReqs = 512;   // requests the workspace has entries for
 
@@ -27,7 +27,7 @@ constexpr int kNgramSplitReqs = 512;   // requests the workspace has entries for
 // one tile stays with workgroup 0 alone; else the workgroups combine their first_e[n] in the
 // workspace (agent-scope atomics, each waited for before the count that announces it), and the last
 // of them to finish picks the draft and clears the request's entries for the next call.  Eight
-// histories of 131072 tokens took 104 us as 32 tiles one after another, and take 7.0 us side by side:
+// histories of 131072 tokens took 104 us as 32 tiles one after another, and take 7.4 us side by side:
 // a launch, three dependent loads, one tile and two rounds of atomics.
 template <bool SPLIT>
 __global__ __launch_bounds__(kNgThreads) void ngram_kernel(NgramParams p) {

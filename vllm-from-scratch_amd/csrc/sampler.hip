@@ -1,6 +1,7 @@
 // Row kernels of the regular sampler as the rejection sampler uses it for bonus tokens
 // (minivllm/sample/sampler.py:73-120, :243-349; ops/topk_topp_sampler.py:82-91):
-//   argmax_rows      greedy_sample: argmax of each row (NaN first, lowest index on ties)
+//   argmax_rows      argmax of each row (NaN first, lowest index on ties), for callers of the C
+//                    entry point; the Sampler's greedy_sample is the race's greedy rows
 //   min_p_rows       apply_min_p: p = softmax(x); entries with p < max(p) * min_p -> -inf
 //   log_softmax_rows compute_logprobs: (x - max) - log(sum exp(x - max))
 // one 256-thread workgroup per row; and the exponential race of random_sample (argmax of

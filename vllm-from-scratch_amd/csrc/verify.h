@@ -136,8 +136,9 @@ hipError_t launch_verify(const VerifyParams& params, int target_dtype, int grid,
 hipError_t launch_constraints(const VerifyParams& params, int target_dtype, hipStream_t stream);
 // The same masks (params.masks, or scratch of its own when that is null) with each row split over
 // workgroups.  The scratch holds split_constraints_bytes(rows, V) bytes, 256-byte aligned; 0 where
-// the split path does not apply (above 128 rows).  Without top-p, launch_constraints is as fast.  params.cu null: one row per request; params.temperature null:
-// no divide, no greedy row.  bonus_rows (or null) adds request r's bonus row, target row
+// the split path does not apply (above 128 rows, below 65536 columns, above 524288).  Without
+// top-p, launch_constraints is as fast.  params.cu null: one row per request; params.temperature
+// null: no divide, no greedy row.  bonus_rows (or null) adds request r's bonus row, target row
 // bonus_rows[r], as row P + r of the masks (P + B rows in all).  apply: masked entries of the
 // (fp32) rows become -inf.
 int64_t split_constraints_bytes(int64_t rows, int64_t V);

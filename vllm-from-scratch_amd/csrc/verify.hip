@@ -1213,8 +1213,9 @@ __device__ inline void task_columns(const VerifyParams& p, int part, bool tail, 
 // ------------------------------------------------------------------ main kernel ------
 // DD: the draft probabilities' dtype (MVSD_F32, MVSD_BF16, MVSD_F16), -1 for point-mass drafts,
 // or kGreedyOnly for launches whose requests are all greedy: no softmax statistics and no score
-// tasks, two fifths of the code and a quarter of its spilled scalar registers, which small greedy
-// batches, bound by latency, pay for (four requests of three fp32 rows: 12.8 -> 11.9 us a call).
+// tasks, 20.7 KB of code instead of 56.4 and 77 spilled scalar registers instead of 135 (fp32),
+// which small greedy batches, bound by latency, pay for (four requests of three fp32 rows: 12.8 ->
+// 11.9 us a call).
 template <int DT, int EPT, int G, int DD, bool MASKED>
 __global__ __launch_bounds__(kVThreads) void verify_kernel(VerifyParams p) {
   static_assert(EPT % Elem<DT>::kVec == 0, "EPT must be a multiple of the vector width");

@@ -1,7 +1,7 @@
 """top-k / top-p masking (drop-in for minivllm/sample/ops/topk_topp_sampler.py:48-79).
 
-Rows split over workgroups (``mvsd_apply_top_k_top_p_split``, up to 128 rows with top-p) or one
-HIP workgroup per row (``mvsd_apply_top_k_top_p``): the k-th largest value from the
+Rows split over workgroups (``mvsd_apply_top_k_top_p_split``, up to 128 rows of at least 65536
+columns with top-p) or one HIP workgroup per row (``mvsd_apply_top_k_top_p``): the k-th largest value from the
 entries at or above the k-th largest per-thread maximum, gathered and sorted in LDS; the
 top-p crossing from a logarithmic mass histogram and the entries of the crossing bin; then one
 masking pass -- no sort of the vocabulary.

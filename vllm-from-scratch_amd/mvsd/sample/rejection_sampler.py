@@ -302,7 +302,8 @@ class RejectionSampler:
         ``metadata.target_logits_indices``; the bonus rows from ``bonus_logits`` [B, V] or, when
         it is None, from ``logits`` at ``metadata.bonus_logits_indices``.  The values are the
         log-softmax of each row, or the rows themselves in the ``*_logits`` modes.  One
-        ``mvsd_spec_logprobs_split`` call (``mvsd_spec_logprobs`` above 128 logprobs); when both
+        ``mvsd_spec_logprobs_split`` call (``mvsd_spec_logprobs`` above 128 logprobs, or for a few
+        short rows); when both
         kinds of rows come from ``logits`` the former reads them in place in their own dtype.
         """
         from ..outputs import LogprobsTensors
@@ -816,7 +817,7 @@ def _step_masks(logits: torch.Tensor, metadata: "SpecDecodeMetadata", sm: Sampli
 
 def _constraints_scratch(num_rows: int, vocab_size: int, top_p, device) -> torch.Tensor | None:
     """Scratch of the sampling constraints' split path for one call; None where one workgroup
-    per row is as fast (no top-p, or more than 128 rows)."""
+    per row is as fast (no top-p, more than 128 rows, or fewer than 65536 columns)."""
     if top_p is None:
         return None
     size = nat.lib().mvsd_constraints_scratch_bytes(num_rows, vocab_size)

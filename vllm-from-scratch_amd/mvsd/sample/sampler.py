@@ -163,7 +163,7 @@ def row_logprobs(rows: torch.Tensor, num_logprobs: int, token_ids: torch.Tensor,
     """Each row's token first, then its top ``num_logprobs`` (value, then index), as the row's
     log-softmax or (``logits_mode``) its values, and the token's rank: one
     ``mvsd_row_logprobs_split`` call on rows of any float dtype.  None where that path does not
-    apply (above 128 logprobs)."""
+    apply (above 128 logprobs, a few short rows)."""
     n, V = rows.shape
     device = rows.device
     token_ids = token_ids.reshape(n)  # one per row, or an error here
@@ -239,7 +239,7 @@ class Sampler:
     def _reads_rows_in_place(self, logits: torch.Tensor, sm: SamplingMetadata,
                              logprobs_mode: str) -> bool:
         """True when this batch needs no row written: no penalty or active min_tokens, no min_p,
-        and only raw logprobs, up to the 128 of the split path.  (With top-k or top-p, the
+        and only raw logprobs, where the split path takes them.  (With top-k or top-p, the
         caller's own contiguous fp32 rows are to be divided and masked in place; other rows are
         copied before that, so there it does not show.)"""
         from .rejection_sampler import _has_active_min_tokens

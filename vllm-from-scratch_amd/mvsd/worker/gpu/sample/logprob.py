@@ -1,5 +1,6 @@
 """``compute_topk_scores`` of the V2 sampler on the HIP logprobs kernel (csrc/logprobs.hip,
-C ABI ``mvsd_topk_scores_split`` for up to 128 logprobs, ``mvsd_topk_scores`` above).
+C ABI ``mvsd_topk_scores_split`` for up to 128 logprobs, ``mvsd_topk_scores`` above and for a few
+rows too short to split).
 
 Replaces minivllm/worker/gpu/sample/logprob.py:140-216 on the path without per-request
 logprob token ids (the only path the V2 verification reaches): for every row n of
@@ -12,8 +13,8 @@ logprob token ids (the only path the V2 verification reaches): for every row n o
 * ``selected_token_ranks[n] = #{i : logits[n, i] >= logits[n, token]}`` (``_ranks_kernel``,
   :86-104), int64.
 
-Up to 128 logprobs, every row is read once, in its own dtype, split over workgroups; above, one
-workgroup per fp32 row reads it once for its max and sum and once per 32 top-k keys.
+Split rows are read once, in their own dtype, by as many workgroups as they have chunks; otherwise
+one workgroup per fp32 row reads it once for its max and sum and once per 32 top-k keys.
 """
 
 from __future__ import annotations
