@@ -115,3 +115,12 @@ def test_draft_counts_of_any_integer_type(counts):
 def test_gather_logprobs_takes_one_token_per_row(shape):
     with pytest.raises(RuntimeError, match="shape"):
         Sampler.gather_logprobs(torch.zeros(2, 16), 1, torch.zeros(shape, dtype=torch.int64))
+
+
+@pytest.mark.parametrize("rows", [None, torch.zeros(0, dtype=torch.int32)])
+def test_no_rows_have_no_masks(rows):
+    """A batch without requests is taken, with limits as without."""
+    sm = SamplingMetadata(temperature=torch.ones(0), all_greedy=False, all_random=True,
+                          top_k=torch.ones(0), top_p=torch.ones(0))
+    logits = torch.zeros(0 if rows is None else 3, 16)
+    assert smp.constraint_masks(logits, rows, sm) is None

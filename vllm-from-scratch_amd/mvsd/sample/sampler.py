@@ -131,6 +131,8 @@ def constraint_masks(logits: torch.Tensor, row_index: torch.Tensor | None,
     one request each, for ``race_rows``; None when no request has either."""
     if sm.all_greedy or (sm.top_k is None and sm.top_p is None):
         return None
+    if (logits if row_index is None else row_index).shape[0] == 0:
+        return None
     device = logits.device
 
     def on_device(values, dtype):
