@@ -1,18 +1,11 @@
 // Host-side work on Python token lists, as a CPython extension module (mvsd._hostops): what the
 // penalties need to know of each request's history, gathered without converting every list to an
-// array first.  32 requests of 650 tokens: 4.0 ms with numpy (np.unique per request), 0.2 here.
+// array first.  32 requests of 650 tokens: 4.0 ms with numpy (np.unique per request), 0.17 here.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #include <stdint.h>
 #include <stdlib.h>
 #include <string.h>
-
-// One request's distinct tokens: an open-addressing table of places in the entry arrays.
-typedef struct {
-  int32_t* slot;    // place + 1, 0 = free
-  size_t cap;       // slots in use for this request, a power of two
-  size_t room;      // slots allocated
-} Table;
 
 static uint64_t mix(uint64_t x) {
   x ^= x >> 31;
@@ -20,17 +13,45 @@ static uint64_t mix(uint64_t x) {
   return x ^ (x >> 29);
 }
 
-// The place of token t among this request's entries [0, *n), added when it is new.
-static int32_t place_of(Table* tb, int64_t* keys, int32_t* n, int64_t t) {
-  size_t i = (size_t)mix((uint64_t)t) & (tb->cap - 1);
-  while (tb->slot[i]) {
-    const int32_t at = tb->slot[i] - 1;
+// The place of token t among this request's entries [0, *n), added when it is new: an
+// open-addressing table of mask + 1 slots (a power of two) that hold a place + 1, or 0.
+static int32_t place_of(int32_t* slots, size_t mask, int64_t* keys, int32_t* n, int64_t t) {
+  size_t i = (size_t)mix((uint64_t)t) & mask;
+  while (slots[i]) {
+    const int32_t at = slots[i] - 1;
     if (keys[at] == t) return at;
-    i = (i + 1) & (tb->cap - 1);
+    i = (i + 1) & mask;
   }
   keys[*n] = t;
-  tb->slot[i] = *n + 1;
+  slots[i] = *n + 1;
   return (*n)++;
+}
+
+// Adds the first `len` tokens of a fast sequence to the request's entries: of its prompt (kind 0),
+// output (1) or drafts (2).  0 where a token is no integer (the exception is set).
+static int add_tokens(PyObject* seq, Py_ssize_t len, int kind, int32_t* slots, size_t mask,
+                      int64_t* keys, int32_t* info, int32_t* n) {
+  // a list can change while __index__ of an element runs: look at it afresh each time
+  for (Py_ssize_t i = 0; i < len && i < PySequence_Fast_GET_SIZE(seq); ++i) {
+    PyObject* item = PySequence_Fast_GET_ITEM(seq, i);
+    int64_t t;
+    if (PyLong_CheckExact(item)) {
+      t = PyLong_AsLongLong(item);
+    } else {
+      Py_INCREF(item);
+      PyObject* whole = PyNumber_Index(item);
+      t = whole ? PyLong_AsLongLong(whole) : -1;
+      Py_XDECREF(whole);
+      Py_DECREF(item);
+    }
+    if (t == -1 && PyErr_Occurred()) return 0;
+    const int32_t before = *n;
+    const int32_t at = place_of(slots, mask, keys, n, t);
+    if (at == before) info[at] = 0;
+    if (kind == 0) info[at] |= (int32_t)0x80000000u;
+    if (kind == 1) ++info[at];
+  }
+  return 1;
 }
 
 // penalty_entries(prompts, outputs, specs, buffer) -> number of entries E
@@ -48,8 +69,8 @@ static PyObject* penalty_entries(PyObject* self, PyObject* args) {
   PyObject* result = NULL;
   int64_t* keys = NULL;
   int32_t* info = NULL;
-  Table tb = {NULL, 0, 0};
-  size_t keys_cap = 0;
+  int32_t* slots = NULL;
+  size_t slots_room = 0, keys_cap = 0;
   for (int s = 0; s < 3; ++s) {
     outer[s] = PySequence_Fast(lists[s], "a sequence of token sequences is expected");
     if (!outer[s]) goto out;
@@ -88,52 +109,29 @@ static PyObject* penalty_entries(PyObject* self, PyObject* args) {
         PyErr_SetString(PyExc_ValueError, "buffer too small");
         ok = 0;
       }
+      // The table has this request's own size, so that a short history after a long one clears a
+      // small one; at most a quarter full (half full: 0.20 ms instead of 0.17 for 32 requests).
       size_t cap = 16;
-      while (cap < 2 * all) cap *= 2;
-      tb.cap = cap;  // its own size: a short history after a long one clears a small table
-      if (ok && cap > tb.room) {
-        free(tb.slot);
-        tb.slot = (int32_t*)malloc(cap * sizeof(int32_t));
-        tb.room = tb.slot ? cap : 0;
+      while (cap < 4 * all) cap *= 2;
+      if (ok && cap > slots_room) {
+        free(slots);
+        slots = (int32_t*)malloc(cap * sizeof(int32_t));
+        slots_room = slots ? cap : 0;
       }
       if (ok && all > keys_cap) {
         free(keys);
         keys_cap = all;
         keys = (int64_t*)malloc(keys_cap * sizeof(int64_t));
       }
-      if (ok && (!tb.slot || (all && !keys))) {
+      if (ok && (!slots || (all && !keys))) {
         PyErr_NoMemory();
         ok = 0;
       }
       if (ok) {
-        memset(tb.slot, 0, tb.cap * sizeof(int32_t));
+        memset(slots, 0, cap * sizeof(int32_t));
         int32_t n = 0;
-        for (int s = 0; s < 3 && ok; ++s) {
-          // a list can change while __index__ of an element runs: look at it afresh each time
-          for (Py_ssize_t i = 0; inner[s] && i < len[s] && i < PySequence_Fast_GET_SIZE(inner[s]);
-               ++i) {
-            PyObject* item = PySequence_Fast_GET_ITEM(inner[s], i);
-            int64_t t;
-            if (PyLong_CheckExact(item)) {
-              t = PyLong_AsLongLong(item);
-            } else {
-              Py_INCREF(item);
-              PyObject* whole = PyNumber_Index(item);
-              t = whole ? PyLong_AsLongLong(whole) : -1;
-              Py_XDECREF(whole);
-              Py_DECREF(item);
-            }
-            if (t == -1 && PyErr_Occurred()) {
-              ok = 0;
-              break;
-            }
-            const int32_t before = n;
-            const int32_t at = place_of(&tb, keys, &n, t);
-            if (at == before) info[total + at] = 0;
-            if (s == 0) info[total + at] |= (int32_t)0x80000000u;
-            if (s == 1) ++info[total + at];
-          }
-        }
+        for (int s = 0; s < 3 && ok; ++s)
+          ok = !inner[s] || add_tokens(inner[s], len[s], s, slots, cap - 1, keys, info + total, &n);
         for (int32_t e = 0; ok && e < n; ++e) tok[total + e] = (int32_t)keys[e];
         total += ok ? n : 0;
         off[r + 1] = (int32_t)total;
@@ -146,7 +144,7 @@ static PyObject* penalty_entries(PyObject* self, PyObject* args) {
   }
 out:
   for (int s = 0; s < 3; ++s) Py_XDECREF(outer[s]);
-  free(tb.slot);
+  free(slots);
   free(keys);
   free(info);
   PyBuffer_Release(&buf);

@@ -206,12 +206,14 @@ class RejectionSampler:
             return False
         if sm.no_penalties:
             return True
-        counts = [int(k) for k in metadata.num_draft_tokens]
+        counts = metadata.num_draft_tokens
+        if type(counts) is not list:
+            counts = list(map(int, counts))
         return (getattr(self.apply_logits_processors, "__func__", None)
                 is _APPLY_LOGITS_PROCESSORS
                 and (apply_sampling_constraints, apply_top_k_top_p) == _CONSTRAINT_FUNCTIONS
                 and logits.shape[0] == sum(counts) + len(counts)
-                and bool(sm.spec_token_ids) and [len(s) for s in sm.spec_token_ids] == counts)
+                and bool(sm.spec_token_ids) and list(map(len, sm.spec_token_ids)) == counts)
 
     def _forward_race_only(self, metadata: "SpecDecodeMetadata",
                            draft_probs: torch.Tensor | None, logits: torch.Tensor,
@@ -255,16 +257,15 @@ class RejectionSampler:
                            if masks is None else masks[num_tokens:])
         bonus = smp.race_rows(logits, metadata.bonus_logits_indices, bonus_noise,
                               None if all_greedy else sm.temperature, masks=bonus_masks)
-        sample = (rejection_sample if masks is None
-                  else functools.partial(_rejection_sample, row_masks=masks))
-        output_token_ids = sample(
+        own = rejection_sample is _REJECTION_SAMPLE  # a replacement takes no masks, but finds them
+        output_token_ids = (_rejection_sample if own else rejection_sample)(
             metadata.draft_token_ids, metadata.num_draft_tokens, metadata.max_spec_len,
             metadata.cu_num_draft_tokens, draft_probs, logits, bonus.view(B, 1), sm,
             synthetic_mode=self.synthetic_mode,
             synthetic_conditional_rates=self.synthetic_conditional_rates,
             uniform_probs=uniforms, exp_noise=exp_noise,
             target_rows=metadata.target_logits_indices, apply_temperature=True,
-            apply_top_k_top_p=constrained)
+            apply_top_k_top_p=constrained, **({"row_masks": masks} if own else {}))
         logprobs_tensors = None
         if sm.max_num_logprobs is not None:
             logprobs_tensors = self._get_logprobs_tensors(
@@ -470,7 +471,8 @@ def _penalty_entries(prompts, outputs, specs):
     from .. import _hostops
 
     B = len(specs)
-    room = sum(sum(map(len, islice(lists, B))) for lists in (prompts, outputs, specs))
+    room = (sum(map(len, islice(prompts, B))) + sum(map(len, islice(outputs, B)))
+            + sum(map(len, specs)))
     buffer = np.empty(B + 1 + 2 * room, dtype=np.int32)
     try:
         n = _hostops.penalty_entries(prompts, outputs, specs, buffer)

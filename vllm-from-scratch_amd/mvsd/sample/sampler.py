@@ -442,10 +442,11 @@ class Sampler:
 
 
 # The steps that Sampler.forward takes one after another, and the functions that they call.
-_STEPS = {name: Sampler.__dict__[name] for name in (
+_STEPS = frozenset((
     "forward", "apply_logits_processors", "apply_penalties", "_combine_outputs_with_spec_tokens",
     "apply_min_tokens", "sample", "apply_min_p", "greedy_sample", "compute_logprobs",
-    "gather_logprobs")}
+    "gather_logprobs"))
+_OWN_STEPS = list(map(Sampler.__dict__.get, _STEPS))
 _TOP_K_TOP_P_CALL = TopKTopPSampler.__call__
 _STEP_FUNCTIONS = (apply_top_k_top_p, random_sample)
 
@@ -458,7 +459,7 @@ def runs_own_steps(sampler) -> bool:
         return False
     limits = sampler.topk_topp_sampler
     return (type(limits) is TopKTopPSampler and limits.logprobs_mode not in _PROCESSED_MODES
-            and _STEPS.keys().isdisjoint(vars(sampler))
-            and all(Sampler.__dict__.get(name) is step for name, step in _STEPS.items())
+            and _STEPS.isdisjoint(vars(sampler))
+            and list(map(Sampler.__dict__.get, _STEPS)) == _OWN_STEPS
             and TopKTopPSampler.__call__ is _TOP_K_TOP_P_CALL
             and (apply_top_k_top_p, random_sample) == _STEP_FUNCTIONS)
