@@ -287,7 +287,7 @@ __global__ __launch_bounds__(kLpThreads) void spec_logprobs_kernel(LogprobParams
 //   - More candidates than LDS holds: the entries strictly above theta, then as many entries equal
 //     to it as are missing, lowest index first; or, if even those above do not fit, the lists.
 // What bounds it: the scan is one read of the rows with about 12 VALU operations per entry
-// (131 us for 1280 fp32 rows of 151936 columns under the profiler, 5.9 TB/s); the finish is a chain
+// (128 us for 1280 fp32 rows of 151936 columns under the profiler, 6.1 TB/s); the finish is a chain
 // of a few small loads and barriers (21 us for those rows, 28 before the 64 unions and the compare;
 // 8 us for 32).  The scan's exponentials are exp2 of the rounded product (x - max) log2(e), where the
 // lists call expf: against 64 bits the values are as close (the mean error over 60 sets of rows
