@@ -39,7 +39,7 @@ from __future__ import annotations
 
 import functools
 from dataclasses import replace
-from itertools import islice
+from itertools import accumulate, islice
 from typing import TYPE_CHECKING
 
 import numpy as np
@@ -509,9 +509,9 @@ def _expand_opt(values: torch.Tensor | None, cu: torch.Tensor, num_rows: int):
     return None if values is None else expand_batch_to_tokens(values, cu, num_rows)
 
 
-def _upload(arrays, device) -> list[torch.Tensor]:
-    """int32 device copies of host arrays, through one pinned buffer and one copy that the host
-    does not wait for.  Refused in a graph capture: a replay would read the pinned buffer again,
+def _upload(arrays, device) -> tuple[torch.Tensor, list[int]]:
+    """One int32 device tensor with the host arrays one after another, and each one's address in
+    it; through one pinned buffer and one copy that the host does not wait for.  Refused in a graph capture: a replay would read the pinned buffer again,
     which by then holds another call's arrays."""
     if torch.cuda.is_current_stream_capturing():
         raise RuntimeError("penalties and min_tokens upload host lists, which a graph capture "
@@ -519,7 +519,9 @@ def _upload(arrays, device) -> list[torch.Tensor]:
     arrays = [np.asarray(a, dtype=np.int32) for a in arrays]
     host = torch.empty(sum(a.size for a in arrays), dtype=torch.int32, pin_memory=True)
     np.concatenate(arrays, out=host.numpy())
-    return list(host.to(device, non_blocking=True).split([a.size for a in arrays]))
+    uploaded = host.to(device, non_blocking=True)
+    return uploaded, list(accumulate((4 * a.size for a in arrays[:-1]),
+                                     initial=uploaded.data_ptr()))
 
 
 def _launch_logits_processors(logits, cu, num_draft, specs, entries, penalties, masks,
@@ -551,19 +553,19 @@ def _launch_logits_processors(logits, cu, num_draft, specs, entries, penalties, 
     cu_t = _as(cu, torch.int32, device)
     spec = np.asarray([t for row in specs for t in row], dtype=np.int32)
     host = [spec, *(entries or ()), *(masks or ())]
-    on_device = iter(_upload(host, device))
-    spec_t = next(on_device)
+    uploaded, addresses = _upload(host, device)
+    keep.append(uploaded)
+    spec_ptr, *addresses = addresses
     ent_off = ent_tok = ent_info = None
     presence = frequency = repetition = None
     if entries is not None:
-        ent_off, ent_tok, ent_info = (next(on_device).data_ptr() for _ in range(3))
+        ent_off, ent_tok, ent_info, *addresses = addresses
         presence = dev_opt(penalties.presence_penalties)
         frequency = dev_opt(penalties.frequency_penalties)
         repetition = dev_opt(penalties.repetition_penalties)
     n_mask = stop_off = stop_tok = None
     if masks is not None:
-        n_mask, stop_off, stop_tok = (next(on_device).data_ptr() for _ in range(3))
-    spec_ptr = spec_t.data_ptr() if spec.size else None
+        n_mask, stop_off, stop_tok = addresses
     if bonus_rows is None:
         nat.check(nat.lib().mvsd_apply_logits_processors(
             logits.data_ptr(), logits.stride(0), num_rows, V, len(num_draft), cu_t.data_ptr(),
