@@ -1837,8 +1837,8 @@ struct SplitLayout {
 // against 38 (split) for 8 rows, 75 / 49 for 64, 77 / 68 for 128, 78 / 82 for 192 and 112 / 165 for
 // 512; half greedy, a quarter top-k, a quarter top-p: 75 / 60 for 128, 78 / 77 for 256.  On short
 // rows the chain of launches is the longer one for batches of every class: those mixed rows took
-// 42 / 36 us for 16 rows of 65536 entries and 42 / 43 for 64, but 36 / 36 and 37 / 45 of 50257 and 30 /
-// 36 and 30 / 43 of 32000 (top-p rows alone still gain there for few rows: 37 / 30 for 16 of 50257, 30 /
+// 42 / 37 us for 16 rows of 65536 entries and 42 / 43 for 64, but 36 / 36 and 37 / 45 of 50257 and 30 /
+// 36 and 30 / 37 of 32000 (top-p rows alone still gain there for few rows: 37 / 30 for 16 of 50257, 30 /
 // 28 of 32000).
 constexpr int64_t kSplitRows = 128, kSplitMinV = 65536;
 bool split_rows(int64_t P, int64_t V) {
