@@ -304,8 +304,9 @@ constexpr int kThetaWaveK = 32;       // largest k whose theta is read off 64 ke
 constexpr float kLpLog2e = 1.44269504088896340736f;
 
 // Columns per chunk: 8192, or 2048 where rows of 8192-column chunks would leave compute units
-// idle (fewer than 4 workgroups each) or give fewer than two groups per candidate wanted, so that
-// theta is a poor bound or none: 1000 fp32 rows of 32000 columns took 90 us with long chunks and 45
+// idle (fewer than 4 workgroups each; fp32 rows, k = 20, short / long chunks: 64 rows of 151936 columns
+// 19 / 21 us, 1000 rows 127 / 115; of 100000 16 / 18 and 85 / 79; of 50257 13 / 16 and 44 / 50) or give
+// fewer than two groups per candidate wanted, so that theta is a poor bound or none: 1000 fp32 rows of 32000 columns took 90 us with long chunks and 45
 // with short ones for k = 64 (64 long groups), 1488 and 53 for k = 128; of 65536 columns 70 and 62
 // for k = 64 (128 groups, where the two meet).
 constexpr int kChunkLong = 8192, kChunkShort = 2048;
