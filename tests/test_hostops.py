@@ -71,7 +71,7 @@ def test_a_long_history_costs_no_more_first_than_last():
             best = min(best, time.perf_counter() - start)
         return best
 
-    assert seconds(long + short) < 3 * seconds(short + long)
+    assert seconds(long + short) < 10 * seconds(short + long)  # about 40 with one table for all
 
 
 def test_errors():

@@ -171,3 +171,27 @@ def test_forward_with_penalties_in_other_forms(device, form):
         torch.manual_seed(11)
         outs.append(rs.RejectionSampler(cls()).forward(meta, None, logits, sm))
     same(*outs, 0.0)
+
+
+def test_forward_calls_a_replaced_rejection_sample(device, monkeypatch):
+    """A batch without limits races its bonus rows, then calls rejection_sample by its name, with
+    the arguments it had before there were limits on that route."""
+    V, drafts = 300, [[3], []]
+    meta = make_metadata(drafts, device=device)
+    logits = torch.randn(3, V, device=device)
+    real, seen = rs.rejection_sample, []
+
+    def replacement(*args, synthetic_mode, synthetic_conditional_rates, uniform_probs, exp_noise,
+                    target_rows, apply_temperature):
+        seen.append(args)
+        return real(*args, uniform_probs=uniform_probs, exp_noise=exp_noise,
+                    target_rows=target_rows, apply_temperature=apply_temperature)
+
+    outs = []
+    for function in (real, replacement):
+        monkeypatch.setattr(rs, "rejection_sample", function)
+        torch.manual_seed(2)
+        outs.append(rs.RejectionSampler(Sampler()).forward(
+            meta, None, logits, sampling_metadata([1.0, 0.6], drafts, device=device)))
+    same(*outs, 0.0)
+    assert len(seen) == 1

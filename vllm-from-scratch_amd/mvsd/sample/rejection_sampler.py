@@ -257,7 +257,7 @@ class RejectionSampler:
                            if masks is None else masks[num_tokens:])
         bonus = smp.race_rows(logits, metadata.bonus_logits_indices, bonus_noise,
                               None if all_greedy else sm.temperature, masks=bonus_masks)
-        own = rejection_sample is _REJECTION_SAMPLE  # a replacement takes no masks, but finds them
+        own = rejection_sample is _REJECTION_SAMPLE  # a replacement meets no limits here
         output_token_ids = (_rejection_sample if own else rejection_sample)(
             metadata.draft_token_ids, metadata.num_draft_tokens, metadata.max_spec_len,
             metadata.cu_num_draft_tokens, draft_probs, logits, bonus.view(B, 1), sm,
@@ -265,7 +265,7 @@ class RejectionSampler:
             synthetic_conditional_rates=self.synthetic_conditional_rates,
             uniform_probs=uniforms, exp_noise=exp_noise,
             target_rows=metadata.target_logits_indices, apply_temperature=True,
-            apply_top_k_top_p=constrained, **({"row_masks": masks} if own else {}))
+            **({"apply_top_k_top_p": constrained, "row_masks": masks} if own else {}))
         logprobs_tensors = None
         if sm.max_num_logprobs is not None:
             logprobs_tensors = self._get_logprobs_tensors(
